@@ -343,7 +343,7 @@ int ppmg_p2m(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, const void
     if (!force_general && p2m3d_fast_applicable(m, kernel, prec, fg)) {
         if (p2m3d_fast(plan, m, kernel, prec, np, xp, fg, up, field->data, nullptr, s)) return g_status.info;
     } else if (!force_general && p2m2d_fast_applicable(m, kernel, fg)) {
-        if (p2m2d_fast(plan, m, kernel, prec, xp, fg, up, field->data, s)) return g_status.info;
+        if (p2m2d_fast(plan, m, kernel, prec, xp, fg, up, field->data, nullptr, s)) return g_status.info;
     } else if (p2m_general(plan, m, kernel, prec, np, xp, lda, up, fg, field->data, nullptr, s)) {
         return g_status.info;
     }
@@ -571,17 +571,22 @@ int ppmg_rmsh_remesh(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, co
     hipStream_t s = as_stream(stream);
     int64_t nbad = 0;
     plan->have_forward = false;
-    if (bin_particles(plan, m, prec, np, xp, s, &nbad)) return g_status.info;
+    // the tiled deposits with the caller's weights (PPMG_GENERAL=1 forces the
+    // general path, for cross-checks)
+    const char* gen = std::getenv("PPMG_GENERAL");
+    const bool force_general = gen && gen[0] && gen[0] != '0';
+    if (bin_particles(plan, m, prec, np, xp, s, &nbad,
+                      !force_general &&
+                          (p2m3d_table_applicable(m, kernel, prec, fg) || p2m2d_table_applicable(m, kernel, fg))))
+        return g_status.info;
     if (nbad > 0)
         return fail(PPMG_ERROR_FATAL, PPMG_ERR_PART_UNASS,
                     "MAJOR PROBLEM: " + std::to_string(nbad) + " particles lie in no sub");
     const void* tabs[3] = {wx1, wx2, wx3};
-    // 3D M'4 on the tiled deposit with the caller's weights (PPMG_GENERAL=1
-    // forces the general path, for cross-checks)
-    const char* gen = std::getenv("PPMG_GENERAL");
-    const bool force_general = gen && gen[0] && gen[0] != '0';
-    if (!force_general && kernel == PPMG_KERNEL_MP4 && p2m3d_fast_applicable(m, kernel, prec, fg)) {
+    if (!force_general && p2m3d_fast_applicable(m, kernel, prec, fg)) {
         if (p2m3d_fast(plan, m, kernel, prec, np, xp, fg, up, field->data, tabs, s)) return g_status.info;
+    } else if (!force_general && p2m2d_fast_applicable(m, kernel, fg)) {
+        if (p2m2d_fast(plan, m, kernel, prec, xp, fg, up, field->data, tabs, s)) return g_status.info;
     } else if (p2m_general(plan, m, kernel, prec, np, xp, lda, up, fg, field->data, tabs, s)) {
         return g_status.info;
     }

@@ -23,8 +23,8 @@ int create_part_general(ppmg_plan* plan, const DevMesh& m, int prec, const Field
 bool p2m3d_fast_applicable(const DevMesh& m, int kernel, int prec, const FieldGeom& fg);
 // ... and it reads a slot-table binning (bin_particles' `table`) there.
 bool p2m3d_table_applicable(const DevMesh& m, int kernel, int prec, const FieldGeom& fg);
-// wtab: NULL (weights from the positions), or, for M'4 only, the remesh weight
-// tables (four per particle and axis, ppm_rmsh_comp_weights' layout).
+// wtab: NULL (weights from the positions), or the remesh weight tables (the
+// stencil width per particle and axis, ppm_rmsh_comp_weights' layout).
 int p2m3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp,
                const FieldGeom& fg, const void* up, void* field, const void* const* wtab, hipStream_t s);
 
@@ -34,7 +34,7 @@ bool p2m2d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg);
 // ... and it reads a slot-table binning (bin_particles' `table`) there.
 bool p2m2d_table_applicable(const DevMesh& m, int kernel, const FieldGeom& fg);
 int p2m2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, const void* xp, const FieldGeom& fg,
-               const void* up, void* field, hipStream_t s);
+               const void* up, void* field, const void* const* wtab, hipStream_t s);
 
 // 3D tiled gather (ppmg_m2p3d.hip), M'4 or BSP2, same layouts as the deposit:
 // bins the particles into the plan first (unless prebinned: the plan already

@@ -34,12 +34,17 @@ constexpr int P2_RING = 8;     // node rows in the ring (a step touches 4 + H <=
 
 // TABLE: the binning is a slot table (byte counts, particle r of cell c at
 // bt.table[r * ncells + c]) instead of heads and a permutation; a cell's
-// particles come in the same order.
-template <int KS, int LDA, typename PosT, typename ValT, bool OPEN, bool TABLE>
+// particles come in the same order.  TAB: the 1D weights come from the
+// caller's tables (ppm_rmsh_remesh's wx1/wx2, KS per particle and axis)
+// instead of the positions.
+template <int KS, int LDA, typename PosT, typename ValT, bool OPEN, bool TABLE, bool TAB>
 __global__ void __launch_bounds__(64)
 k_p2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ up, FieldGeom fg, int c0, int ty,
-          ValT* __restrict__ field) {
+          ValT* __restrict__ field, WTab<ValT> wt) {
+    // per-particle data besides the strengths: the position, or (TAB) the 2 KS 1D weights
+    constexpr int NPD = TAB ? 2 * KS : 2;
+    using PD = std::conditional_t<TAB, ValT, PosT>;
     constexpr int H = Stencil<KS>::H, B = Stencil<KS>::B;
     constexpr int TT = 16 - H;                    // owned node columns per strip
     constexpr int ROW = TT * LDA;                 // ring slots per node row: [c][x]
@@ -103,13 +108,21 @@ k_p2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
         if constexpr (TABLE) return bt.table[(int64_t)r * bt.ncells + f];
         else return perm ? perm[f + r] : f + r;
     };
-    auto load = [&](int p, bool has, PosT (&x)[2], ValT (&u)[LDA]) {
-        x[0] = x[1] = PosT(0);
+    auto load = [&](int p, bool has, PD (&x)[NPD], ValT (&u)[LDA]) {
+#pragma unroll
+        for (int d = 0; d < NPD; ++d) x[d] = PD(0);
 #pragma unroll
         for (int c = 0; c < LDA; ++c) u[c] = ValT(0);
         if (has) {
-            x[0] = xp[(int64_t)p * 2];
-            x[1] = xp[(int64_t)p * 2 + 1];
+            if constexpr (TAB) {
+#pragma unroll
+                for (int d = 0; d < 2; ++d)
+#pragma unroll
+                    for (int o = 0; o < KS; ++o) x[KS * d + o] = wt.w[d][(int64_t)p * KS + o];
+            } else {
+                x[0] = xp[(int64_t)p * 2];
+                x[1] = xp[(int64_t)p * 2 + 1];
+            }
 #pragma unroll
             for (int c = 0; c < LDA; ++c) u[c] = up[(int64_t)p * lda + c0 + c];
         }
@@ -127,7 +140,7 @@ k_p2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     heads(0, f1, n1, t1);
     heads(1, f2, n2, t2);
     int pn = lookup(f1, n1, t1);
-    PosT xn[2];
+    PD xn[NPD];
     ValT un[LDA];
     load(pn, count_of(f1, n1) > 0, xn, un);
 
@@ -142,11 +155,20 @@ k_p2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
         const int ly0 = 4 * st + erow - H;          // chunk node row of y offset 0
         // one round: every lane deposits one particle of its cell (zero
         // strength where it has none)
-        auto round = [&](const PosT (&x)[2], const ValT (&u)[LDA]) {
-            ValT fr[2], wx[KS], wy[KS];
-            offsets(x, fr);
-            tile_weights<KS, ValT>(fr[0], wx);
-            tile_weights<KS, ValT>(fr[1], wy);
+        auto round = [&](const PD (&x)[NPD], const ValT (&u)[LDA]) {
+            ValT wx[KS], wy[KS];
+            if constexpr (TAB) {
+#pragma unroll
+                for (int o = 0; o < KS; ++o) {
+                    wx[o] = x[o];
+                    wy[o] = x[KS + o];
+                }
+            } else {
+                ValT fr[2];
+                offsets(x, fr);
+                tile_weights<KS, ValT>(fr[0], wx);
+                tile_weights<KS, ValT>(fr[1], wy);
+            }
             // G[k][c] = wx_k u_c and the y weights of the particle k lanes below
             ValT G[KS][LDA], WY[KS][KS];
 #pragma unroll
@@ -188,7 +210,7 @@ k_p2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
             uint64_t act = __ballot(cnt > r);
             if (act == 0ull) break;
             if (__popcll(act) > P2_SERIAL) {
-                PosT x[2];
+                PD x[NPD];
                 ValT u[LDA];
                 load(cnt > r ? entry(first, r) : 0, cnt > r, x, u);
                 round(x, u);
@@ -205,11 +227,16 @@ k_p2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                 const bool own = slane && nx >= 0 && nx < nxo && ny >= 0 && ny < nyo;
                 double* row = ring + (ny & (P2_RING - 1)) * ROW;
                 for (int rr = r; rr < sc; ++rr) {
-                    PosT x[2];
-                    ValT u[LDA], fr[2];
+                    PD x[NPD];
+                    ValT u[LDA], w;
                     load(entry(sf, rr), true, x, u);
-                    offsets(x, fr);
-                    const ValT w = tile_weight_at<KS, ValT>(fr[0], ox) * tile_weight_at<KS, ValT>(fr[1], oy);
+                    if constexpr (TAB) {
+                        w = x[ox] * x[KS + oy];
+                    } else {
+                        ValT fr[2];
+                        offsets(x, fr);
+                        w = tile_weight_at<KS, ValT>(fr[0], ox) * tile_weight_at<KS, ValT>(fr[1], oy);
+                    }
                     if (own) {
 #pragma unroll
                         for (int c = 0; c < LDA; ++c) atomicAdd(row + c * TT + nx, (double)(w * u[c]));
@@ -261,24 +288,24 @@ bool p2m2d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg) {
 
 // One launch for components c0 .. c0+LL-1.  The chunk height comes from the
 // resident workgroup count (each chunk marches H extra cell rows).
-template <int KS, int LL, typename PosT, typename ValT, bool OPEN, bool TABLE = false>
+template <int KS, int LL, typename PosT, typename ValT, bool OPEN, bool TABLE, bool TAB>
 static void launch_p2_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
-                           const FieldGeom& fg, int c0, ValT* field, hipStream_t s) {
+                           const FieldGeom& fg, int c0, ValT* field, const WTab<ValT>& wt, hipStream_t s) {
     constexpr int H = Stencil<KS>::H, TT = 16 - H;
     static std::atomic<int> slots{0};
-    if (slots.load() == 0) slots.store(resident_workgroups(k_p2_tile<KS, LL, PosT, ValT, OPEN, TABLE>, 64));
+    if (slots.load() == 0) slots.store(resident_workgroups(k_p2_tile<KS, LL, PosT, ValT, OPEN, TABLE, TAB>, 64));
     const int Rx = m.N[0] + !m.periodic[0], Ry = m.N[1] + !m.periodic[1];
     const int tx = (Rx + TT - 1) / TT;
     const int ty = pick_z_chunk(tx, Ry, slots.load(), H);
     dim3 grid((unsigned)((int64_t)tx * ((Ry + ty - 1) / ty)));
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
-    hipLaunchKernelGGL((k_p2_tile<KS, LL, PosT, ValT, OPEN, TABLE>), grid, dim3(64), 0, s, m, plan->start.as<int>(),
-                       perm, bt, xp, up, fg, c0, ty, field);
+    hipLaunchKernelGGL((k_p2_tile<KS, LL, PosT, ValT, OPEN, TABLE, TAB>), grid, dim3(64), 0, s, m, plan->start.as<int>(),
+                       perm, bt, xp, up, fg, c0, ty, field, wt);
 }
 
-template <int KS, typename PosT, typename ValT>
+template <int KS, typename PosT, typename ValT, bool TAB>
 static int p2m2d_typed(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, const ValT* up,
-                       ValT* field, hipStream_t s) {
+                       ValT* field, const WTab<ValT>& wt, hipStream_t s) {
     mark(plan, s);
     const int lda = fg.lda;
     const bool open = !(m.periodic[0] && m.periodic[1]);
@@ -289,9 +316,9 @@ static int p2m2d_typed(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const 
         const int L = lda - c0 < 4 ? lda - c0 : 4;
 #define TL(LL)                                                                              \
     do {                                                                                    \
-        if (plan->bin_table) launch_p2_open<KS, LL, PosT, ValT, false, true>(plan, m, xp, up, pk, fg, c0, field, s); \
-        else if (open) launch_p2_open<KS, LL, PosT, ValT, true>(plan, m, xp, up, pk, fg, c0, field, s); \
-        else launch_p2_open<KS, LL, PosT, ValT, false>(plan, m, xp, up, pk, fg, c0, field, s);     \
+        if (plan->bin_table) launch_p2_open<KS, LL, PosT, ValT, false, true, TAB>(plan, m, xp, up, pk, fg, c0, field, wt, s); \
+        else if (open) launch_p2_open<KS, LL, PosT, ValT, true, false, TAB>(plan, m, xp, up, pk, fg, c0, field, wt, s); \
+        else launch_p2_open<KS, LL, PosT, ValT, false, false, TAB>(plan, m, xp, up, pk, fg, c0, field, wt, s);     \
     } while (0)
         if (L == 1) TL(1);
         else if (L == 2) TL(2);
@@ -300,27 +327,31 @@ static int p2m2d_typed(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const 
 #undef TL
         PPMG_HIP(hipGetLastError());
     }
-    const WTab<ValT> wt{{nullptr, nullptr, nullptr}};
     if (fill_stored_box<2, KS, PosT, ValT>(plan, m, xp, up, fg, field, wt, s)) return 1;
     mark(plan, s);
     return 0;
 }
 
+// wtab: NULL (weights from the positions) or the remesh weight tables.
 int p2m2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, const void* xp, const FieldGeom& fg,
-               const void* up, void* field, hipStream_t s) {
-#define TYPED(KS)                                                                                           \
-    do {                                                                                                    \
-        if (prec == PPMG_PREC_F64)                                                                          \
-            return p2m2d_typed<KS, double, double>(plan, m, (const double*)xp, fg, (const double*)up,      \
-                                                   (double*)field, s);                                      \
-        if (prec == PPMG_PREC_F32C)                                                                         \
-            return p2m2d_typed<KS, double, float>(plan, m, (const double*)xp, fg, (const float*)up,        \
-                                                  (float*)field, s);                                        \
-        return p2m2d_typed<KS, float, float>(plan, m, (const float*)xp, fg, (const float*)up, (float*)field, s); \
+               const void* up, void* field, const void* const* wtab, hipStream_t s) {
+#define FORM(KS, P, V)                                                                                         \
+    do {                                                                                                       \
+        WTab<V> wt{{nullptr, nullptr, nullptr}};                                                               \
+        if (!wtab) return p2m2d_typed<KS, P, V, false>(plan, m, (const P*)xp, fg, (const V*)up, (V*)field, wt, s); \
+        for (int d = 0; d < 2; ++d) wt.w[d] = (const V*)wtab[d];                                               \
+        return p2m2d_typed<KS, P, V, true>(plan, m, (const P*)xp, fg, (const V*)up, (V*)field, wt, s);         \
+    } while (0)
+#define TYPED(KS)                                            \
+    do {                                                     \
+        if (prec == PPMG_PREC_F64) FORM(KS, double, double); \
+        if (prec == PPMG_PREC_F32C) FORM(KS, double, float); \
+        FORM(KS, float, float);                              \
     } while (0)
     if (kernel == PPMG_KERNEL_BSP2) TYPED(2);
     TYPED(4);
 #undef TYPED
+#undef FORM
 }
 
 }  // namespace ppmg

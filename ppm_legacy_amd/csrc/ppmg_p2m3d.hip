@@ -91,7 +91,7 @@ __device__ __forceinline__ void shift_in(const ValT (&wx)[KS], const ValT (&wz)[
 // fewer halo cells: the window is 16 x (TY+3) cells for 13 x TY nodes.
 //
 // TAB: the 1D weights come from the caller's tables (ppm_rmsh_remesh's
-// wx1/wx2/wx3, four per particle and axis) instead of the positions.
+// wx1/wx2/wx3, KS per particle and axis) instead of the positions.
 //
 // TABLE: the binning is a slot table (byte counts `bt.count`, particle r of
 // cell c at bt.table[r * ncells + c]) instead of heads and a permutation: a
@@ -107,14 +107,13 @@ __global__ void __launch_bounds__(64 * NW)
 k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ up, FieldGeom fg, int c0, int tz,
           ValT* __restrict__ field, WTab<ValT> wt) {
-    static_assert(KS == 4 || !TAB, "weight tables are M'4 only");
     constexpr int H = Stencil<KS>::H, B = Stencil<KS>::B;
     constexpr int TT = 16 - H;                     // owned nodes per tile along x
     constexpr int RP = KS;                         // ring planes
     const int lda = fg.lda;
     // per-particle data besides the strengths: the position, or (TAB) the
-    // twelve 1D weights
-    constexpr int NPD = TAB ? 12 : 3;
+    // 3 KS 1D weights
+    constexpr int NPD = TAB ? 3 * KS : 3;
     using PD = std::conditional_t<TAB, ValT, PosT>;
     using A = LdsAcc<ValT>;
     using slot_t = typename A::slot_t;
@@ -214,7 +213,7 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
 #pragma unroll
-                    for (int o = 0; o < 4; ++o) x[4 * d + o] = wt.w[d][(int64_t)p * 4 + o];
+                    for (int o = 0; o < KS; ++o) x[KS * d + o] = wt.w[d][(int64_t)p * KS + o];
             } else {
 #pragma unroll
                 for (int d = 0; d < 3; ++d) x[d] = xp[(int64_t)p * 3 + d];
@@ -235,8 +234,8 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 #pragma unroll
             for (int o = 0; o < KS; ++o) {
                 wx[o] = x[o];
-                wy[o] = x[4 + o];
-                wz[o] = x[8 + o];
+                wy[o] = x[KS + o];
+                wz[o] = x[2 * KS + o];
             }
         } else {
             ValT fr[3];
@@ -359,7 +358,7 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                         ValT u[LDA], wyz, wxo;
                         load(entry(sf, rr), true, x, u);
                         if constexpr (TAB) {
-                            wyz = x[4 + oy] * x[8 + oz];
+                            wyz = x[KS + oy] * x[2 * KS + oz];
                             wxo = x[ox];
                         } else {
                             ValT fr[3];
@@ -510,13 +509,11 @@ static void launch_p3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, co
 template <int KS, int LL, typename PosT, typename ValT, bool TAB>
 static void launch_p3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
                       const FieldGeom& fg, int c0, ValT* field, const WTab<ValT>& wt, hipStream_t s) {
-    if constexpr (!TAB) {
-        // a slot table (p2m3d_table_applicable: periodic, default tile)
-        if (plan->bin_table) {
-            launch_p3_shape<KS, LL, PosT, ValT, KS == 2 ? 23 : P3_TY, 3, false, false, true>(plan, m, xp, up, perm, fg,
-                                                                                            c0, field, wt, s);
-            return;
-        }
+    // a slot table (p2m3d_table_applicable: periodic, default tile)
+    if (plan->bin_table) {
+        launch_p3_shape<KS, LL, PosT, ValT, KS == 2 ? 23 : P3_TY, 3, false, TAB, true>(plan, m, xp, up, perm, fg, c0,
+                                                                                       field, wt, s);
+        return;
     }
     if (m.periodic[0] && m.periodic[1] && m.periodic[2])
         launch_p3_open<KS, LL, PosT, ValT, false, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
@@ -533,21 +530,17 @@ static int p2m3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const PosT
     if (wtab)
         for (int d = 0; d < 3; ++d) wt.w[d] = wtab[d];
     (void)np;
-    // the slot table is read on a periodic mesh with the default tile, without
-    // weight tables; elsewhere the heads and permutation are built from it
-    if (plan->bin_table && (wtab || !(m.periodic[0] && m.periodic[1] && m.periodic[2]) || (KS == 4 && p3_rows() != P3_TY)))
+    // the slot table is read on a periodic mesh with the default tile;
+    // elsewhere the heads and permutation are built from it
+    if (plan->bin_table && (!(m.periodic[0] && m.periodic[1] && m.periodic[2]) || (KS == 4 && p3_rows() != P3_TY)))
         if (materialize_heads(plan, s)) return 1;
     const int* pk = tile_perm(plan);
     for (int c0 = 0; c0 < lda; c0 += 4) {
         int L = lda - c0 < 4 ? lda - c0 : 4;
 #define TL(LL)                                                                            \
     do {                                                                                  \
-        if constexpr (KS == 4) {                                                          \
-            if (wtab) launch_p3<KS, LL, PosT, ValT, true>(plan, m, xp, up, pk, fg, c0, field, wt, s);   \
-            else launch_p3<KS, LL, PosT, ValT, false>(plan, m, xp, up, pk, fg, c0, field, wt, s);       \
-        } else {                                                                          \
-            launch_p3<KS, LL, PosT, ValT, false>(plan, m, xp, up, pk, fg, c0, field, wt, s);            \
-        }                                                                                 \
+        if (wtab) launch_p3<KS, LL, PosT, ValT, true>(plan, m, xp, up, pk, fg, c0, field, wt, s);      \
+        else launch_p3<KS, LL, PosT, ValT, false>(plan, m, xp, up, pk, fg, c0, field, wt, s);          \
     } while (0)
         if (L == 1) TL(1);
         else if (L == 2) TL(2);
@@ -575,10 +568,7 @@ int p2m3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t 
         return p2m3d_typed<KS, float, float>(plan, m, np, (const float*)xp, fg, (const float*)up,           \
                                              (float*)field, (const float* const*)wtab, s);                  \
     } while (0)
-    if (kernel == PPMG_KERNEL_BSP2) {
-        if (wtab) return PPMG_ERR_ARGUMENT;   // weight tables are M'4 only
-        TYPED(2);
-    }
+    if (kernel == PPMG_KERNEL_BSP2) TYPED(2);
     TYPED(4);
 #undef TYPED
 }

@@ -8,8 +8,8 @@
 
 namespace ppmg {
 
-// Weight tables of ppm_rmsh_remesh (wx1/wx2/wx3, four per particle and axis),
-// used in place of the positions' weights (3D M'4 only).
+// Weight tables of ppm_rmsh_remesh (wx1/wx2/wx3, the stencil width per
+// particle and axis), used in place of the positions' weights.
 template <typename ValT> struct WTab {
     const ValT* w[3];
 };
@@ -134,9 +134,9 @@ __global__ void __launch_bounds__(256) k_box_shell(DevMesh m, FieldGeom fg, int3
         for (int c = 0; c < LL; ++c) acc[c] += (double)(w * u[c]);
     };
     auto add = [&](int p, int ox, int oy, int oz) {
-        if (DIM == 3 && KS == 4 && wt.w[0]) {
-            const ValT w =
-                (wt.w[0][(int64_t)p * 4 + ox] * wt.w[1][(int64_t)p * 4 + oy]) * wt.w[2][(int64_t)p * 4 + oz];
+        if (wt.w[0]) {
+            ValT w = wt.w[0][(int64_t)p * KS + ox] * wt.w[1][(int64_t)p * KS + oy];
+            if constexpr (DIM == 3) w = w * wt.w[2][(int64_t)p * KS + oz];
 #pragma unroll
             for (int c = 0; c < LL; ++c) acc[c] += (double)(w * up[(int64_t)p * fg.lda + c0 + c]);
             return;
