@@ -129,70 +129,159 @@ int ghost_blocks(const DevMesh& m, const int* g, GhostBlock* out) {
     return nb;
 }
 
-// One block, one direction.  Node (i,j,k) (1-based, the reference's
-// numbering) of the block is src + (i,j,k) - 1; its image adds off.
-//   PACK_SRC: buf <- field(src block)        (ghost_get push)
-//   PACK_IMG: buf <- field(image block)      (ghost_put push)
-//   POP_SET:  field(image block) <- buf      (ghost_get pop, replace)
-//   POP_ADD:  field(src block) += buf        (ghost_put pop, add)
+// The blocks of one mapping and where each starts in the pack buffer
+// (elements) and in the launch (workgroups).
+struct GhostList {
+    GhostBlock b[26];
+    int64_t base[27];
+    unsigned wg[27];
+    int64_t per;                // elements per workgroup
+    int N[3];                   // cells per axis (0: not an axis of the mesh)
+    int nb;
+};
+constexpr int GHOST_WG = 256;   // threads per workgroup
+
+// Both steps run as one launch over all blocks, an element per thread: a
+// 3D periodic box has 26 blocks, most of them small, and a launch per block
+// and direction was 52 launches of 4-7 us (256^3 box, ghost size
+// 2, lda 3, FP64: 0.30 ms for ghost_get against 0.05 ms for the two).
+//
+// Node (i,j,k) (1-based, the reference's numbering) of a block is src +
+// (i,j,k) - 1; its image adds off.
+// push: every block is read before any is written,
+//   GET: buf <- field(src block),    PUT: buf <- field(image block).
+// pop, in list order where blocks overlap,
+//   GET: field(image block) <- buf,  PUT: field(src block) += buf.
+// Blocks meet only where a coordinate lies on two images at once, so a node's
+// whole list is carried out by one thread: for GET the node's last block (the
+// value the list leaves), for PUT its first block, which adds the buffered
+// values of every block of the node in list order.
 // LOGIC: the elements are logicals (nonzero = .TRUE.), set as 1 / 0; the pop
 // adds by .AND.  mask (nullptr: every node) holds one logical per stored node.
-enum GhostOp { PACK_SRC = 0, PACK_IMG = 1, POP_SET = 2, POP_ADD = 3 };
 
-template <typename T, bool LOGIC>
-__global__ void __launch_bounds__(256) k_ghost_block(T* __restrict__ field, FieldGeom fg, GhostBlock b,
-                                                     T* __restrict__ buf, int op, const int* __restrict__ mask) {
-    const int lda = fg.lda;
-    const int64_t n = (int64_t)b.size[0] * b.size[1] * b.size[2] * lda;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(e % lda);
-        int64_t r = e / lda;
-        const int i = (int)(r % b.size[0]);
-        r /= b.size[0];
-        const int j = (int)(r % b.size[1]);
-        const int k = (int)(r / b.size[1]);
-        const bool img = op == PACK_IMG || op == POP_SET;
-        // 0-based node index, then the stored box
-        const int nx = b.src[0] + i - 1 + (img ? b.off[0] : 0);
-        const int ny = b.src[1] + j - 1 + (img ? b.off[1] : 0);
-        const int nz = b.src[2] + k - 1 + (img ? b.off[2] : 0);
-        const int64_t node = ((int64_t)(nz - fg.lo[2]) * fg.ext[1] + (ny - fg.lo[1])) * fg.ext[0] + (nx - fg.lo[0]);
-        const int64_t at = node * lda + c;
-        if (op == PACK_SRC || op == PACK_IMG) {
-            buf[e] = field[at];
-            continue;
-        }
-        if (mask && mask[node] == 0) continue;
-        if constexpr (LOGIC) {
-            const bool v = buf[e] != T(0);
-            field[at] = (op == POP_SET ? v : (field[at] != T(0) && v)) ? T(1) : T(0);
-        } else if constexpr (std::is_integral<T>::value) {
-            // two's-complement wrap on overflow, as the hardware add
-            field[at] = op == POP_SET ? buf[e] : (T)((uint32_t)field[at] + (uint32_t)buf[e]);
-        } else {
-            field[at] = op == POP_SET ? buf[e] : field[at] + buf[e];
-        }
+// This workgroup's block.
+__device__ __forceinline__ int ghost_block_of(const GhostList& l) {
+    int q = 0;
+    while (blockIdx.x >= l.wg[q + 1]) ++q;
+    return q;
+}
+
+// Component and 0-based real node of element e of block b.
+__device__ __forceinline__ void ghost_element(const GhostBlock& b, int lda, int64_t e, int& c, int (&n)[3]) {
+    auto split = [&](auto r) {   // 32-bit divisions wherever e fits
+        using U = decltype(r);
+        const U node = r / (U)lda;
+        c = (int)(r - node * (U)lda);
+        const U row = node / (U)b.size[0];
+        n[0] = (int)(node - row * (U)b.size[0]);
+        const U pl = row / (U)b.size[1];
+        n[1] = (int)(row - pl * (U)b.size[1]);
+        n[2] = (int)pl;
+    };
+    if ((uint64_t)e >> 32) split((uint64_t)e);
+    else split((uint32_t)e);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) n[d] += b.src[d] - 1;
+}
+
+__device__ __forceinline__ int64_t ghost_node(const FieldGeom& fg, const int (&n)[3]) {
+    return ((int64_t)(n[2] - fg.lo[2]) * fg.ext[1] + (n[1] - fg.lo[1])) * fg.ext[0] + (n[0] - fg.lo[0]);
+}
+
+// Node n (0-based) in block b's real nodes (img false) or their images (true).
+__device__ __forceinline__ bool ghost_holds(const GhostBlock& b, const int (&n)[3], bool img) {
+    bool in = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int i = n[d] - (b.src[d] - 1) - (img ? b.off[d] : 0);
+        in = in && i >= 0 && i < b.size[d];
+    }
+    return in;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(GHOST_WG) k_ghost_push(const T* __restrict__ field, FieldGeom fg, GhostList l,
+                                                         T* __restrict__ buf, bool get) {
+    const int q = ghost_block_of(l);
+    const GhostBlock& b = l.b[q];
+    const int64_t e0 = (int64_t)(blockIdx.x - l.wg[q]) * l.per;
+    const int64_t e1 = min(e0 + l.per, l.base[q + 1] - l.base[q]);
+    for (int64_t e = e0 + threadIdx.x; e < e1; e += GHOST_WG) {
+        int c, n[3];
+        ghost_element(b, fg.lda, e, c, n);
+        if (!get)
+            for (int d = 0; d < 3; ++d) n[d] += b.off[d];
+        buf[l.base[q] + e] = field[ghost_node(fg, n) * fg.lda + c];
     }
 }
 
 template <typename T, bool LOGIC>
-static int ghost_typed(T* field, const FieldGeom& fg, const GhostBlock* b, int nb, bool get, const int* mask,
-                       DevBuf& scratch, hipStream_t s) {
-    int64_t base[27];
-    base[0] = 0;
-    for (int q = 0; q < nb; ++q) base[q + 1] = base[q] + (int64_t)b[q].size[0] * b[q].size[1] * b[q].size[2] * fg.lda;
-    if (base[nb] == 0) return 0;
-    if (scratch.ensure(sizeof(T) * (size_t)base[nb])) return PPMG_ERROR_FATAL;
+__global__ void __launch_bounds__(GHOST_WG) k_ghost_pop(T* __restrict__ field, FieldGeom fg, GhostList l,
+                                                        const T* __restrict__ buf, bool get,
+                                                        const int* __restrict__ mask) {
+    const int q = ghost_block_of(l);
+    const int64_t e0 = (int64_t)(blockIdx.x - l.wg[q]) * l.per;
+    const int64_t e1 = min(e0 + l.per, l.base[q + 1] - l.base[q]);
+    for (int64_t e = e0 + threadIdx.x; e < e1; e += GHOST_WG) {
+        int c, n[3];
+        ghost_element(l.b[q], fg.lda, e, c, n);
+        bool other = false;   // another block's thread carries out this node's list
+        if (get) {
+            for (int d = 0; d < 3; ++d) n[d] += l.b[q].off[d];
+            // two images of the real range 0..N meet on the nodes 0 and N only
+            bool seam = false;
+            for (int d = 0; d < 3; ++d) seam = seam || (l.N[d] && (n[d] == 0 || n[d] == l.N[d]));
+            if (seam)
+                for (int p = q + 1; p < l.nb && !other; ++p) other = ghost_holds(l.b[p], n, true);
+        } else {
+            for (int p = 0; p < q && !other; ++p) other = ghost_holds(l.b[p], n, false);
+        }
+        if (other) continue;
+        const int64_t node = ghost_node(fg, n);
+        if (mask && mask[node] == 0) continue;
+        T* at = field + node * fg.lda + c;
+        if (get) {
+            const T v = buf[l.base[q] + e];
+            if constexpr (LOGIC) *at = v != T(0) ? T(1) : T(0);
+            else *at = v;
+            continue;
+        }
+        T v = *at;
+        for (int p = q; p < l.nb; ++p) {
+            const GhostBlock& b = l.b[p];
+            if (!ghost_holds(b, n, false)) continue;
+            const T w = buf[l.base[p] +
+                            (((int64_t)(n[2] - (b.src[2] - 1)) * b.size[1] + (n[1] - (b.src[1] - 1))) * b.size[0] +
+                             (n[0] - (b.src[0] - 1))) * fg.lda + c];
+            if constexpr (LOGIC) v = v != T(0) && w != T(0) ? T(1) : T(0);
+            else if constexpr (std::is_integral<T>::value) v = (T)((uint32_t)v + (uint32_t)w);   // wraps, as the hardware add
+            else v = v + w;
+        }
+        *at = v;
+    }
+}
+
+template <typename T, bool LOGIC>
+static int ghost_typed(const DevMesh& m, T* field, const FieldGeom& fg, const GhostBlock* b, int nb, bool get,
+                       const int* mask, DevBuf& scratch, hipStream_t s) {
+    GhostList l;
+    l.nb = nb;
+    for (int d = 0; d < 3; ++d) l.N[d] = d < m.dim ? m.N[d] : 0;
+    l.base[0] = 0;
+    for (int q = 0; q < nb; ++q) {
+        l.b[q] = b[q];
+        l.base[q + 1] = l.base[q] + (int64_t)b[q].size[0] * b[q].size[1] * b[q].size[2] * fg.lda;
+    }
+    if (l.base[nb] == 0) return 0;
+    // one element per thread, more where that would be over 2^20 workgroups
+    l.per = GHOST_WG * ((l.base[nb] >> 28) + 1);
+    l.wg[0] = 0;
+    for (int q = 0; q < nb; ++q) l.wg[q + 1] = l.wg[q] + (unsigned)((l.base[q + 1] - l.base[q] + l.per - 1) / l.per);
+    const unsigned wg = l.wg[nb];
+    if (scratch.ensure(sizeof(T) * (size_t)l.base[nb])) return PPMG_ERROR_FATAL;
     T* buf = scratch.as<T>();
-    auto grid = [](int64_t n) { return dim3((unsigned)((n + 255) / 256 < 65536 ? (n + 255) / 256 : 65536)); };
-    // push: every block is read before any is written
-    for (int q = 0; q < nb; ++q)
-        hipLaunchKernelGGL((k_ghost_block<T, LOGIC>), grid(base[q + 1] - base[q]), dim3(256), 0, s, field, fg, b[q],
-                           buf + base[q], get ? (int)PACK_SRC : (int)PACK_IMG, (const int*)nullptr);
-    // pop, in list order (a launch per block keeps the order of overlapping blocks)
-    for (int q = 0; q < nb; ++q)
-        hipLaunchKernelGGL((k_ghost_block<T, LOGIC>), grid(base[q + 1] - base[q]), dim3(256), 0, s, field, fg, b[q],
-                           buf + base[q], get ? (int)POP_SET : (int)POP_ADD, mask);
+    hipLaunchKernelGGL(k_ghost_push<T>, dim3(wg), dim3(GHOST_WG), 0, s, field, fg, l, buf, get);
+    hipLaunchKernelGGL((k_ghost_pop<T, LOGIC>), dim3(wg), dim3(GHOST_WG), 0, s, field, fg, l, buf, get, mask);
     PPMG_HIP(hipGetLastError());
     return 0;
 }
@@ -203,16 +292,16 @@ int map_field_ghost(const DevMesh& m, int kind, const FieldGeom& fg_in, void* fi
     const int nb = ghost_blocks(m, g, b);
     FieldGeom fg = fg_in;
     switch (kind) {
-    case PPMG_KIND_D: return ghost_typed<double, false>((double*)field, fg, b, nb, get, mask, scratch, s);
-    case PPMG_KIND_S: return ghost_typed<float, false>((float*)field, fg, b, nb, get, mask, scratch, s);
-    case PPMG_KIND_I: return ghost_typed<int, false>((int*)field, fg, b, nb, get, mask, scratch, s);
-    case PPMG_KIND_L: return ghost_typed<int, true>((int*)field, fg, b, nb, get, mask, scratch, s);
+    case PPMG_KIND_D: return ghost_typed<double, false>(m, (double*)field, fg, b, nb, get, mask, scratch, s);
+    case PPMG_KIND_S: return ghost_typed<float, false>(m, (float*)field, fg, b, nb, get, mask, scratch, s);
+    case PPMG_KIND_I: return ghost_typed<int, false>(m, (int*)field, fg, b, nb, get, mask, scratch, s);
+    case PPMG_KIND_L: return ghost_typed<int, true>(m, (int*)field, fg, b, nb, get, mask, scratch, s);
     case PPMG_KIND_DC:
         fg.lda *= 2;   // (re, im) pairs: each part maps and adds as a real component
-        return ghost_typed<double, false>((double*)field, fg, b, nb, get, mask, scratch, s);
+        return ghost_typed<double, false>(m, (double*)field, fg, b, nb, get, mask, scratch, s);
     case PPMG_KIND_SC:
         fg.lda *= 2;
-        return ghost_typed<float, false>((float*)field, fg, b, nb, get, mask, scratch, s);
+        return ghost_typed<float, false>(m, (float*)field, fg, b, nb, get, mask, scratch, s);
     default:
         set_error(PPMG_ERROR_ERROR, PPMG_ERR_ARGUMENT, "unknown element kind");
         return PPMG_ERROR_ERROR;
