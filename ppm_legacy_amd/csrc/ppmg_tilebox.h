@@ -3,6 +3,8 @@
 // whose stored box holds the whole real range, and the ghost layers.  Shared
 // by ppmg_p2m2d.hip and ppmg_p2m3d.hip.
 #pragma once
+#include <type_traits>
+
 #include "ppmg_internal.h"
 #include "ppmg_sort.h"
 
@@ -64,205 +66,161 @@ __global__ void __launch_bounds__(256) k_box_dup(FieldGeom fg, int3 n, int3 r, i
 // width (4 M'4, 2 BSP2); DIM 2: one plane (no z stencil), positions of two
 // coordinates.  TABLE: the binning is a slot table instead of heads and a
 // permutation; a cell's particles come in the same order.
+//
+// Bound by latency: a node's cells (at most 16 on a periodic box, whose
+// outside axis meets one stencil offset) lead to list heads and then to
+// particles, a chain of two loads, with little arithmetic.  Four lanes share a
+// node, cell j going to lane j mod 4; a lane has the heads of four cells and
+// then their first particles in flight at once, so a node takes one pass of the
+// chain, and the short register list leaves many wavefronts resident.  The
+// four partial sums are added in a fixed order.  (One lane per node, 16 heads
+// and then four batches of four particles, against this: 115 and 84 us at
+// 256^3, ghost size 2, lda 3, FP32c; 40 and 11 us at 64^3, FP64.)
+constexpr int SHELL_LANES = 4;   // lanes per node (a DPP quad)
+constexpr int SHELL_CELLS = 4;   // cells per lane and pass
+
+// Sum over the lanes of a quad, in the same order in every lane.
+__device__ __forceinline__ double quad_sum(double v) {
+    auto perm = [](double w, auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(w), C, 0xF, 0xF, true);
+        const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(w), C, 0xF, 0xF, true);
+        return __hiloint2double(hi, lo);
+    };
+    v += perm(v, std::integral_constant<int, 0xB1>{});   // lanes 1 0 3 2
+    v += perm(v, std::integral_constant<int, 0x4E>{});   // lanes 2 3 0 1
+    return v;
+}
+
 template <int DIM, int KS, typename PosT, typename ValT, int LL, bool TABLE>
 __global__ void __launch_bounds__(256) k_box_shell(DevMesh m, FieldGeom fg, int3 r, const int* __restrict__ start,
                                                   const int* __restrict__ perm, BinTable bt,
                                                   const PosT* __restrict__ xp, const ValT* __restrict__ up, int c0,
-                                                  ValT* __restrict__ field, int64_t nshell, WTab<ValT> wt) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nshell) return;
+                                                  ValT* __restrict__ field, int64_t t0, int64_t nshell,
+                                                  WTab<ValT> wt) {
+    const int sub = threadIdx.x & (SHELL_LANES - 1);
+    const int64_t tq = t0 + ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / SHELL_LANES;
+    const bool live = tq < nshell;   // a quad past the end works on the last node and stores nothing
+    const int64_t t = live ? tq : nshell - 1;
     const int e0 = fg.ext[0], e1 = fg.ext[1], e2 = fg.ext[2];
     const int o0 = e0 - r.x, o1 = e1 - r.y, o2 = e2 - r.z;
     // q-th stored node of axis d outside the real range: below 0, then above N
     auto outer = [&](int d, int q) { return q < -fg.lo[d] ? fg.lo[d] + q : m.N[d] + 1 + (q + fg.lo[d]); };
-    const int64_t ra = (int64_t)o2 * e1 * e0, rb = (int64_t)r.z * o1 * e0;
     int n[3];
-    if (t < ra) {
-        n[0] = fg.lo[0] + (int)(t % e0);
-        n[1] = fg.lo[1] + (int)((t / e0) % e1);
-        n[2] = outer(2, (int)(t / ((int64_t)e0 * e1)));
-    } else if (t < ra + rb) {
-        const int64_t q = t - ra;
-        n[0] = fg.lo[0] + (int)(q % e0);
-        n[1] = outer(1, (int)((q / e0) % o1));
-        n[2] = (int)(q / ((int64_t)e0 * o1));
-    } else {
-        const int64_t q = t - ra - rb;
-        n[0] = outer(0, (int)(q % o0));
-        n[1] = (int)((q / o0) % r.y);
-        n[2] = (int)(q / ((int64_t)o0 * r.y));
-    }
+    auto locate = [&](auto q) {   // 32-bit divisions wherever the shell's node count fits
+        using U = decltype(q);
+        const U ra = (U)o2 * (U)e1 * (U)e0, rb = (U)r.z * (U)o1 * (U)e0;
+        if (q < ra) {
+            const U row = q / (U)e0, pl = row / (U)e1;
+            n[0] = fg.lo[0] + (int)(q - row * (U)e0);
+            n[1] = fg.lo[1] + (int)(row - pl * (U)e1);
+            n[2] = outer(2, (int)pl);
+        } else if (q < ra + rb) {
+            q -= ra;
+            const U row = q / (U)e0, pl = row / (U)o1;
+            n[0] = fg.lo[0] + (int)(q - row * (U)e0);
+            n[1] = outer(1, (int)(row - pl * (U)o1));
+            n[2] = (int)pl;
+        } else {
+            q -= ra + rb;
+            const U row = q / (U)o0, pl = row / (U)r.y;
+            n[0] = outer(0, (int)(q - row * (U)o0));
+            n[1] = (int)(row - pl * (U)r.y);
+            n[2] = (int)pl;
+        }
+    };
+    if ((uint64_t)nshell >> 32) locate((uint64_t)t);
+    else locate((uint32_t)t);
     double acc[LL];
 #pragma unroll
     for (int c = 0; c < LL; ++c) acc[c] = 0.0;
     constexpr int B = Stencil<KS>::B;
-    // The stencil offsets o of each axis whose cell n + B - o exists, walked
-    // in the order z, y, x (x fastest) with the next cell's list head (count
-    // and first particle) fetched while the current cell is summed: the same
-    // additions in the same order as a plain loop over the KS^DIM offsets,
-    // with one cell's lookups in flight instead of none.
-    int olo[3], ohi[3];
+    // The stencil offsets of each axis whose cell n + B - o exists: olo ..
+    // olo + num - 1.  Cell j of the num[0] num[1] num[2] cells counts x fastest.
+    int olo[3], num[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         olo[d] = d < DIM ? max(0, n[d] + B - (m.nbin[d] - 1)) : 0;
-        ohi[d] = d < DIM ? min(KS - 1, n[d] + B) : 0;
+        num[d] = d < DIM ? max(0, min(KS - 1, n[d] + B) - olo[d] + 1) : 1;
     }
-    auto key_of = [&](int ox, int oy, int oz) {
-        const int cz = DIM == 3 ? n[2] + B - oz : 0;
-        return (n[0] + B - ox) + m.nbin[0] * ((n[1] + B - oy) + m.nbin[1] * cz);
-    };
-    // list of cell `key`: particles q in [b, e), particle p0 at q = b (if any)
-    auto head = [&](int key, int& b, int& e, int& p0) {
-        b = TABLE ? 0 : start[key];
-        e = TABLE ? (int)((bt.count[count_word(key)] >> count_shift(key)) & 255u) : start[key + 1];
-        p0 = e > b ? (TABLE ? bt.table[key] : perm ? perm[b] : b) : 0;
-    };
+    const int ncell = num[0] * num[1] * num[2];
+    // j / k for j < 64 and k = 1..4
+    auto quotient = [](int j, int k) { return (j * (k == 1 ? 257 : k == 2 ? 129 : k == 3 ? 86 : 65)) >> 8; };
     auto particle_of = [&](int key, int q) {
         return TABLE ? bt.table[(int64_t)q * bt.ncells + key] : perm ? perm[q] : q;
     };
-    // one particle's contribution from its position and strengths
-    auto add_vals = [&](const PosT (&x)[DIM], const ValT (&u)[LL], int ox, int oy, int oz) {
-        ValT fr[DIM];
+    const bool tab = wt.w[0] != nullptr;
+    // a particle's position or, with tables, its weights at the offsets o
+    // (a weight converts to the position type and back exactly)
+    auto load = [&](int p, const int (&o)[3], PosT (&x)[DIM], ValT (&u)[LL]) {
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+            x[d] = tab ? (PosT)wt.w[d][(int64_t)p * KS + o[d]] : xp[(int64_t)p * DIM + d];
+#pragma unroll
+        for (int c = 0; c < LL; ++c) u[c] = up[(int64_t)p * fg.lda + c0 + c];
+    };
+    auto add = [&](const int (&o)[3], const PosT (&x)[DIM], const ValT (&u)[LL]) {
+        ValT w1[DIM];
 #pragma unroll
         for (int d = 0; d < DIM; ++d) {
             int ci;
-            fr[d] = (ValT)cell_offset<PosT>(x[d], (PosT)m.minv[d], (PosT)m.dxi[d], ci);
+            w1[d] = tab ? (ValT)x[d]
+                        : tile_weight_at<KS, ValT>(
+                              (ValT)cell_offset<PosT>(x[d], (PosT)m.minv[d], (PosT)m.dxi[d], ci), o[d]);
         }
-        ValT w = tile_weight_at<KS, ValT>(fr[0], ox) * tile_weight_at<KS, ValT>(fr[1], oy);
-        if constexpr (DIM == 3) w = w * tile_weight_at<KS, ValT>(fr[2], oz);
+        ValT w = w1[0] * w1[1];
+        if constexpr (DIM == 3) w = w * w1[2];
 #pragma unroll
         for (int c = 0; c < LL; ++c) acc[c] += (double)(w * u[c]);
     };
-    auto add = [&](int p, int ox, int oy, int oz) {
-        if (wt.w[0]) {
-            ValT w = wt.w[0][(int64_t)p * KS + ox] * wt.w[1][(int64_t)p * KS + oy];
-            if constexpr (DIM == 3) w = w * wt.w[2][(int64_t)p * KS + oz];
+    for (int j0 = sub; j0 < ncell; j0 += SHELL_LANES * SHELL_CELLS) {
+        int o[SHELL_CELLS][3], key[SHELL_CELLS], b[SHELL_CELLS], e[SHELL_CELLS], p[SHELL_CELLS];
 #pragma unroll
-            for (int c = 0; c < LL; ++c) acc[c] += (double)(w * up[(int64_t)p * fg.lda + c0 + c]);
-            return;
+        for (int i = 0; i < SHELL_CELLS; ++i) {
+            const int j = j0 + SHELL_LANES * i;
+            const int row = quotient(j, num[0]), pl = quotient(row, num[1]);
+            o[i][0] = olo[0] + j - row * num[0];
+            o[i][1] = olo[1] + row - pl * num[1];
+            o[i][2] = olo[2] + pl;
+            key[i] = b[i] = e[i] = p[i] = 0;
+            if (j < ncell) {
+                const int cz = DIM == 3 ? n[2] + B - o[i][2] : 0;
+                key[i] = (n[0] + B - o[i][0]) + m.nbin[0] * ((n[1] + B - o[i][1]) + m.nbin[1] * cz);
+                if constexpr (TABLE) {
+                    e[i] = (int)bt.count[count_word(key[i])];   // decoded below: the loads stay in flight
+                    p[i] = bt.table[key[i]];
+                } else {
+                    b[i] = start[key[i]];
+                    e[i] = start[key[i] + 1];
+                }
+            }
         }
-        PosT x[DIM];
-        ValT u[LL];
+        PosT x[SHELL_CELLS][DIM];
+        ValT u[SHELL_CELLS][LL];
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) x[d] = xp[(int64_t)p * DIM + d];
+        for (int i = 0; i < SHELL_CELLS; ++i) {
+            if constexpr (TABLE) e[i] = j0 + SHELL_LANES * i < ncell ? (int)(((unsigned)e[i] >> count_shift(key[i])) & 255u) : 0;
+            if (e[i] > b[i]) {
+                if constexpr (!TABLE) p[i] = perm ? perm[b[i]] : b[i];
+                load(p[i], o[i], x[i], u[i]);
+            }
+        }
 #pragma unroll
-        for (int c = 0; c < LL; ++c) u[c] = up[(int64_t)p * fg.lda + c0 + c];
-        add_vals(x, u, ox, oy, oz);
-    };
-    // A node outside the real range on an axis f of a periodic 3D M'4 box
-    // meets one stencil offset there (node -1: cell 0, node N+1: cell N-1),
-    // so its cells are at most 4 x 4 along the other two axes: they are taken
-    // as 16 fixed slots (outer free axis, then inner), all 16 list heads
-    // loaded at once and the first particles (position or table weights, and
-    // strengths) of 4 slots at a time, then summed in the same order as the
-    // walk below.
-    int f = -1;
-    if constexpr (DIM == 3 && KS == 4) {
-        if (olo[0] <= ohi[0] && olo[1] <= ohi[1] && olo[2] <= ohi[2]) {
-#pragma unroll
-            for (int d = 2; d >= 0; --d)
-                if (olo[d] == ohi[d]) f = d;
+        for (int i = 0; i < SHELL_CELLS; ++i) {
+            if (e[i] > b[i]) {
+                add(o[i], x[i], u[i]);
+                for (int q = b[i] + 1; q < e[i]; ++q) {
+                    PosT xq[DIM];
+                    ValT uq[LL];
+                    load(particle_of(key[i], q), o[i], xq, uq);
+                    add(o[i], xq, uq);
+                }
+            }
         }
     }
-    if (f >= 0) {
-        const int A = f == 2 ? 1 : 2, Bx = f == 0 ? 1 : 0;   // outer and inner free axes
-        auto offs = [&](int sl, int& ox, int& oy, int& oz) {
-            int o[3];
-            o[f] = olo[f];
-            o[A] = olo[A] + (sl >> 2);
-            o[Bx] = olo[Bx] + (sl & 3);
-            ox = o[0];
-            oy = o[1];
-            oz = o[2];
-            return o[A] <= ohi[A] && o[Bx] <= ohi[Bx];
-        };
-        int cb[16], ce[16], cp[16];
 #pragma unroll
-        for (int sl = 0; sl < 16; ++sl) {
-            int ox, oy, oz;
-            cb[sl] = ce[sl] = cp[sl] = 0;
-            if (offs(sl, ox, oy, oz)) head(key_of(ox, oy, oz), cb[sl], ce[sl], cp[sl]);
-        }
-#pragma unroll
-        for (int s0 = 0; s0 < 16; s0 += 4) {
-            // one batch's particle loads in flight at a time (register bound)
-            asm volatile("" ::: "memory");
-            // per slot: the position, or with weight tables the particle's
-            // three table weights at the slot's offsets (held in the same
-            // registers: a weight converts to the position type and back
-            // exactly)
-            PosT xs[4][DIM];
-            ValT us[4][LL];
-            const bool tab = wt.w[0] != nullptr;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (ce[s0 + j] > cb[s0 + j]) {
-                    const int p = cp[s0 + j];
-                    if (tab) {
-                        int ox, oy, oz;
-                        offs(s0 + j, ox, oy, oz);
-                        xs[j][0] = (PosT)wt.w[0][(int64_t)p * 4 + ox];
-                        xs[j][1] = (PosT)wt.w[1][(int64_t)p * 4 + oy];
-                        xs[j][2] = (PosT)wt.w[2][(int64_t)p * 4 + oz];
-                    } else {
-#pragma unroll
-                        for (int d = 0; d < DIM; ++d) xs[j][d] = xp[(int64_t)p * DIM + d];
-                    }
-#pragma unroll
-                    for (int c = 0; c < LL; ++c) us[j][c] = up[(int64_t)p * fg.lda + c0 + c];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int sl = s0 + j;
-                if (ce[sl] > cb[sl]) {
-                    int ox, oy, oz;
-                    offs(sl, ox, oy, oz);
-                    if (tab) {
-                        const ValT w = ((ValT)xs[j][0] * (ValT)xs[j][1]) * (ValT)xs[j][2];
-#pragma unroll
-                        for (int c = 0; c < LL; ++c) acc[c] += (double)(w * us[j][c]);
-                    } else {
-                        add_vals(xs[j], us[j], ox, oy, oz);
-                    }
-                    for (int q = cb[sl] + 1; q < ce[sl]; ++q) add(particle_of(key_of(ox, oy, oz), q), ox, oy, oz);
-                }
-            }
-        }
-    } else if (olo[0] <= ohi[0] && olo[1] <= ohi[1] && olo[2] <= ohi[2]) {
-        int ox = olo[0], oy = olo[1], oz = olo[2];
-        int key = key_of(ox, oy, oz), b, e, p0;
-        head(key, b, e, p0);
-        for (;;) {
-            // the cell after this one
-            int nx = ox + 1, ny = oy, nz = oz;
-            if (nx > ohi[0]) {
-                nx = olo[0];
-                if (++ny > ohi[1]) {
-                    ny = olo[1];
-                    ++nz;
-                }
-            }
-            const bool more = nz <= ohi[2];
-            int nkey = 0, nb = 0, ne = 0, np0 = 0;
-            if (more) {
-                nkey = key_of(nx, ny, nz);
-                head(nkey, nb, ne, np0);
-            }
-            if (e > b) {
-                add(p0, ox, oy, oz);
-                for (int q = b + 1; q < e; ++q) add(particle_of(key, q), ox, oy, oz);
-            }
-            if (!more) break;
-            ox = nx;
-            oy = ny;
-            oz = nz;
-            key = nkey;
-            b = nb;
-            e = ne;
-            p0 = np0;
-        }
-    }
+    for (int c = 0; c < LL; ++c) acc[c] = quad_sum(acc[c]);
+    if (!live || sub != 0) return;
     ValT* out = field + (((int64_t)(n[2] - fg.lo[2]) * e1 + (n[1] - fg.lo[1])) * e0 + (n[0] - fg.lo[0])) * fg.lda + c0;
 #pragma unroll
     for (int c = 0; c < LL; ++c) out[c] = (ValT)acc[c];
@@ -289,18 +247,23 @@ int fill_stored_box(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const Val
                            field, ndup);
     const int64_t nshell = (int64_t)fg.ext[0] * fg.ext[1] * fg.ext[2] - (int64_t)R[0] * R[1] * R[2];
     if (nshell > 0) {
-        const unsigned g = (unsigned)((nshell + 255) / 256);
         const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
         const bool table = plan->bin_table;
         if (!table && materialize_heads(plan, s)) return 1;
         for (int c0 = 0; c0 < lda; c0 += 4) {
             const int L = lda - c0 < 4 ? lda - c0 : 4;
-#define SH(LL, TB) hipLaunchKernelGGL((k_box_shell<DIM, KS, PosT, ValT, LL, TB>), dim3(g), dim3(256), 0, s, m, fg, r3, \
-                                      plan->start.as<int>(), tile_perm(plan), bt, xp, up, c0, field, nshell, wt)
+// (2^28 nodes a launch: under 2^32 threads)
+#define SH(LL, TB)                                                                                                    \
+    for (int64_t t0 = 0; t0 < nshell; t0 += (int64_t)1 << 28) {                                                       \
+        const int64_t nt = nshell - t0 < ((int64_t)1 << 28) ? nshell - t0 : (int64_t)1 << 28;                          \
+        hipLaunchKernelGGL((k_box_shell<DIM, KS, PosT, ValT, LL, TB>),                                                \
+                           dim3((unsigned)((nt * SHELL_LANES + 255) / 256)), dim3(256), 0, s, m, fg, r3,              \
+                           plan->start.as<int>(), tile_perm(plan), bt, xp, up, c0, field, t0, t0 + nt, wt);           \
+    }
 #define SHL(LL)                      \
     do {                             \
-        if (table) SH(LL, true);     \
-        else SH(LL, false);          \
+        if (table) SH(LL, true)      \
+        else SH(LL, false)           \
     } while (0)
             if (L == 1) SHL(1);
             else if (L == 2) SHL(2);
