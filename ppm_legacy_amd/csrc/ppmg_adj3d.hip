@@ -19,7 +19,6 @@
 //   dL/dx_1 = sum_c u_c sum_k wx_k Cy_k, dL/dx_2 = sum_c u_c sum_k wx_k Cz_k.
 // All sums are FP64 in registers; the FP32 forms keep FP32 only for g, u and
 // the outputs.
-#include <atomic>
 
 #include "ppmg_internal.h"
 #include "ppmg_interp.h"
@@ -383,11 +382,13 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 template <int LL, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE = false>
 static void launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
                            const FieldGeom& fg, ValT* gu, ValT* gx, int lda, int c0, int acc, hipStream_t s) {
-    static std::atomic<int> slots{0};
-    if (slots.load() == 0)
-        slots.store(resident_workgroups(k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>, A3_THREADS));
+    static const Residency res = residency(k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>, A3_THREADS);
     const int tx = (m.N[0] + A3_TX - 1) / A3_TX, ty = (m.N[1] + A3_TY - 1) / A3_TY;
-    const int tz = pick_z_chunk_balanced((int64_t)tx * ty, m.N[2], slots.load(), 32);
+    // a step is long here: a chunk's three extra plane loads weigh little
+    const int64_t ncells = (int64_t)m.N[0] * m.N[1] * m.N[2];
+    const int tz = plan->crowded_cells > ncells / 1024
+                       ? pick_z_chunk_balanced((int64_t)tx * ty, m.N[2], res.slots(), 32)
+                       : pick_chunk((int64_t)tx * ty, m.N[2], res, 0.3, 0.3);
     dim3 grid((unsigned)((int64_t)tx * ty * ((m.N[2] + tz - 1) / tz)));
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
     hipLaunchKernelGGL((k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>), grid, dim3(A3_THREADS), 0, s, m,

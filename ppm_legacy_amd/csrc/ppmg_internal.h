@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <cmath>
 #include <cstring>
 #include <string>
 
@@ -81,20 +82,64 @@ __device__ __forceinline__ T scaled_coord(T x, T mn, T dxi) {
 }
 
 // ------------------------------------------------------ z-chunk choice --
-// Workgroups of `kernel` (launched with `threads` threads) resident on the
-// whole device at once, from the occupancy API (cached by the caller).
+// Compute units of the device and workgroups of `kernel` (launched with
+// `threads` threads) resident on each, from the occupancy API (cached by the
+// caller).
+struct Residency {
+    int cus, per_cu;
+    int slots() const { return cus * per_cu; }
+};
 template <typename K>
-inline int resident_workgroups(K kernel, int threads) {
+inline Residency residency(K kernel, int threads) {
     int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 1;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess) return 1;
-    return cus * per_cu > 0 ? cus * per_cu : 1;
+    if (hipGetDevice(&dev) != hipSuccess) return {1, 1};
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return {1, 1};
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess) return {1, 1};
+    return cus > 0 && per_cu > 0 ? Residency{cus, per_cu} : Residency{1, 1};
+}
+template <typename K>
+inline int resident_workgroups(K kernel, int threads) { return residency(kernel, threads).slots(); }
+
+// Cell planes per workgroup of the 3D tile kernels: the candidate with the
+// least modelled time, (chunk + halo) plane steps of the time a step takes
+// with the compute units so loaded.  A workgroup alone on its unit waits for
+// its own chain of loads and barriers (the unit of time here); with all
+// per_cu resident a step takes 1.85 of it, and beyond that the launch takes
+// its workgroups in turn, with about one more per unit as its tail.  (Deposit,
+// FP64, lda 3: 10, 11.4, 12.9, 14.3 and 18 us a step with 1 to 5 workgroups
+// on a unit.)  halo: planes of extra work per chunk once the device is full,
+// halo_few: while workgroups wait for themselves.  Long chunks are left out:
+// tiles that march far apart stop sharing their halos in L2.  Chunks start at
+// one plane, so that a small mesh still spreads over the device: deposit of
+// 32^3 cells 116 -> 47 us (8 against 1 plane), 64^3 125 -> 88 us (2), 192^3
+// 643 -> 563 us (24), 256^3 1434 -> 1235 us (64 against 32); adjoint of 32^3
+// 99 -> 22 us, 64^3 112 -> 55 us, 96^3 177 -> 135 us.
+inline int pick_chunk(int64_t tiles_xy, int planes, const Residency& r, double halo, double halo_few) {
+    static const int sizes[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    int best = 1;
+    double best_cost = -1.0;
+    for (int c : sizes) {
+        if (c > planes && c > 1) break;
+        const double load = (double)(tiles_xy * (int64_t)((planes + c - 1) / c)) / r.cus;
+        double cost;
+        if (load <= r.per_cu) {
+            const double k = ceil(load) - 1.0;
+            const double x = r.per_cu > 1 ? k / (r.per_cu - 1) : 1.0;
+            cost = (c + halo_few) * (1.0 + 0.85 * x * sqrt(x));
+        } else {
+            cost = (c + halo) * 1.85 * (load + 1.0) / r.per_cu;
+        }
+        if (best_cost < 0.0 || cost <= best_cost) {
+            best_cost = cost;
+            best = c;
+        }
+    }
+    return best;
 }
 
-// Cell planes per workgroup for the z-marching tile kernels.  A workgroup
-// spends ~(tz + halo) plane steps; the launch takes ceil(workgroups / slots)
-// such rounds.  Picks the chunk with the fewest plane steps overall (larger
+// Cell rows per workgroup of the 2D tile kernels.  A workgroup
+// spends ~(tz + halo) row steps; the launch takes ceil(workgroups / slots)
+// such rounds.  Picks the chunk with the fewest steps overall (larger
 // chunk on ties), so small meshes still fill the device and large ones march
 // long chunks with little halo overhead.
 inline int pick_z_chunk(int64_t tiles_xy, int nz, int slots, int halo) {
@@ -112,12 +157,11 @@ inline int pick_z_chunk(int64_t tiles_xy, int nz, int slots, int halo) {
     return best;
 }
 
-// Cell planes per workgroup for the gathers (M2P, adjoint), whose z halo costs
-// only ring loads: the longest chunk (8..128) that still gives `per_slot`
-// workgroups per resident slot, so that workgroups of crowded tiles are short
-// and the device balances them dynamically.  At 512^3 the clustered M2P takes
-// 9.9 ms with 16-plane chunks against 18.3 ms with the 128 that pick_z_chunk's
-// model of lockstep rounds prefers; the lattice's is unchanged (2.9 ms).
+// Cell planes per workgroup where the binning saw crowded cells: the longest
+// chunk (8..128) that still gives `per_slot` workgroups per resident slot, so
+// that workgroups of crowded tiles are short and the device balances them
+// dynamically.  At 512^3 the clustered M2P takes 9.9 ms with 16-plane chunks
+// against 18.3 ms with 128.
 inline int pick_z_chunk_balanced(int64_t tiles_xy, int nz, int slots, int per_slot) {
     int best = 8;
     for (int tz = 8; tz <= 128; tz *= 2)

@@ -28,7 +28,6 @@
 //   Ck(L) = sum_{oy,oz} wy_oy(L+1-k) wz_oz(L+1-k) f(L, oy, oz).
 // Output order is the caller's particle order (written through the
 // permutation).
-#include <atomic>
 
 #include "ppmg_internal.h"
 #include "ppmg_interp.h"
@@ -368,9 +367,7 @@ bool m2p3d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg) {
 // field's layout).
 bool m2p3d_table_applicable(const DevMesh& m) { return m.dim == 3 && m.periodic[0] && m.periodic[1] && m.periodic[2]; }
 
-// One launch of the gather for components c0 .. c0+LL-1; the z chunk comes
-// from the resident workgroup count (pick_z_chunk_balanced: each chunk loads
-// 3 extra node planes, cheap beside the balance short chunks give).
+// One launch of the gather for components c0 .. c0+LL-1.
 template <int KS, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool MIX, bool TABLE = false,
           bool LAT = false>
 static void launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
@@ -378,10 +375,14 @@ static void launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, co
     constexpr int TX = M3Geom<KS>::TX;
     constexpr int WPE = KS == 4 && (LL == 4 || MIX) ? 3 : 4;
     auto kernel = k_m3_tile<KS, LL, PosT, ValT, AccT, WPE, OPEN, MIX, TABLE, LAT>;
-    static std::atomic<int> slots{0};
-    if (slots.load() == 0) slots.store(resident_workgroups(kernel, M3_THREADS));
+    static const Residency res = residency(kernel, M3_THREADS);
     const int tx = (m.nbin[0] + TX - 1) / TX, ty = (m.nbin[1] + M3_TY - 1) / M3_TY;
-    const int tz = pick_z_chunk_balanced((int64_t)tx * ty, m.nbin[2], slots.load(), 32);
+    // a chunk loads KS - 1 more planes before its first step: a plane's worth
+    // of time on a full device, their latency on a small mesh
+    const int64_t ncells = (int64_t)m.nbin[0] * m.nbin[1] * m.nbin[2];
+    const int tz = plan->crowded_cells > ncells / 1024
+                       ? pick_z_chunk_balanced((int64_t)tx * ty, m.nbin[2], res.slots(), 32)
+                       : pick_chunk((int64_t)tx * ty, m.nbin[2], res, 1.0, KS - 1);
     dim3 grid((unsigned)((int64_t)tx * ty * ((m.nbin[2] + tz - 1) / tz)));
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
     hipLaunchKernelGGL(kernel, grid, dim3(M3_THREADS), 0, s, m, plan->start.as<int>(),

@@ -21,7 +21,6 @@
 // so the order of every node's additions is a fixed function of the binning,
 // and results are bitwise reproducible with no global float atomics.  The
 // periodic fold happens through the index wrap of the cells around the tile.
-#include <atomic>
 #include <cstdlib>
 
 #include "ppmg_internal.h"
@@ -455,9 +454,7 @@ template <int KS, int LL, typename PosT, typename ValT, int TY, int NW, bool OPE
 static void launch_p3_shape(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
                             const FieldGeom& fg, int c0, ValT* field, const WTab<ValT>& wt, hipStream_t s) {
     constexpr int H = Stencil<KS>::H, TT = 16 - H;
-    static std::atomic<int> slots{0};
-    if (slots.load() == 0)
-        slots.store(resident_workgroups(k_p3_tile<KS, LL, PosT, ValT, TY, NW, OPEN, TAB, TABLE>, 64 * NW));
+    static const Residency res = residency(k_p3_tile<KS, LL, PosT, ValT, TY, NW, OPEN, TAB, TABLE>, 64 * NW);
     const int Rx = m.N[0] + !m.periodic[0], Ry = m.N[1] + !m.periodic[1], Rz = m.N[2] + !m.periodic[2];
     const int tx = (Rx + TT - 1) / TT, ty = (Ry + TY - 1) / TY;
     // crowded cells (more than 1/1024 of the cells hold nine or more
@@ -465,8 +462,8 @@ static void launch_p3_shape(ppmg_plan* plan, const DevMesh& m, const PosT* xp, c
     // (clustered 512^3: 13.8 against 15.6 ms); the lattice keeps the chunk
     // that costs the least halo (4.56 against 4.82 ms with 16 planes)
     const int64_t ncells = (int64_t)m.nbin[0] * m.nbin[1] * m.nbin[2];
-    const int tz = plan->crowded_cells > ncells / 1024 ? pick_z_chunk_balanced((int64_t)tx * ty, Rz, slots.load(), 16)
-                                                       : pick_z_chunk((int64_t)tx * ty, Rz, slots.load(), H);
+    const int tz = plan->crowded_cells > ncells / 1024 ? pick_z_chunk_balanced((int64_t)tx * ty, Rz, res.slots(), 16)
+                                                       : pick_chunk((int64_t)tx * ty, Rz, res, H, H);
     dim3 grid((unsigned)((int64_t)tx * ty * ((Rz + tz - 1) / tz)));
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
     hipLaunchKernelGGL((k_p3_tile<KS, LL, PosT, ValT, TY, NW, OPEN, TAB, TABLE>), grid, dim3(64 * NW), 0, s, m,
