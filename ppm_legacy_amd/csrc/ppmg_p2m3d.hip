@@ -33,6 +33,7 @@ namespace ppmg {
 constexpr int P3_TT = 13;   // owned nodes per tile along x (16-lane DPP row = 13 + 3 halo cells)
 constexpr int P3_TY = 21;   // owned node rows per tile along y (24 cell rows: 6 chunks, 3 wavefronts)
 constexpr int P3_SERIAL = 4; // later rounds with at most this many active lanes go one particle at a time
+constexpr int P3_STAGE = 15; // second particles of a chunk staged in LDS (more take a full round)
 
 // LDS accumulator of one node component.  Every form accumulates in an FP64
 // slot with ds_add_f64 (fire-and-forget, no read-modify-write latency chain):
@@ -124,6 +125,11 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     constexpr int NC = NW == 1 ? NQ : 2;           // chunks per wavefront and plane
     constexpr int PLANE = P3_PL * LDA;            // slots per ring plane: [c][node]
     __shared__ slot_t ring[RP * PLANE];
+    // Second particles of a wavefront's chunk: [1D weights x, y, z and
+    // strengths][particle].  15 apart, the four values a stencil offset picks
+    // from lie in different banks.
+    constexpr int NV = 3 * KS + LDA;
+    __shared__ ValT stage_all[NW * NV * P3_STAGE];
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     // nodes the tiles produce per axis: the N unique nodes of a periodic axis,
@@ -261,6 +267,24 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     PD xn[NPD];
     ValT un[LDA];
     load(pn, count_of(f1, n1) > 0, xn, un);
+    // The cell's second particle likewise: entry one step ahead, data at the
+    // end of the step before; at the start of its step its weights go to LDS.
+    PD xl[NPD];
+    ValT ul[LDA];
+    int pl2 = count_of(f1, n1) > 1 ? entry(f1, 1) : 0;
+    load(pl2, count_of(f1, n1) > 1, xl, ul);
+    ValT* const stage = stage_all + wave * (NV * P3_STAGE);
+    // stencil offset of this lane when the wavefront takes one particle (the
+    // 64 lanes its 64 nodes; with KS = 2 lanes 0..7 the 8 nodes), recomputed
+    // where it is used rather than held through the rounds
+    auto stencil_lane = [&](int& ox, int& oy, int& oz) {
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        ox = l & (KS - 1);
+        oy = (l / KS) & (KS - 1);
+        oz = l / (KS * KS);
+        return l < KS * KS * KS;
+    };
 
     for (int cz = cz0; cz <= cz1; ++cz) {
 #pragma unroll
@@ -273,6 +297,7 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
             n1 = n2;
             t1 = t2;
             pn = lookup(f1, n1, t1);
+            pl2 = count_of(f1, n1) > 1 ? entry(f1, 1) : 0;
             if (j + 2 < NC) heads(cz, j + 2, f2, n2, t2);
             else if (j + 2 - NC < NC) heads(cz + 1, j + 2 - NC, f2, n2, t2);
             else heads(cz + 2, 0, f2, n2, t2);
@@ -321,15 +346,66 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                     }
                 }
             };
+            // Second particles, where at most P3_STAGE cells of the chunk have one
+            // (41% of an advected lattice's chunks do, with 5 such cells on
+            // average): their weights go to LDS ahead of round 0, so that nothing
+            // is waited for when they are deposited after it.  512^3, FP64, lda
+            // 3, advected by up to half a cell: deposit 5.33 -> 5.08 ms against
+            // loading them after round 0 (a full round for more than four cells,
+            // each of the others on its own); 3.84 ms with them left out.  What
+            // they cost now is their LDS traffic: three 64-lane atomics and six
+            // reads each.
+            const uint64_t act1 = __ballot(cnt > 1);
+            const int nl = (int)__popcll(act1);
+            const bool staged = nl > 0 && nl <= P3_STAGE;
+            if (staged) {
+                ValT wx[KS], wy[KS], wz[KS];
+                weights(xl, wx, wy, wz);
+                if (cnt > 1) {
+                    ValT* q = stage + __builtin_amdgcn_mbcnt_hi((unsigned)(act1 >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((unsigned)act1, 0u));
+#pragma unroll
+                    for (int o = 0; o < KS; ++o) {
+                        q[o * P3_STAGE] = wx[o];
+                        q[(KS + o) * P3_STAGE] = wy[o];
+                        q[(2 * KS + o) * P3_STAGE] = wz[o];
+                    }
+#pragma unroll
+                    for (int c = 0; c < LDA; ++c) q[(3 * KS + c) * P3_STAGE] = ul[c];
+                }
+                wave_lds_sync();
+            }
+            const int qrow = ey4[j] - erow;          // first cell row of the chunk
             // round 0 with the particle loaded during the previous step
             if (__ballot(cnt > 0) != 0ull) round(xn, un);
+            // the staged second particles, one at a time
+            if (staged) {
+                int sox, soy, soz;
+                const bool slane = stencil_lane(sox, soy, soz);
+                slot_t* pl = ring + ((cz - B + soz) & (RP - 1)) * PLANE;
+                uint64_t a = act1;
+                for (int k = 0; k < nl; ++k) {
+                    const int src = __builtin_ctzll(a);
+                    a &= a - 1;
+                    const int nx = (src & 15) - H + sox, ny = qrow + (src >> 4) - H + soy;
+                    const bool own = slane && (unsigned)nx < (unsigned)nxo && (unsigned)ny < (unsigned)nyo;
+                    const ValT* q = stage + k;
+                    const ValT wyz = q[(KS + soy) * P3_STAGE] * q[(2 * KS + soz) * P3_STAGE];
+                    const ValT wxo = q[sox * P3_STAGE];
+                    if (own) {
+#pragma unroll
+                        for (int c = 0; c < LDA; ++c)
+                            A::add(pl + c * P3_PL + nx + TT * ny, wyz * (wxo * q[(3 * KS + c) * P3_STAGE]));
+                    }
+                }
+            }
             // Later rounds load their own particles.  A round costs the same
             // however few lanes still have a particle, so once at most P3_SERIAL
             // lanes do, their remaining particles are deposited one at a time:
             // the 64 lanes take the 64 nodes of the particle's stencil (distinct
             // nodes, so the additions stay in a fixed order; with KS = 2 lanes
             // 0..7 take the 8 nodes).
-            for (int r = 1;; ++r) {
+            for (int r = staged ? 2 : 1;; ++r) {
                 uint64_t act = __ballot(cnt > r);
                 if (act == 0ull) break;
                 if (__popcll(act) > P3_SERIAL) {
@@ -340,10 +416,9 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                     round(x, u);
                     continue;
                 }
-                const int ox = lane & (KS - 1), oy = (lane / KS) & (KS - 1), oz = lane / (KS * KS);
-                const bool slane = lane < KS * KS * KS;
+                int ox, oy, oz;
+                const bool slane = stencil_lane(ox, oy, oz);
                 slot_t* pl = ring + ((cz - B + oz) & (RP - 1)) * PLANE;
-                const int qrow = ey4[j] - erow;      // first cell row of the chunk
                 do {
                     const int src = __builtin_ctzll(act);
                     act &= act - 1;
@@ -374,6 +449,7 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                 break;
             }
             load(pn, count_of(f1, n1) > 0, xn, un);
+            load(pl2, count_of(f1, n1) > 1, xl, ul);
             // end of a phase: the other phase's chunks share node rows with this one's
             if (NW > 1 || j == NC - 1) __syncthreads();
         }

@@ -1,0 +1,80 @@
+"""The tiled kernels at the occupancies and sizes where they change path."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+MP4, BSP2 = 2, 1
+F64, F32C, F32 = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def core():
+    from ppm_legacy_amd import core as c
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    return c
+
+
+def _general(monkeypatch, call):
+    monkeypatch.setenv("PPMG_GENERAL", "1")
+    r = call()
+    monkeypatch.delenv("PPMG_GENERAL")
+    return r
+
+
+@pytest.mark.parametrize("extra", [0, 1, 4, 14, 15, 16, 17, 64])
+@pytest.mark.parametrize("kernel", [MP4, BSP2])
+@pytest.mark.parametrize("lda", [1, 3, 4])
+def test_deposit_second_particles(core, monkeypatch, extra, kernel, lda):
+    """One particle per cell and a second (every fifth of those a third) in
+    `extra` cells of one 16 x 4 block: around the number of second particles
+    the deposit stages.  FP64 sums of at most 100 terms against the general
+    path: 1e-13 of the maximum; both binning forms bitwise the same."""
+    N = 24
+    rng = np.random.default_rng(extra + 100 * lda)
+    i = np.arange(N ** 3)
+    cells = np.stack([i % N, (i // N) % N, i // N ** 2], 1)
+    block = np.stack([np.arange(extra) % 16 + 3, np.arange(extra) // 16 + 6, np.full(extra, 11)], 1)
+    cells = np.concatenate([cells, block, block[::5]]).astype(float)
+    x = (cells + rng.uniform(0.02, 0.98, cells.shape)) / N
+    order = rng.permutation(len(x))
+    mesh = core.Mesh(3, N + 1)
+    xd = torch.as_tensor(x[order]).cuda()
+    u = torch.as_tensor(rng.normal(size=(len(x), lda))).cuda()
+
+    def p2m():
+        f = torch.empty(mesh.compact_shape(lda), dtype=torch.float64, device="cuda")
+        core.p2m(mesh, xd, u, f, [0] * 3, kernel)
+        return f
+
+    f, ref = p2m(), _general(monkeypatch, p2m)
+    assert ((f - ref).abs().max() / ref.abs().max()).item() < 1e-13
+    monkeypatch.setenv("PPMG_NO_TABLE", "1")
+    assert torch.equal(f, p2m())
+
+
+@pytest.mark.parametrize("N", [4, 7, 16, 31, 33])
+@pytest.mark.parametrize("prec", [F64, F32C, F32])
+def test_small_meshes_short_chunks(core, monkeypatch, N, prec):
+    """Meshes of one to a few planes per workgroup: deposit, gather and adjoint
+    against the general path (1e-13 in FP64; FP32 forms 2e-5 of the maximum)."""
+    rng = np.random.default_rng(N)
+    n = N ** 3 + 5
+    mesh = core.Mesh(3, N + 1)
+    pdt, vdt = core.POS_DTYPE[prec], core.VAL_DTYPE[prec]
+    x = torch.as_tensor(rng.uniform(0, 0.9999, (n, 3))).to(pdt).cuda()
+    u = torch.as_tensor(rng.normal(size=(n, 3))).to(vdt).cuda()
+    g = torch.as_tensor(rng.normal(size=mesh.compact_shape(3))).to(vdt).cuda()
+
+    def run():
+        f = torch.empty(mesh.compact_shape(3), dtype=vdt, device="cuda")
+        plan = core.p2m(mesh, x, u, f, [0] * 3, MP4, prec)
+        gu, gx = core.p2m_adjoint(mesh, x, u, g, [0] * 3, plan, MP4, prec)
+        out = torch.empty_like(u)
+        core.m2p(mesh, x, g, [0] * 3, out, MP4, prec)
+        return f, gu, gx, out
+
+    tol = 1e-13 if prec == F64 else 2e-5
+    for a, b in zip(run(), _general(monkeypatch, run)):
+        assert ((a - b).abs().max() / b.abs().max()).item() < tol
