@@ -87,16 +87,17 @@ template <int LDA, typename PosT, typename ValT, typename AccT, bool BOXED, bool
 __global__ void __launch_bounds__(A3_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
 k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ up, const ValT* __restrict__ g, FieldGeom fg,
-          ValT* __restrict__ grad_u, ValT* __restrict__ grad_x, int lda, int c0, int tz, int accumulate_x) {
+          ValT* __restrict__ grad_u, ValT* __restrict__ grad_x, int lda, int c0, int tz, const int4* __restrict__ items,
+          int accumulate_x) {
     __shared__ ValT ring[4 * LDA * A3_PL];   // [plane][c][ry][nx]
     const int tid = threadIdx.x;
     const int ex = tid & 15, row = tid >> 4;
     const int Nx = m.N[0], Ny = m.N[1], Nz = m.N[2];
     const int ntx = (Nx + A3_TX - 1) / A3_TX, nty = (Ny + A3_TY - 1) / A3_TY;
-    const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
-    const int tx0 = (int)(tile % ntx) * A3_TX, ty0 = (int)((tile / ntx) % nty) * A3_TY;
-    const int z0 = (int)(tile / ((int64_t)ntx * nty)) * tz;
-    const int z1 = min(z0 + tz, Nz);
+    int tx0, ty0, z0, z1;
+    tile_piece(items, ntx, nty, tz, Nz, tx0, ty0, z0, z1);
+    tx0 *= A3_TX;
+    ty0 *= A3_TY;
     const int nxo = min(A3_TX, Nx - tx0), nyo = min(A3_TY, Ny - ty0);
     const int64_t plane = (int64_t)Nx * Ny;
 
@@ -380,19 +381,22 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 }
 
 template <int LL, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE = false>
-static void launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
+static int launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
                            const FieldGeom& fg, ValT* gu, ValT* gx, int lda, int c0, int acc, hipStream_t s) {
     static const Residency res = residency(k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>, A3_THREADS);
     const int tx = (m.N[0] + A3_TX - 1) / A3_TX, ty = (m.N[1] + A3_TY - 1) / A3_TY;
     // a step is long here: a chunk's three extra plane loads weigh little
-    const int64_t ncells = (int64_t)m.N[0] * m.N[1] * m.N[2];
-    const int tz = plan->crowded_cells > ncells / 1024
-                       ? pick_z_chunk_balanced((int64_t)tx * ty, m.N[2], res.slots(), 32)
-                       : pick_chunk((int64_t)tx * ty, m.N[2], res, 0.3, 0.3);
-    dim3 grid((unsigned)((int64_t)tx * ty * ((m.N[2] + tz - 1) / tz)));
+    const int tz = pick_chunk((int64_t)tx * ty, m.N[2], res, 0.3, 0.3);
+    unsigned grid = (unsigned)((int64_t)tx * ty * ((m.N[2] + tz - 1) / tz));
+    const int4* items = nullptr;   // crowded cells: workgroups from a work list
+    if (!TABLE && work_list_applies(plan)) {
+        const int rc = build_work(plan, m, {tx, ty, A3_TX, A3_TY, 0, 0, A3_TX, A3_TY, m.N[2]}, s, &items, &grid);
+        if (rc < 0) return rc;
+    }
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
-    hipLaunchKernelGGL((k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>), grid, dim3(A3_THREADS), 0, s, m,
-                       plan->start.as<int>(), tile_perm(plan), bt, xp, up, g, fg, gu, gx, lda, c0, tz, acc);
+    hipLaunchKernelGGL((k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>), dim3(grid), dim3(A3_THREADS), 0, s, m,
+                       plan->start.as<int>(), tile_perm(plan), bt, xp, up, g, fg, gu, gx, lda, c0, tz, items, acc);
+    return 0;
 }
 
 // The compact layout of every axis, or a stored box on some axis.
@@ -403,15 +407,15 @@ static bool a3_compact(const DevMesh& m, const FieldGeom& fg) {
 }
 
 template <int LL, typename PosT, typename ValT, typename AccT>
-static void launch_a3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
+static int launch_a3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
                       const FieldGeom& fg, ValT* gu, ValT* gx, int lda, int c0, int acc, hipStream_t s) {
     const bool compact = a3_compact(m, fg);
     if (plan->bin_table) {
-        if (compact) launch_a3_form<LL, PosT, ValT, AccT, false, true>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
-        else launch_a3_form<LL, PosT, ValT, AccT, true, true>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
+        if (compact) return launch_a3_form<LL, PosT, ValT, AccT, false, true>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
+        else return launch_a3_form<LL, PosT, ValT, AccT, true, true>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
     } else {
-        if (compact) launch_a3_form<LL, PosT, ValT, AccT, false>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
-        else launch_a3_form<LL, PosT, ValT, AccT, true>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
+        if (compact) return launch_a3_form<LL, PosT, ValT, AccT, false>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
+        else return launch_a3_form<LL, PosT, ValT, AccT, true>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
     }
 }
 
@@ -427,9 +431,8 @@ static int adjoint3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const 
         const int L = lda - c0 < 3 ? lda - c0 : 3;
         const int acc = c0 > 0 ? 1 : 0;
 #define AL(LL) launch_a3<LL, PosT, ValT, double>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s)
-        if (L == 1) AL(1);
-        else if (L == 2) AL(2);
-        else AL(3);
+        const int rc = L == 1 ? AL(1) : L == 2 ? AL(2) : AL(3);
+        if (rc) return rc;
 #undef AL
         PPMG_HIP(hipGetLastError());
     }

@@ -157,18 +157,6 @@ inline int pick_z_chunk(int64_t tiles_xy, int nz, int slots, int halo) {
     return best;
 }
 
-// Cell planes per workgroup where the binning saw crowded cells: the longest
-// chunk (8..128) that still gives `per_slot` workgroups per resident slot, so
-// that workgroups of crowded tiles are short and the device balances them
-// dynamically.  At 512^3 the clustered M2P takes 9.9 ms with 16-plane chunks
-// against 18.3 ms with 128.
-inline int pick_z_chunk_balanced(int64_t tiles_xy, int nz, int slots, int per_slot) {
-    int best = 8;
-    for (int tz = 8; tz <= 128; tz *= 2)
-        if (tiles_xy * (int64_t)((nz + tz - 1) / tz) >= (int64_t)per_slot * slots) best = tz;
-    return best;
-}
-
 // ----------------------------------------------------- XCD tile order --
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on
 // XCD b % 8), each with its own L2.  Tile kernels use a 1D grid and map
@@ -442,7 +430,7 @@ inline bool same_mesh(const DevMesh& a, const DevMesh& b) {
 // Opaque plan: scratch of the binning and the forward record for the adjoint.
 struct ppmg_plan {
     ppmg::DevBuf key, slot, count, start, perm, wsorted, usorted, scan_tmp, err, misc, misc2, gaps, multi,
-        multi_n, ghost, table, rhist;
+        multi_n, ghost, table, rhist, work, work_cnt;
     ppmg::DevBuf rkey[2], rval[2];   // ping-pong pairs of the radix-sort binning of crowded input
     int64_t np = 0;
     int64_t ncells = 0;

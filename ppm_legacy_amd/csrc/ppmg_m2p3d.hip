@@ -74,7 +74,7 @@ template <int KS, int LDA, typename PosT, typename ValT, typename AccT, int WPE,
 __global__ void __launch_bounds__(M3_THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ field, FieldGeom fg, ValT* __restrict__ up, int lda,
-          int c0, int tz, int* __restrict__ lat_err) {
+          int c0, int tz, const int4* __restrict__ items, int* __restrict__ lat_err) {
     static_assert(!(TABLE && LAT), "one binning form");
     constexpr int B = M3Geom<KS>::B, M3_TX = M3Geom<KS>::TX, M3_PL = M3Geom<KS>::PL;
     constexpr int RP = KS;                   // ring planes
@@ -84,10 +84,10 @@ k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     // tiles cover the cells: N per periodic axis, N+1 (0..N) per open one
     const int Nx = m.nbin[0], Ny = m.nbin[1], Nz = m.nbin[2];
     const int ntx = (Nx + M3_TX - 1) / M3_TX, nty = (Ny + M3_TY - 1) / M3_TY;
-    const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
-    const int tx0 = (int)(tile % ntx) * M3_TX, ty0 = (int)((tile / ntx) % nty) * M3_TY;
-    const int z0 = (int)(tile / ((int64_t)ntx * nty)) * tz;
-    const int z1 = min(z0 + tz, Nz);
+    int tx0, ty0, z0, z1;
+    tile_piece(items, ntx, nty, tz, Nz, tx0, ty0, z0, z1);
+    tx0 *= M3_TX;
+    ty0 *= M3_TY;
     const int nxo = min(M3_TX, Nx - tx0), nyo = min(M3_TY, Ny - ty0);
     const int64_t plane = (int64_t)Nx * Ny;
 
@@ -370,7 +370,7 @@ bool m2p3d_table_applicable(const DevMesh& m) { return m.dim == 3 && m.periodic[
 // One launch of the gather for components c0 .. c0+LL-1.
 template <int KS, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool MIX, bool TABLE = false,
           bool LAT = false>
-static void launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
+static int launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
                            const ValT* field, ValT* up, hipStream_t s) {
     constexpr int TX = M3Geom<KS>::TX;
     constexpr int WPE = KS == 4 && (LL == 4 || MIX) ? 3 : 4;
@@ -379,32 +379,37 @@ static void launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, co
     const int tx = (m.nbin[0] + TX - 1) / TX, ty = (m.nbin[1] + M3_TY - 1) / M3_TY;
     // a chunk loads KS - 1 more planes before its first step: a plane's worth
     // of time on a full device, their latency on a small mesh
-    const int64_t ncells = (int64_t)m.nbin[0] * m.nbin[1] * m.nbin[2];
-    const int tz = plan->crowded_cells > ncells / 1024
-                       ? pick_z_chunk_balanced((int64_t)tx * ty, m.nbin[2], res.slots(), 32)
-                       : pick_chunk((int64_t)tx * ty, m.nbin[2], res, 1.0, KS - 1);
-    dim3 grid((unsigned)((int64_t)tx * ty * ((m.nbin[2] + tz - 1) / tz)));
+    const int tz = pick_chunk((int64_t)tx * ty, m.nbin[2], res, 1.0, KS - 1);
+    unsigned grid = (unsigned)((int64_t)tx * ty * ((m.nbin[2] + tz - 1) / tz));
+    // crowded cells: the workgroups come from a work list (clustered 512^3,
+    // FP64, lda 3: 7.7 against 9.5 ms in 16-plane chunks)
+    const int4* items = nullptr;
+    if (!TABLE && !LAT && work_list_applies(plan)) {
+        const int rc = build_work(plan, m, {tx, ty, TX, M3_TY, 0, 0, TX, M3_TY, m.nbin[2]}, s, &items, &grid);
+        if (rc < 0) return rc;
+    }
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
-    hipLaunchKernelGGL(kernel, grid, dim3(M3_THREADS), 0, s, m, plan->start.as<int>(),
-                       tile_perm(plan), bt, xp, field, fg, up, fg.lda, c0, tz, plan->err.as<int>() + 6);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(M3_THREADS), 0, s, m, plan->start.as<int>(),
+                       tile_perm(plan), bt, xp, field, fg, up, fg.lda, c0, tz, items, plan->err.as<int>() + 6);
+    return 0;
 }
 
 // OPEN: some axis is open (a fully periodic mesh compiles without the clamp);
 // MIX: and some periodic axis is stored as a box.
 template <int KS, int LL, typename PosT, typename ValT, typename AccT>
-static void launch_m3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
+static int launch_m3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
                       const ValT* field, ValT* up, hipStream_t s) {
     // a slot table or an unchecked lattice is binned on periodic meshes only (m2p3d_fast)
     if (plan->bin_lattice)
-        launch_m3_open<KS, LL, PosT, ValT, AccT, false, false, false, true>(plan, m, xp, fg, c0, field, up, s);
+        return launch_m3_open<KS, LL, PosT, ValT, AccT, false, false, false, true>(plan, m, xp, fg, c0, field, up, s);
     else if (plan->bin_table)
-        launch_m3_open<KS, LL, PosT, ValT, AccT, false, false, true>(plan, m, xp, fg, c0, field, up, s);
+        return launch_m3_open<KS, LL, PosT, ValT, AccT, false, false, true>(plan, m, xp, fg, c0, field, up, s);
     else if (m.periodic[0] && m.periodic[1] && m.periodic[2])
-        launch_m3_open<KS, LL, PosT, ValT, AccT, false, false>(plan, m, xp, fg, c0, field, up, s);
+        return launch_m3_open<KS, LL, PosT, ValT, AccT, false, false>(plan, m, xp, fg, c0, field, up, s);
     else if (fg.swap[0] || fg.swap[1] || fg.swap[2])
-        launch_m3_open<KS, LL, PosT, ValT, AccT, true, true>(plan, m, xp, fg, c0, field, up, s);
+        return launch_m3_open<KS, LL, PosT, ValT, AccT, true, true>(plan, m, xp, fg, c0, field, up, s);
     else
-        launch_m3_open<KS, LL, PosT, ValT, AccT, true, false>(plan, m, xp, fg, c0, field, up, s);
+        return launch_m3_open<KS, LL, PosT, ValT, AccT, true, false>(plan, m, xp, fg, c0, field, up, s);
 }
 
 template <int KS, typename PosT, typename ValT, typename AccT>
@@ -415,10 +420,8 @@ static int m2p3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const PosT
     for (int c0 = 0; c0 < lda; c0 += 4) {
         int L = lda - c0 < 4 ? lda - c0 : 4;
 #define TL(LL) launch_m3<KS, LL, PosT, ValT, AccT>(plan, m, xp, fg, c0, field, up, s)
-        if (L == 1) TL(1);
-        else if (L == 2) TL(2);
-        else if (L == 3) TL(3);
-        else TL(4);
+        const int rc = L == 1 ? TL(1) : L == 2 ? TL(2) : L == 3 ? TL(3) : TL(4);
+        if (rc) return rc;
 #undef TL
         PPMG_HIP(hipGetLastError());
     }

@@ -106,7 +106,7 @@ template <int KS, int LDA, typename PosT, typename ValT, int TY, int NW, bool OP
 __global__ void __launch_bounds__(64 * NW)
 k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ up, FieldGeom fg, int c0, int tz,
-          ValT* __restrict__ field, WTab<ValT> wt) {
+          const int4* __restrict__ items, ValT* __restrict__ field, WTab<ValT> wt) {
     constexpr int H = Stencil<KS>::H, B = Stencil<KS>::B;
     constexpr int TT = 16 - H;                     // owned nodes per tile along x
     constexpr int RP = KS;                         // ring planes
@@ -136,10 +136,10 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     // the N+1 real nodes 0..N of an open one
     const int Rx = m.N[0] + !m.periodic[0], Ry = m.N[1] + !m.periodic[1], Rz = m.N[2] + !m.periodic[2];
     const int ntx = (Rx + TT - 1) / TT, nty = (Ry + TY - 1) / TY;
-    const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
-    const int tx0 = (int)(tile % ntx) * TT, ty0 = (int)((tile / ntx) % nty) * TY;
-    const int z0 = (int)(tile / ((int64_t)ntx * nty)) * tz;
-    const int z1 = min(z0 + tz, Rz);
+    int tx0, ty0, z0, z1;
+    tile_piece(items, ntx, nty, tz, Rz, tx0, ty0, z0, z1);
+    tx0 *= TT;
+    ty0 *= TY;
     const int nxo = min(TT, Rx - tx0), nyo = min(TY, Ry - ty0);
     for (int i = tid; i < RP * PLANE; i += NT) A::zero(ring[i]);
 
@@ -282,7 +282,7 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
         asm volatile("" : "+v"(l));
         ox = l & (KS - 1);
         oy = (l / KS) & (KS - 1);
-        oz = l / (KS * KS);
+        oz = (l / (KS * KS)) & (KS - 1);
         return l < KS * KS * KS;
     };
 
@@ -527,23 +527,25 @@ bool p2m3d_table_applicable(const DevMesh& m, int kernel, int prec, const FieldG
 // the device's resident workgroup count (queried once per instantiation):
 // each chunk marches H extra cell planes.
 template <int KS, int LL, typename PosT, typename ValT, int TY, int NW, bool OPEN, bool TAB, bool TABLE = false>
-static void launch_p3_shape(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
+static int launch_p3_shape(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
                             const FieldGeom& fg, int c0, ValT* field, const WTab<ValT>& wt, hipStream_t s) {
     constexpr int H = Stencil<KS>::H, TT = 16 - H;
     static const Residency res = residency(k_p3_tile<KS, LL, PosT, ValT, TY, NW, OPEN, TAB, TABLE>, 64 * NW);
     const int Rx = m.N[0] + !m.periodic[0], Ry = m.N[1] + !m.periodic[1], Rz = m.N[2] + !m.periodic[2];
     const int tx = (Rx + TT - 1) / TT, ty = (Ry + TY - 1) / TY;
-    // crowded cells (more than 1/1024 of the cells hold nine or more
-    // particles): shorter chunks keep the workgroups of crowded tiles short
-    // (clustered 512^3: 13.8 against 15.6 ms); the lattice keeps the chunk
-    // that costs the least halo (4.56 against 4.82 ms with 16 planes)
-    const int64_t ncells = (int64_t)m.nbin[0] * m.nbin[1] * m.nbin[2];
-    const int tz = plan->crowded_cells > ncells / 1024 ? pick_z_chunk_balanced((int64_t)tx * ty, Rz, res.slots(), 16)
-                                                       : pick_chunk((int64_t)tx * ty, Rz, res, H, H);
-    dim3 grid((unsigned)((int64_t)tx * ty * ((Rz + tz - 1) / tz)));
+    const int tz = pick_chunk((int64_t)tx * ty, Rz, res, H, H);
+    unsigned grid = (unsigned)((int64_t)tx * ty * ((Rz + tz - 1) / tz));
+    // crowded cells: the workgroups come from a work list (clustered 512^3,
+    // FP64, lda 3: 10.4 against 13.4 ms in 16-plane chunks)
+    const int4* items = nullptr;
+    if (!TABLE && work_list_applies(plan)) {
+        const int rc = build_work(plan, m, {tx, ty, TT, TY, -(H - Stencil<KS>::B), -(H - Stencil<KS>::B), 16, TY + H, Rz}, s, &items, &grid);
+        if (rc < 0) return rc;
+    }
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
-    hipLaunchKernelGGL((k_p3_tile<KS, LL, PosT, ValT, TY, NW, OPEN, TAB, TABLE>), grid, dim3(64 * NW), 0, s, m,
-                       plan->start.as<int>(), perm, bt, xp, up, fg, c0, tz, field, wt);
+    hipLaunchKernelGGL((k_p3_tile<KS, LL, PosT, ValT, TY, NW, OPEN, TAB, TABLE>), dim3(grid), dim3(64 * NW), 0, s, m,
+                       plan->start.as<int>(), perm, bt, xp, up, fg, c0, tz, items, field, wt);
+    return 0;
 }
 
 // Tile height: PPMG_P2M_ROWS (9, 13, 21 or 29 node rows: 1, 2, 3 or 4
@@ -558,40 +560,39 @@ static int p3_rows() {
 }
 
 template <int KS, int LL, typename PosT, typename ValT, bool OPEN, bool TAB>
-static void launch_p3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
+static int launch_p3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
                            const FieldGeom& fg, int c0, ValT* field, const WTab<ValT>& wt, hipStream_t s) {
     if constexpr (KS == 2) {
         // BSP2: 15 x 23 node tiles (24 cell rows, three wavefronts)
-        launch_p3_shape<KS, LL, PosT, ValT, 23, 3, OPEN, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
+        return launch_p3_shape<KS, LL, PosT, ValT, 23, 3, OPEN, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
     } else if constexpr (TAB) {
         // the remesh path takes the default tile only
-        launch_p3_shape<KS, LL, PosT, ValT, 21, 3, OPEN, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
+        return launch_p3_shape<KS, LL, PosT, ValT, 21, 3, OPEN, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
     } else {
 #define SHAPE(TY, NW) \
     launch_p3_shape<KS, LL, PosT, ValT, TY, NW, OPEN, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s)
         switch (p3_rows()) {
-            case 9: SHAPE(9, 1); break;
-            case 13: SHAPE(13, 2); break;
-            case 29: SHAPE(29, 4); break;
-            default: SHAPE(21, 3); break;
+            case 9: return SHAPE(9, 1);
+            case 13: return SHAPE(13, 2);
+            case 29: return SHAPE(29, 4);
+            default: return SHAPE(21, 3);
         }
 #undef SHAPE
     }
 }
 
 template <int KS, int LL, typename PosT, typename ValT, bool TAB>
-static void launch_p3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
+static int launch_p3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const int* perm,
                       const FieldGeom& fg, int c0, ValT* field, const WTab<ValT>& wt, hipStream_t s) {
     // a slot table (p2m3d_table_applicable: periodic, default tile)
     if (plan->bin_table) {
-        launch_p3_shape<KS, LL, PosT, ValT, KS == 2 ? 23 : P3_TY, 3, false, TAB, true>(plan, m, xp, up, perm, fg, c0,
-                                                                                       field, wt, s);
-        return;
+        return launch_p3_shape<KS, LL, PosT, ValT, KS == 2 ? 23 : P3_TY, 3, false, TAB, true>(plan, m, xp, up, perm, fg,
+                                                                                              c0, field, wt, s);
     }
     if (m.periodic[0] && m.periodic[1] && m.periodic[2])
-        launch_p3_open<KS, LL, PosT, ValT, false, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
+        return launch_p3_open<KS, LL, PosT, ValT, false, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
     else
-        launch_p3_open<KS, LL, PosT, ValT, true, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
+        return launch_p3_open<KS, LL, PosT, ValT, true, TAB>(plan, m, xp, up, perm, fg, c0, field, wt, s);
 }
 
 template <int KS, typename PosT, typename ValT>
@@ -610,15 +611,10 @@ static int p2m3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const PosT
     const int* pk = tile_perm(plan);
     for (int c0 = 0; c0 < lda; c0 += 4) {
         int L = lda - c0 < 4 ? lda - c0 : 4;
-#define TL(LL)                                                                            \
-    do {                                                                                  \
-        if (wtab) launch_p3<KS, LL, PosT, ValT, true>(plan, m, xp, up, pk, fg, c0, field, wt, s);      \
-        else launch_p3<KS, LL, PosT, ValT, false>(plan, m, xp, up, pk, fg, c0, field, wt, s);          \
-    } while (0)
-        if (L == 1) TL(1);
-        else if (L == 2) TL(2);
-        else if (L == 3) TL(3);
-        else TL(4);
+#define TL(LL)                                                                                       \
+    (wtab ? launch_p3<KS, LL, PosT, ValT, true>(plan, m, xp, up, pk, fg, c0, field, wt, s)           \
+          : launch_p3<KS, LL, PosT, ValT, false>(plan, m, xp, up, pk, fg, c0, field, wt, s))
+        if (L == 1 ? TL(1) : L == 2 ? TL(2) : L == 3 ? TL(3) : TL(4)) return 1;
 #undef TL
         PPMG_HIP(hipGetLastError());
     }

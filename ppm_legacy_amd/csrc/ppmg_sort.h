@@ -88,4 +88,42 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
 int sort_rows(int dim, int prec, int64_t np, void* xp, const int* lpdx1, const int* lhbx1, int64_t nbox, int* npbx,
               DevBuf& tmp, hipStream_t s);
 
+// ------------------------------------------- work list (ppmg_work.hip) --
+// Tile columns of a 3D tile kernel: ntx x nty tiles of tx x ty, marching
+// `planes` planes; a tile's cells are the ncol x nrow ones starting at offset
+// (wx, wy) from its first.
+struct TileWindow {
+    int ntx, nty, tx, ty;
+    int wx, wy, ncol, nrow;
+    int planes;
+};
+// The plan's last binning found crowded cells and left heads: launches take
+// their workgroups from a work list.
+bool work_list_applies(const ppmg_plan* plan);
+// Pieces (tile column, first plane, end plane) of all tile columns, heaviest
+// first, in the plan's scratch; 0, 1 (no list) or an error.
+int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, hipStream_t s, const int4** items,
+               unsigned* nitems);
+// This workgroup's tile column and planes [z0, z1): from the work list, or
+// (items NULL) the grid's chunks of tz planes in XCD order.
+__device__ __forceinline__ void tile_piece(const int4* __restrict__ items, int ntx, int nty, int tz, int planes,
+                                           int& tx, int& ty, int& z0, int& z1) {
+    int col;
+    if (items) {
+        const int4 it = items[blockIdx.x];
+        col = it.x;
+        z0 = it.y;
+        z1 = it.z;
+    } else {
+        const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
+        const int64_t ncol = (int64_t)ntx * nty;
+        const int chunk = (int)(tile / ncol);
+        col = (int)(tile - chunk * ncol);
+        z0 = chunk * tz;
+        z1 = min(z0 + tz, planes);
+    }
+    ty = col / ntx;
+    tx = col - ty * ntx;
+}
+
 }  // namespace ppmg
