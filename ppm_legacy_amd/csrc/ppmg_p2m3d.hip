@@ -32,8 +32,8 @@ namespace ppmg {
 
 constexpr int P3_TT = 13;   // owned nodes per tile along x (16-lane DPP row = 13 + 3 halo cells)
 constexpr int P3_TY = 21;   // owned node rows per tile along y (24 cell rows: 6 chunks, 3 wavefronts)
-constexpr int P3_SERIAL = 4; // later rounds with at most this many active lanes go one particle at a time
-constexpr int P3_STAGE = 15; // second particles of a chunk staged in LDS (more take a full round)
+constexpr int P3_STAGE = 15; // particles of a chunk staged in LDS at a time
+constexpr int P3_FEW = 8;    // a round of at most this many particles is staged rather than taken by all lanes
 
 // LDS accumulator of one node component.  Every form accumulates in an FP64
 // slot with ds_add_f64 (fire-and-forget, no read-modify-write latency chain):
@@ -125,7 +125,7 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     constexpr int NC = NW == 1 ? NQ : 2;           // chunks per wavefront and plane
     constexpr int PLANE = P3_PL * LDA;            // slots per ring plane: [c][node]
     __shared__ slot_t ring[RP * PLANE];
-    // Second particles of a wavefront's chunk: [1D weights x, y, z and
+    // Staged particles of a wavefront's chunk: [1D weights x, y, z and
     // strengths][particle].  15 apart, the four values a stencil offset picks
     // from lie in different banks.
     constexpr int NV = 3 * KS + LDA;
@@ -346,24 +346,23 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                     }
                 }
             };
-            // Second particles, where at most P3_STAGE cells of the chunk have one
-            // (41% of an advected lattice's chunks do, with 5 such cells on
-            // average): their weights go to LDS ahead of round 0, so that nothing
-            // is waited for when they are deposited after it.  512^3, FP64, lda
-            // 3, advected by up to half a cell: deposit 5.33 -> 5.08 ms against
-            // loading them after round 0 (a full round for more than four cells,
-            // each of the others on its own); 3.84 ms with them left out.  What
-            // they cost now is their LDS traffic: three 64-lane atomics and six
-            // reads each.
-            const uint64_t act1 = __ballot(cnt > 1);
-            const int nl = (int)__popcll(act1);
-            const bool staged = nl > 0 && nl <= P3_STAGE;
-            if (staged) {
+            // A full round costs the same however few lanes hold a particle, so
+            // few particles are staged instead: their weights go to LDS and each
+            // is deposited by the 64 lanes (about 25 instructions, three atomics
+            // and six reads each, against 430 for a round).
+            //   * round 0 of a chunk with at most P3_FEW particles (sparse space);
+            //   * second particles, where at most P3_STAGE cells have one: 41% of an
+            //     advected lattice's chunks do, with 5 such cells on average.  Their
+            //     data came with round 0's, so nothing is waited for: deposit at
+            //     512^3, FP64, lda 3, advected by up to half a cell 5.33 -> 5.08 ms
+            //     against loading them after round 0 (3.84 ms without them);
+            //   * the rest once at most P3_FEW cells have particles left.
+            // put: particle of slot k's weights and strengths
+            auto put = [&](int k, bool has, const PD (&x)[NPD], const ValT (&u)[LDA]) {
                 ValT wx[KS], wy[KS], wz[KS];
-                weights(xl, wx, wy, wz);
-                if (cnt > 1) {
-                    ValT* q = stage + __builtin_amdgcn_mbcnt_hi((unsigned)(act1 >> 32),
-                                                                __builtin_amdgcn_mbcnt_lo((unsigned)act1, 0u));
+                weights(x, wx, wy, wz);
+                if (has) {
+                    ValT* q = stage + k;
 #pragma unroll
                     for (int o = 0; o < KS; ++o) {
                         q[o * P3_STAGE] = wx[o];
@@ -371,82 +370,93 @@ k_p3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                         q[(2 * KS + o) * P3_STAGE] = wz[o];
                     }
 #pragma unroll
-                    for (int c = 0; c < LDA; ++c) q[(3 * KS + c) * P3_STAGE] = ul[c];
+                    for (int c = 0; c < LDA; ++c) q[(3 * KS + c) * P3_STAGE] = u[c];
                 }
                 wave_lds_sync();
-            }
+            };
             const int qrow = ey4[j] - erow;          // first cell row of the chunk
-            // round 0 with the particle loaded during the previous step
-            if (__ballot(cnt > 0) != 0ull) round(xn, un);
-            // the staged second particles, one at a time
-            if (staged) {
-                int sox, soy, soz;
-                const bool slane = stencil_lane(sox, soy, soz);
-                slot_t* pl = ring + ((cz - B + soz) & (RP - 1)) * PLANE;
-                uint64_t a = act1;
-                for (int k = 0; k < nl; ++k) {
-                    const int src = __builtin_ctzll(a);
-                    a &= a - 1;
-                    const int nx = (src & 15) - H + sox, ny = qrow + (src >> 4) - H + soy;
+            // n staged particles in slot order; lane_of(k): the window lane of slot k's cell
+            auto deposit = [&](int n, auto lane_of) {
+                int ox, oy, oz;
+                const bool slane = stencil_lane(ox, oy, oz);
+                slot_t* pl = ring + ((cz - B + oz) & (RP - 1)) * PLANE;
+                for (int k = 0; k < n; ++k) {
+                    const int src = lane_of(k);
+                    const int nx = (src & 15) - H + ox, ny = qrow + (src >> 4) - H + oy;
                     const bool own = slane && (unsigned)nx < (unsigned)nxo && (unsigned)ny < (unsigned)nyo;
                     const ValT* q = stage + k;
-                    const ValT wyz = q[(KS + soy) * P3_STAGE] * q[(2 * KS + soz) * P3_STAGE];
-                    const ValT wxo = q[sox * P3_STAGE];
+                    const ValT wyz = q[(KS + oy) * P3_STAGE] * q[(2 * KS + oz) * P3_STAGE];
+                    const ValT wxo = q[ox * P3_STAGE];
                     if (own) {
 #pragma unroll
                         for (int c = 0; c < LDA; ++c)
                             A::add(pl + c * P3_PL + nx + TT * ny, wyz * (wxo * q[(3 * KS + c) * P3_STAGE]));
                     }
                 }
-            }
-            // Later rounds load their own particles.  A round costs the same
-            // however few lanes still have a particle, so once at most P3_SERIAL
-            // lanes do, their remaining particles are deposited one at a time:
-            // the 64 lanes take the 64 nodes of the particle's stencil (distinct
-            // nodes, so the additions stay in a fixed order; with KS = 2 lanes
-            // 0..7 take the 8 nodes).
-            for (int r = staged ? 2 : 1;; ++r) {
-                uint64_t act = __ballot(cnt > r);
-                if (act == 0ull) break;
-                if (__popcll(act) > P3_SERIAL) {
-                    PD x[NPD];
-                    ValT u[LDA];
-                    const int p = cnt > r ? entry(first, r) : 0;
-                    load(p, cnt > r, x, u);
-                    round(x, u);
-                    continue;
-                }
-                int ox, oy, oz;
-                const bool slane = stencil_lane(ox, oy, oz);
-                slot_t* pl = ring + ((cz - B + oz) & (RP - 1)) * PLANE;
-                do {
-                    const int src = __builtin_ctzll(act);
-                    act &= act - 1;
-                    const int sf = __builtin_amdgcn_readlane(first, src);
-                    const int sc = __builtin_amdgcn_readlane(cnt, src);
-                    // node of this lane's stencil offset, relative to the tile
-                    const int nx = (src & 15) - H + ox, ny = qrow + (src >> 4) - H + oy;
-                    const bool own = slane && nx >= 0 && nx < nxo && ny >= 0 && ny < nyo;
-                    for (int rr = r; rr < sc; ++rr) {
-                        PD x[NPD];
-                        ValT u[LDA], wyz, wxo;
-                        load(entry(sf, rr), true, x, u);
-                        if constexpr (TAB) {
-                            wyz = x[KS + oy] * x[2 * KS + oz];
-                            wxo = x[ox];
-                        } else {
-                            ValT fr[3];
-                            offsets(x, fr);
-                            wyz = tile_weight_at<KS, ValT>(fr[1], oy) * tile_weight_at<KS, ValT>(fr[2], oz);
-                            wxo = tile_weight_at<KS, ValT>(fr[0], ox);
-                        }
-                        if (own) {
+                wave_lds_sync();
+            };
+            const uint64_t act0 = __ballot(cnt > 0), act1 = __ballot(cnt > 1);
+            const bool few = act0 != 0ull && __popcll(act0) <= P3_FEW;
+            const bool second = !few && act1 != 0ull && __popcll(act1) <= P3_STAGE;
+            const uint64_t staged = few ? act0 : second ? act1 : 0ull;
+            if (staged) {
+                if (few) {
 #pragma unroll
-                            for (int c = 0; c < LDA; ++c) A::add(pl + c * P3_PL + nx + TT * ny, wyz * (wxo * u[c]));
-                        }
+                    for (int d = 0; d < NPD; ++d) xl[d] = xn[d];
+#pragma unroll
+                    for (int c = 0; c < LDA; ++c) ul[c] = un[c];
+                }
+                put((int)__builtin_amdgcn_mbcnt_hi((unsigned)(staged >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)staged, 0u)),
+                    cnt > (few ? 0 : 1), xl, ul);
+            }
+            // round 0 with the particle loaded during the previous step
+            if (act0 != 0ull && !few) round(xn, un);
+            if (staged) {
+                uint64_t a = staged;
+                deposit((int)__popcll(staged), [&](int) {
+                    const int src = __builtin_ctzll(a);
+                    a &= a - 1;
+                    return src;
+                });
+            }
+            // Later rounds load their own particles, the entry of the next round's
+            // ahead of this one's arithmetic.
+            int r = second ? 2 : 1;
+            uint64_t act = __ballot(cnt > r);
+            int pr = act != 0ull && cnt > r ? entry(first, r) : 0;
+            while (__popcll(act) > P3_FEW) {
+                PD x[NPD];
+                ValT u[LDA];
+                load(pr, cnt > r, x, u);
+                pr = cnt > r + 1 ? entry(first, r + 1) : 0;
+                round(x, u);
+                ++r;
+                act = __ballot(cnt > r);
+            }
+            // the particles left, cell by cell, P3_STAGE at a time: their loads
+            // are in flight together
+            for (int done = 0, left = act != 0ull ? 1 : 0; left > 0; done += P3_STAGE) {
+                int total = 0, msrc = 0, mp = -1;   // this lane's particle: its cell's lane, its place there
+                for (uint64_t a = act; a != 0ull; a &= a - 1) {
+                    const int src = __builtin_ctzll(a);
+                    const int n = __builtin_amdgcn_readlane(cnt, src) - r, k = done + lane - total;
+                    if (k >= 0 && k < n) {
+                        msrc = src;
+                        mp = r + k;
                     }
-                } while (act != 0ull);
-                break;
+                    total += n;
+                }
+                left = total - done;
+                const int n = min(left, P3_STAGE);
+                const int mf = __shfl(first, msrc, 64);
+                const bool has = lane < n;
+                PD x[NPD];
+                ValT u[LDA];
+                load(has ? entry(mf, mp) : 0, has, x, u);
+                put(lane, has, x, u);
+                deposit(n, [&](int k) { return __builtin_amdgcn_readlane(msrc, k); });
+                left -= n;
             }
             load(pn, count_of(f1, n1) > 0, xn, un);
             load(pl2, count_of(f1, n1) > 1, xl, ul);
