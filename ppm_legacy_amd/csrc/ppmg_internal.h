@@ -436,6 +436,7 @@ struct ppmg_plan {
     int64_t ncells = 0;
     bool sorted_input = false;   // last binning found the input already in cell order
     int64_t crowded_cells = 0;   // estimate (1-in-64 sample) of the last binning's cells holding nine or more particles
+    int64_t far_particles = 0;   // ... and of its particles more than 1024 cells from the one before them
     // The last binning left a slot table (ppmg::TABLE_SLOTS int32 planes of
     // ncells: particle r of cell c at table[r * ncells + c], with the byte
     // counts in `count`) instead of `start` and `perm`; materialize_heads()

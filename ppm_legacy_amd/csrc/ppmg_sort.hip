@@ -18,14 +18,25 @@ namespace ppmg {
 // seen, err[2] queued runs of empty cells, err[3] a byte count overflowed,
 // err[4] a cell with more particles than the slot table holds, err[5] a
 // particle p not in cell p, err[6] (the gather's check of a lattice
-// binning) the same, err[8..71] sampled crowded cells.
-constexpr int ERR_WORDS = 72;
+// binning) the same, err[8..71] sampled crowded cells, err[72..135] sampled
+// particles far from the one before them.
+constexpr int ERR_WORDS = 136;
+// Input of FAR_MIN_NP particles or more, of which at least a quarter lie more
+// than FAR_CELLS cells from their predecessor, is in no order: the slot atomics
+// and table writes of its key pass each touch a line of their own.
+constexpr int FAR_CELLS = 1024;
+constexpr int64_t FAR_MIN_NP = 1 << 21;
+// Particles from which util_rank sorts by radix.
+constexpr int64_t RANK_RADIX_NP = 1 << 20;
 
 constexpr int SCAN_BLOCK = 256;
 constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
+static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b > 0 ? (n + b - 1) / b : 1); }
+
 // Block-wide exclusive scan of one value per thread; returns the block total.
+template <int THREADS = SCAN_BLOCK>
 __device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* sh, int64_t& excl) {
     const int t = threadIdx.x;
     const int lane = t & 63;
@@ -41,16 +52,16 @@ __device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* sh, 
     __syncthreads();
     if (t == 0) {
         int64_t run = 0;
-        for (int w = 0; w < SCAN_BLOCK / 64; ++w) {
+        for (int w = 0; w < THREADS / 64; ++w) {
             int64_t s = sh[w];
             sh[w] = run;
             run += s;
         }
-        sh[SCAN_BLOCK / 64] = run;
+        sh[THREADS / 64] = run;
     }
     __syncthreads();
     excl = x - v + sh[wid];
-    int64_t total = sh[SCAN_BLOCK / 64];
+    int64_t total = sh[THREADS / 64];
     __syncthreads();
     return total;
 }
@@ -332,7 +343,7 @@ __global__ void __launch_bounds__(256) k_keys(const PosT* __restrict__ xp, int64
 #pragma unroll
     for (int d = 0; d < DIM; ++d) sv[d] = has_seam ? xp[(w0 - 1) * DIM + d] : PosT(0);
     int k[KEYS_PPT];
-    int nbad = 0;
+    int nbad = 0, nfar = 0;
     uint64_t anydesc = 0, notlat = 0;
     bool desc[KEYS_PPT];
     int prev = has_seam ? cell_key<DIM, PosT>(sv, m) : -1;   // key before run j's lane 0
@@ -346,6 +357,7 @@ __global__ void __launch_bounds__(256) k_keys(const PosT* __restrict__ xp, int64
         prev = __builtin_amdgcn_readlane(k[j], 63);
         desc[j] = live && p > 0 && k[j] < left;
         nbad += (int)__popcll(__ballot(live && k[j] < 0));
+        if (SLOT) nfar += (int)__popcll(__ballot(live && p > 0 && abs(k[j] - left) > FAR_CELLS));
         anydesc |= __ballot(desc[j]);
         notlat |= __ballot(live && k[j] != (int)p);
         if (!SLOT) {
@@ -363,6 +375,7 @@ __global__ void __launch_bounds__(256) k_keys(const PosT* __restrict__ xp, int64
             if (nbad) atomicAdd(&err[0], nbad);
             if (anydesc && *(volatile int*)&err[1] == 0) err[1] = 1;
             if (notlat && *(volatile int*)&err[5] == 0) err[5] = 1;
+            if (SLOT && nfar && (blockIdx.x & 63) == 0) atomicAdd(&err[72 + ((blockIdx.x >> 6) & 63)], nfar);
         }
     };
     if (!SLOT) report();
@@ -455,15 +468,20 @@ __global__ void __launch_bounds__(256) k_identity(int64_t np, int* __restrict__ 
 
 
 // Cell key with the arithmetic of ppm_util_rank3d.f:414-475 (FLOOR, ghost
-// cells, upper-boundary corrections, -1 for particles in no box).
-template <int DIM, typename PosT>
+// cells, upper-boundary corrections).  SLOT: arrival slots by atomic counts,
+// key -1 for particles in no box; otherwise (for the radix sort) those get the
+// key past the last box.  stats[0] counts the particles in no box, stats[1]
+// the corrections.
+template <int DIM, typename PosT, bool SLOT>
 __global__ void __launch_bounds__(256) k_rank_keys(const PosT* __restrict__ xp, int64_t np,
                                                    RankGeom g, int* __restrict__ key,
                                                    int* __restrict__ slot, int* __restrict__ count,
                                                    int* __restrict__ stats) {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const PosT* x = xp + p * DIM;
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = p < np;
+    PosT x[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) x[d] = live ? xp[p * DIM + d] : (PosT)g.xmin[d];
     int idx[3] = {0, 0, 0};
     int corr = 0;
     bool in = true;
@@ -481,15 +499,17 @@ __global__ void __launch_bounds__(256) k_rank_keys(const PosT* __restrict__ xp, 
         if (x[d] < mx && idx[d] >= g.nm[d] + g.ngl_lo[d]) { idx[d] = g.nm[d] + g.ngl_lo[d] - 1; ++corr; }
         if (idx[d] < 0 || idx[d] >= g.ntot[d]) in = false;
     }
-    if (corr) atomicAdd(&stats[1], corr);
-    if (!in) {
-        key[p] = -1;
-        atomicAdd(&stats[0], 1);
-        return;
+    if (live && corr) atomicAdd(&stats[1], corr);
+    const uint64_t out = __ballot(live && !in);
+    if (out != 0ull && (threadIdx.x & 63) == 0) atomicAdd(&stats[0], (int)__popcll(out));
+    if (!live) return;
+    const int k = idx[0] + g.ntot[0] * (idx[1] + g.ntot[1] * idx[2]);
+    if constexpr (SLOT) {
+        key[p] = in ? k : -1;
+        if (in) slot[p] = atomicAdd(&count[k], 1);
+    } else {
+        key[p] = in ? k : g.ntot[0] * g.ntot[1] * g.ntot[2];
     }
-    int k = idx[0] + g.ntot[0] * (idx[1] + g.ntot[1] * idx[2]);
-    key[p] = k;
-    slot[p] = atomicAdd(&count[k], 1);
 }
 
 // Four particles per thread: keys and slots as vector loads (plan buffers
@@ -634,7 +654,6 @@ __global__ void k_fill_zero(uint32_t* __restrict__ p, int64_t n) {
     for (; i < n; i += stride) p[i] = 0u;
 }
 
-static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b > 0 ? (n + b - 1) / b : 1); }
 
 // Zero fill with a kernel (graph-capture safe, unlike hipMemsetAsync).
 int fill_zero(void* p, size_t bytes, hipStream_t s) {
@@ -664,16 +683,21 @@ __global__ void __launch_bounds__(256) k_keys_only(const PosT* __restrict__ xp, 
 // k_keys' atomic slots contend on the crowded cells' count words, the scatter
 // writes at random and the per-cell insertion sorts grow with the square of
 // the occupancy.  Such input is binned by a stable LSD radix sort of the
-// (cell key, particle) pairs instead, RS_BITS bits a pass: no atomics on
+// (cell key, particle) pairs instead: no atomics on
 // crowded words, writes in runs, and a stable sort of the keys in particle
 // order is the reference's permutation as it stands (ppm_util_rank3d.f:
-// 505-532).  The heads follow from the runs of the sorted keys.
-constexpr int RS_THREADS = 256;
+// 505-532).  The heads follow from the runs of the sorted keys.  Large input
+// in no order takes the same path, and so does util_rank.
+//
+// A pass sorts by 8 or 9 bits, whichever takes fewer passes over the key's
+// bits (27 bits at 512^3: three passes of 9), with one thread per digit.
 constexpr int RS_ITEMS = 8;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;   // pairs per workgroup
-constexpr int RS_BITS = 8;
-constexpr int RS_BUCKETS = 1 << RS_BITS;
-static_assert(RS_BUCKETS == RS_THREADS, "one digit per thread in the tile loops");
+template <int BITS> struct Radix {
+    static constexpr int BUCKETS = 1 << BITS;
+    static constexpr int THREADS = BUCKETS;                // one digit per thread in the tile loops
+    static constexpr int TILE = THREADS * RS_ITEMS;        // pairs per workgroup
+    static constexpr int NWAVE = THREADS / 64;
+};
 
 // Keys of all particles (key[p]), the particles in no cell (err[0]) and the
 // descent flag (err[1]), as k_keys reports them.
@@ -696,18 +720,21 @@ __global__ void __launch_bounds__(256) k_keys_plain(const PosT* __restrict__ xp,
     int left = __shfl_up(k, 1);
     if (lane == 0) left = seam;
     const uint64_t bb = __ballot(live && k < 0), bd = __ballot(live && p > 0 && k < left);
+    const int nfar = (int)__popcll(__ballot(live && p > 0 && abs(k - left) > FAR_CELLS));
     if (live) key[p] = k;
     if (lane == 0) {
         if (bb) atomicAdd(&err[0], (int)__popcll(bb));
         if (bd && *(volatile int*)&err[1] == 0) err[1] = 1;
+        if (nfar && (blockIdx.x & 63) == 0) atomicAdd(&err[72 + ((blockIdx.x >> 6) & 63)], nfar);
     }
 }
 
 // Lanes of the wavefront holding the same digit as this lane (among `live`).
+template <int BITS>
 __device__ __forceinline__ uint64_t digit_peers(int d, bool live) {
     uint64_t peers = __ballot(live);
 #pragma unroll
-    for (int b = 0; b < RS_BITS; ++b) {
+    for (int b = 0; b < BITS; ++b) {
         const uint64_t on = __ballot((d >> b) & 1);
         peers &= ((d >> b) & 1) ? on : ~on;
     }
@@ -717,21 +744,28 @@ __device__ __forceinline__ uint64_t digit_peers(int d, bool live) {
 // Digit counts of every tile, digit-major: hist[d * ntiles + tile].  Tiles
 // are numbered XCD-contiguously (xcd_tile), as in k_rs_scatter: the tiles
 // one XCD sorts are neighbours, and so are their runs of each digit.
-__global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const int* __restrict__ keys, int64_t n, int shift,
-                                                        int* __restrict__ hist, int64_t ntiles) {
-    __shared__ int h[RS_BUCKETS];
+template <int BITS>
+__global__ void __launch_bounds__(Radix<BITS>::THREADS) k_rs_hist(const int* __restrict__ keys, int64_t n, int shift,
+                                                                  int* __restrict__ hist, int64_t ntiles) {
+    using R = Radix<BITS>;
+    __shared__ int h[R::BUCKETS];
     const int tid = threadIdx.x, lane = tid & 63;
     const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
     h[tid] = 0;
     __syncthreads();
-    const int64_t t0 = tile * RS_TILE;
+    const int64_t t0 = tile * R::TILE;
+    int k[RS_ITEMS];   // all loads in flight before the first count
 #pragma unroll
     for (int j = 0; j < RS_ITEMS; ++j) {
-        const int64_t i = t0 + j * RS_THREADS + tid;
-        const bool live = i < n;
-        const int d = live ? (keys[i] >> shift) & (RS_BUCKETS - 1) : 0;
+        const int64_t i = t0 + j * R::THREADS + tid;
+        k[j] = i < n ? keys[i] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j) {
+        const bool live = t0 + j * R::THREADS + tid < n;
+        const int d = (k[j] >> shift) & (R::BUCKETS - 1);
         // one LDS add per digit and wavefront
-        const uint64_t peers = digit_peers(d, live);
+        const uint64_t peers = digit_peers<BITS>(d, live);
         if (live && (int)__builtin_ctzll(peers) == lane) atomicAdd(&h[d], (int)__popcll(peers));
     }
     __syncthreads();
@@ -739,146 +773,232 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const int* __restrict__ 
 }
 
 // One stable pass.  The pairs of a tile are first ordered by digit in LDS: a
-// tile is taken RS_THREADS pairs a round in index order, and a pair's place
+// tile is taken THREADS pairs a round in index order, and a pair's place
 // is its digit's start in the tile plus its rank among the tile's pairs of
 // that digit (the count from earlier rounds, earlier wavefronts of its round
 // and earlier lanes of its wavefront).  The tile then writes its digit runs
 // at their offsets (offs: the exclusive scan of hist), consecutive threads to
 // consecutive addresses.  vin nullptr: the values are the pairs' indices
-// (the first pass).
-__global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const int* __restrict__ kin, const int* __restrict__ vin,
-                                                           int64_t n, int shift, const int* __restrict__ hist,
-                                                           const int* __restrict__ offs, int64_t ntiles,
-                                                           int* __restrict__ kout, int* __restrict__ vout) {
-    constexpr int NWAVE = RS_THREADS / 64;
-    __shared__ int base[RS_BUCKETS];     // next place of each digit in the tile's order
-    __shared__ int shift_out[RS_BUCKETS];   // global position minus place, per digit
-    __shared__ int wcnt[NWAVE][RS_BUCKETS];
-    __shared__ int sk[RS_TILE], sv[RS_TILE];
-    __shared__ int64_t sh[RS_THREADS / 64 + 1];
+// (the first pass); vadd is added to the values written (1: one-based ranks).
+// vmax: values at positions from vmax on are not written.
+template <int BITS>
+__global__ void __launch_bounds__(Radix<BITS>::THREADS)
+k_rs_scatter(const int* __restrict__ kin, const int* __restrict__ vin, int64_t n, int shift,
+             const int* __restrict__ hist, const int* __restrict__ offs, int64_t ntiles, int* __restrict__ kout,
+             int* __restrict__ vout, int vadd, int64_t vmax) {
+    using R = Radix<BITS>;
+    __shared__ int base[R::BUCKETS];     // next place of each digit in the tile's order
+    __shared__ int shift_out[R::BUCKETS];   // global position minus place, per digit
+    __shared__ int wcnt[R::NWAVE][R::BUCKETS];
+    __shared__ int sk[R::TILE], sv[R::TILE];
+    __shared__ int64_t sh[R::NWAVE + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t t0 = tile * RS_TILE;
-    const int tn = (int)min((int64_t)RS_TILE, n - t0);
+    const int64_t t0 = tile * R::TILE;
+    const int tn = (int)min((int64_t)R::TILE, n - t0);
+    int kk[RS_ITEMS], vv[RS_ITEMS];   // all loads in flight before the first round
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j) {
+        const int64_t i = t0 + j * R::THREADS + tid;
+        kk[j] = i < n ? kin[i] : 0;
+        vv[j] = i < n ? (vin ? vin[i] : (int)i) : 0;
+    }
     // thread t = digit t: its start in the tile (exclusive scan of the tile's counts)
     int64_t lb;
-    block_exclusive_scan((int64_t)hist[(int64_t)tid * ntiles + tile], sh, lb);
+    block_exclusive_scan<R::THREADS>((int64_t)hist[(int64_t)tid * ntiles + tile], sh, lb);
     base[tid] = (int)lb;
     shift_out[tid] = offs[(int64_t)tid * ntiles + tile] - (int)lb;
 #pragma unroll
-    for (int w = 0; w < NWAVE; ++w) wcnt[w][tid] = 0;
+    for (int w = 0; w < R::NWAVE; ++w) wcnt[w][tid] = 0;
     const uint64_t lt = lane ? ~0ull >> (64 - lane) : 0ull;   // lanes below this one
     __syncthreads();
+#pragma unroll
     for (int j = 0; j < RS_ITEMS; ++j) {
-        const int64_t i = t0 + j * RS_THREADS + tid;
-        const bool live = i < n;
-        const int k = live ? kin[i] : 0;
-        const int v = live ? (vin ? vin[i] : (int)i) : 0;
-        const int d = (k >> shift) & (RS_BUCKETS - 1);
-        const uint64_t peers = digit_peers(d, live);
+        const bool live = t0 + j * R::THREADS + tid < n;
+        const int d = (kk[j] >> shift) & (R::BUCKETS - 1);
+        const uint64_t peers = digit_peers<BITS>(d, live);
         if (live && (int)__builtin_ctzll(peers) == lane) wcnt[wave][d] = (int)__popcll(peers);
         __syncthreads();
         if (live) {
             int r = base[d] + (int)__popcll(peers & lt);
             for (int w = 0; w < wave; ++w) r += wcnt[w][d];
-            sk[r] = k;
-            sv[r] = v;
+            sk[r] = kk[j];
+            sv[r] = vv[j];
         }
         __syncthreads();
         // thread t owns digit t: advance its place, clear its counts
         int add = 0;
 #pragma unroll
-        for (int w = 0; w < NWAVE; ++w) {
+        for (int w = 0; w < R::NWAVE; ++w) {
             add += wcnt[w][tid];
             wcnt[w][tid] = 0;
         }
         base[tid] += add;
         __syncthreads();
     }
-    for (int q = tid; q < tn; q += RS_THREADS) {
+    for (int q = tid; q < tn; q += R::THREADS) {
         const int k = sk[q];
-        const int o = shift_out[(k >> shift) & (RS_BUCKETS - 1)] + q;
+        const int o = shift_out[(k >> shift) & (R::BUCKETS - 1)] + q;
         kout[o] = k;
-        vout[o] = sv[q];
+        if (o < vmax) vout[o] = sv[q] + vadd;
     }
 }
 
-// Cell counts from the sorted keys: each run of equal keys adds its length
-// to cnt[key] (zeroed) by two atomics at its ends, on distinct runs' words;
-// a run of one particle stores its count.
-// (Writing the heads straight from the runs, as the cell-order path does,
-// took longer on crowded input: most cells are empty, and a lane fills each
-// run of empty cells before its own or queues it on one counter word.)  One
-// workgroup in 64 counts its runs of nine or more into err[8 .. 71] (the
-// same sample k_keys takes).
-__global__ void __launch_bounds__(256) k_rs_runs(const int* __restrict__ ks, int64_t n, int* __restrict__ cnt,
-                                                 int* __restrict__ err) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool crowd = false;
-    if (i < n) {
-        const int k = ks[i];
-        const bool first = i == 0 || ks[i - 1] != k, last = i == n - 1 || ks[i + 1] != k;
-        if (first && last) {
-            cnt[k] = 1;
-        } else {
-            if (first) atomicAdd(&cnt[k], -(int)i);
-            if (last) atomicAdd(&cnt[k], (int)i + 1);
+// Heads from sorted keys: start[c] + add = first position whose key is c or
+// more, for c = 0 .. ncells - 1, and start[ncells] = n + add.  A workgroup
+// takes HEADS_CELLS cells: its wavefronts find the cells' range of the keys
+// by a 64-way search, the first key of each run notes its position in LDS, and
+// empty cells take the position of the next run.  Bound by memory: the keys
+// are read and the heads written once (2^26 crowded keys in 2^27 cells: 0.38
+// ms; the runs' lengths by atomics into zeroed counts and a scan of them took
+// 0.85 ms).  One
+// workgroup in `stride` counts its cells of nine particles or more into
+// err[8 .. 71] (err NULL: none does).
+constexpr int HEADS_CELLS = 4096;
+constexpr int HEADS_PER = HEADS_CELLS / 256;
+__global__ void __launch_bounds__(256) k_heads(const int* __restrict__ ks, int64_t n, int64_t ncells,
+                                               int* __restrict__ start, int add, int stride, int* __restrict__ err) {
+    __shared__ int pos[HEADS_CELLS];
+    __shared__ int64_t range[2];
+    __shared__ int wmin[4], ncrowd;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t c0 = (int64_t)blockIdx.x * HEADS_CELLS;
+    const int nc = (int)min((int64_t)HEADS_CELLS, ncells - c0);
+    for (int i = tid; i < HEADS_CELLS; i += 256) pos[i] = INT_MAX;
+    if (tid == 0) ncrowd = 0;
+    if (wave < 2) {
+        // first position whose key is not below `want`, in [lo, hi]
+        const int64_t want = wave == 0 ? c0 : c0 + nc;
+        int64_t lo = 0, hi = n;
+        while (lo < hi) {
+            // probes lo + (l + 1) step - 1, l = 0 .. 63, past hi taken as found
+            const int64_t step = (hi - lo + 63) / 64, at = lo + (lane + 1) * step - 1;
+            const bool below = at < hi && (int64_t)ks[at] < want;
+            const int m = (int)__popcll(__ballot(below));   // probes below: a prefix of the lanes
+            const int64_t nlo = lo + m * step, nhi = lo + (int64_t)(m + 1) * step - 1;
+            lo = nlo;
+            hi = nhi < hi ? nhi : hi;
         }
-        crowd = last && i >= 8 && ks[i - 8] == k;
+        if (lane == 0) range[wave] = lo;
     }
-    if ((blockIdx.x & 63) == 0) {
-        const uint64_t c = __ballot(crowd);
-        if (c && (threadIdx.x & 63) == 0) atomicAdd(&err[8 + ((blockIdx.x >> 6) & 63)], (int)__popcll(c));
+    __syncthreads();
+    const int64_t r0 = range[0], r1 = range[1];
+    for (int64_t i0 = r0; i0 < r1; i0 += 4 * 256) {
+        int k[4], left[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t i = i0 + j * 256 + tid;
+            k[j] = i < r1 ? ks[i] : -1;
+            left[j] = i < r1 && i > r0 ? ks[i - 1] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (k[j] >= 0 && k[j] != left[j]) pos[k[j] - (int)c0] = (int)(i0 + j * 256 + tid);
     }
+    __syncthreads();
+    // suffix minimum: a thread's HEADS_PER cells, then the threads after it
+    int v[HEADS_PER];
+    int run = INT_MAX;
+#pragma unroll
+    for (int i = HEADS_PER - 1; i >= 0; --i) {
+        run = min(run, pos[tid * HEADS_PER + i]);
+        v[i] = run;
+    }
+    int after = run;   // minimum over lanes >= this one
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_down(after, o, 64);
+        if (lane + o < 64) after = min(after, y);
+    }
+    if (lane == 0) wmin[wave] = after;
+    int next = __shfl_down(after, 1, 64);
+    if (lane == 63) next = INT_MAX;
+    __syncthreads();
+    for (int w = wave + 1; w < 4; ++w) next = min(next, wmin[w]);
+    next = min(next, (int)r1);
+#pragma unroll
+    for (int i = 0; i < HEADS_PER; ++i) v[i] = min(v[i], next);
+    const bool sampled = err && blockIdx.x % stride == 0;
+    int crowd = 0;
+#pragma unroll
+    for (int i = 0; i < HEADS_PER; ++i) crowd += (i + 1 < HEADS_PER ? v[i + 1] : next) - v[i] >= 9;
+    if (sampled && crowd) atomicAdd(&ncrowd, crowd);
+    int* out = start + c0 + tid * HEADS_PER;
+    if (nc == HEADS_CELLS && (reinterpret_cast<uintptr_t>(start) & 15) == 0) {
+        int4* q = reinterpret_cast<int4*>(out);
+#pragma unroll
+        for (int i = 0; i < HEADS_PER / 4; ++i)
+            q[i] = make_int4(v[4 * i] + add, v[4 * i + 1] + add, v[4 * i + 2] + add, v[4 * i + 3] + add);
+    } else {
+#pragma unroll
+        for (int i = 0; i < HEADS_PER; ++i)
+            if (tid * HEADS_PER + i < nc) out[i] = v[i] + add;
+    }
+    if (c0 + nc == ncells && tid == 0) start[ncells] = (int)r1 + add;
+    __syncthreads();
+    if (sampled && tid == 0 && ncrowd > 0) atomicAdd(&err[8 + (blockIdx.x / stride & 63)], ncrowd);
 }
 
-// Radix-sort binning of crowded input (see above); the keys pass has run.
-static int bin_radix(ppmg_plan* plan, int64_t np, int64_t ncells, hipStream_t s, const int** sorted_keys) {
-    const int64_t ntiles = (np + RS_TILE - 1) / RS_TILE;
-    if (plan->rkey[0].ensure(sizeof(int) * (size_t)np) || plan->rkey[1].ensure(sizeof(int) * (size_t)np) ||
-        plan->rval[0].ensure(sizeof(int) * (size_t)np) || plan->rval[1].ensure(sizeof(int) * (size_t)np) ||
-        plan->rhist.ensure(sizeof(int) * (size_t)(2 * (RS_BUCKETS * ntiles + 4))))
+// Stable sort of n keys below 2^bits by LSD radix passes: the sorted keys
+// (*sorted_keys, in the plan's scratch), and the permutation (plus vadd) at
+// positions below vmax in vout.
+template <int BITS>
+static int radix_sort_bits(ppmg_plan* plan, const int* keys, int64_t n, int passes, int* vout, int vadd, int64_t vmax,
+                           hipStream_t s, const int** sorted_keys) {
+    using R = Radix<BITS>;
+    const int64_t ntiles = (n + R::TILE - 1) / R::TILE;
+    if (plan->rkey[0].ensure(sizeof(int) * (size_t)n) || plan->rkey[1].ensure(sizeof(int) * (size_t)n) ||
+        plan->rval[0].ensure(sizeof(int) * (size_t)n) || plan->rval[1].ensure(sizeof(int) * (size_t)n) ||
+        plan->rhist.ensure(sizeof(int) * (size_t)(2 * (R::BUCKETS * ntiles + 4))))
         return PPMG_ERROR_FATAL;
-    int bits = 1;
-    while (bits < 31 && ((int64_t)1 << bits) < ncells) ++bits;
-    const int passes = (bits + RS_BITS - 1) / RS_BITS;
     int* hist = plan->rhist.as<int>();
-    int* offs = hist + RS_BUCKETS * ntiles + 4;   // 16-byte aligned, n + 1 entries
-    const int* kin = plan->key.as<int>();
+    int* offs = hist + R::BUCKETS * ntiles + 4;   // 16-byte aligned, n + 1 entries
+    const int* kin = keys;
     const int* vin = nullptr;
     for (int pass = 0; pass < passes; ++pass) {
-        const int shift = pass * RS_BITS;
+        const int shift = pass * BITS;
         const bool last = pass == passes - 1;
         int* kout = plan->rkey[pass & 1].as<int>();
-        int* vout = last ? plan->perm.as<int>() : plan->rval[pass & 1].as<int>();
-        hipLaunchKernelGGL(k_rs_hist, dim3((unsigned)ntiles), dim3(RS_THREADS), 0, s, kin, np, shift, hist, ntiles);
-        if (exclusive_scan(hist, RS_BUCKETS * ntiles, offs, plan->scan_tmp, np, s)) return PPMG_ERROR_FATAL;
-        hipLaunchKernelGGL(k_rs_scatter, dim3((unsigned)ntiles), dim3(RS_THREADS), 0, s, kin, vin, np, shift, hist,
-                           offs, ntiles, kout, vout);
+        int* vo = last ? vout : plan->rval[pass & 1].as<int>();
+        hipLaunchKernelGGL(k_rs_hist<BITS>, dim3((unsigned)ntiles), dim3(R::THREADS), 0, s, kin, n, shift, hist, ntiles);
+        if (exclusive_scan(hist, R::BUCKETS * ntiles, offs, plan->scan_tmp, n, s)) return PPMG_ERROR_FATAL;
+        hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3((unsigned)ntiles), dim3(R::THREADS), 0, s, kin, vin, n, shift, hist,
+                           offs, ntiles, kout, vo, last ? vadd : 0, last ? vmax : n);
         kin = kout;
-        vin = vout;
+        vin = vo;
     }
     *sorted_keys = kin;
     PPMG_HIP(hipGetLastError());
     return 0;
 }
 
-// Heads of the sorted keys ks (run lengths into zeroed counts, then their
-// exclusive scan), and the plan's crowded-cell estimate from the sample.
+static int radix_sort(ppmg_plan* plan, const int* keys, int64_t n, int64_t nkeys, int* vout, int vadd, int64_t vmax,
+                      hipStream_t s, const int** sorted_keys) {
+    int bits = 1;
+    while (bits < 31 && ((int64_t)1 << bits) < nkeys) ++bits;
+    const int p8 = (bits + 7) / 8, p9 = (bits + 8) / 9;
+    if (p9 < p8) return radix_sort_bits<9>(plan, keys, n, p9, vout, vadd, vmax, s, sorted_keys);
+    return radix_sort_bits<8>(plan, keys, n, p8, vout, vadd, vmax, s, sorted_keys);
+}
+
+// Heads of the sorted keys ks, and the plan's crowded-cell estimate from a
+// sample of them.
 static int heads_from_sorted(ppmg_plan* plan, const int* ks, int64_t np, int64_t ncells, hipStream_t s) {
     int* err = plan->err.as<int>();
-    if (plan->count.ensure(sizeof(int) * (size_t)ncells)) return PPMG_ERROR_FATAL;
-    int* cnt = plan->count.as<int>();
-    if (fill_zero(cnt, sizeof(int) * (size_t)ncells, s)) return PPMG_ERROR_FATAL;
-    hipLaunchKernelGGL(k_rs_runs, dim3(nblk(np, 256)), dim3(256), 0, s, ks, np, cnt, err);
-    if (exclusive_scan(cnt, ncells, plan->start.as<int>(), plan->scan_tmp, np, s)) return PPMG_ERROR_FATAL;
+    const unsigned g = nblk(ncells, HEADS_CELLS);
+    const int stride = g > 2048 ? (int)(g / 2048) : 1;
+    hipLaunchKernelGGL(k_heads, dim3(g), dim3(256), 0, s, ks, np, ncells, plan->start.as<int>(), 0, stride, err);
     PPMG_HIP(hipGetLastError());
-    int sample[64];
+    int sample[128];
     PPMG_HIP(hipMemcpyAsync(sample, err + 8, sizeof(sample), hipMemcpyDeviceToHost, s));
     PPMG_HIP(hipStreamSynchronize(s));
-    int64_t sampled = 0;
-    for (int v : sample) sampled += v;
-    plan->crowded_cells = 64 * sampled;
+    int64_t crowd = 0, far = 0;
+    for (int i = 0; i < 64; ++i) {
+        crowd += sample[i];
+        far += sample[64 + i];
+    }
+    plan->crowded_cells = stride * crowd;
+    plan->far_particles = 64 * far;
     return 0;
 }
 
@@ -908,7 +1028,7 @@ static int bin_crowded(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, 
     // permutation the identity (written on demand)
     const bool sorted = herr[1] == 0;
     const int* ks = key;
-    if (!sorted && bin_radix(plan, np, ncells, s, &ks)) return PPMG_ERROR_FATAL;
+    if (!sorted && radix_sort(plan, key, np, ncells, plan->perm.as<int>(), 0, np, s, &ks)) return PPMG_ERROR_FATAL;
     if (heads_from_sorted(plan, ks, np, ncells, s)) return PPMG_ERROR_FATAL;
     plan->perm_identity = sorted;
     plan->perm_written = !sorted;
@@ -983,12 +1103,16 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     const bool use_table = table && !predict_sorted && plan->table_skip == 0 && !arena_bound();
     if (table && !predict_sorted && plan->table_skip > 0) --plan->table_skip;
     // Crowded input (the last binning's sample found a cell of nine or more
-    // particles per 64 particles) is binned by the radix sort; PPMG_RADIX=1
+    // particles per 64 particles), and large input in no order, is binned by the
+    // radix sort (16.8M particles of 256^3 cells in random order: 0.68 against
+    // 1.04 ms; the two meet at 2^21 particles, P2M 335 and 341 us); PPMG_RADIX=1
     // forces that path for input not predicted in cell order, PPMG_RADIX=0
     // rules it out (both for tests).  Allocation-free calls keep the counting
     // path (the sort needs four more int32 per particle).
     const char* rx = std::getenv("PPMG_RADIX");
-    const bool radix = rx && rx[0] ? rx[0] == '1' : plan->crowded_cells * 64 > np;
+    const bool radix = rx && rx[0] ? rx[0] == '1'
+                                   : plan->crowded_cells * 64 > np ||
+                                         (np >= FAR_MIN_NP && plan->far_particles * 4 > np);
     if (!predict_sorted && radix && !arena_bound()) return bin_crowded(plan, m, prec, np, xp, s, nbad);
     if (use_table && plan->table.ensure(sizeof(int) * TABLE_SLOTS * (size_t)ncells)) return PPMG_ERROR_FATAL;
     int* tab = use_table ? plan->table.as<int>() : nullptr;
@@ -1027,9 +1151,13 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     PPMG_HIP(hipMemcpyAsync(herr, plan->err.p, sizeof(int) * ERR_WORDS, hipMemcpyDeviceToHost, s));
     PPMG_HIP(hipStreamSynchronize(s));
     *nbad = herr[0];
-    int64_t sampled = 0;
-    for (int i = 8; i < ERR_WORDS; ++i) sampled += herr[i];
-    plan->crowded_cells = 64 * sampled;   // estimate from the 1-in-64 sample
+    int64_t crowd = 0, far = 0;
+    for (int i = 8; i < 72; ++i) {
+        crowd += herr[i];
+        far += herr[64 + i];
+    }
+    plan->crowded_cells = 64 * crowd;   // estimates from the 1-in-64 samples
+    plan->far_particles = 64 * far;
     if (herr[0]) return 0;
     plan->lattice_pred = herr[5] == 0 && np == ncells;
     plan->lattice_prec = prec;
@@ -1206,44 +1334,60 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
     // overwritten, so its heads are built first
     if (materialize_heads(plan, s)) return PPMG_ERROR_FATAL;
     plan->prebinned = false;
-    if (plan->key.ensure(sizeof(int) * (size_t)(np > 0 ? np : 1)) ||
-        plan->slot.ensure(sizeof(int) * (size_t)(np > 0 ? np : 1)) ||
-        plan->count.ensure(sizeof(int) * (size_t)ncells) || plan->err.ensure(sizeof(int) * 4))
+    // Large input is ranked by the radix sort of its cell keys (2^24 particles in
+    // no order, eight to a box: 0.56 against 1.34 ms; 2^20: 122 against 135 us,
+    // 2^19: 119 against 107); slot
+    // atomics and per-cell sorts keep the small ones, whose counts stay in L2
+    // and which have few launches (PPMG_RADIX forces either, as in the binning).
+    const char* rx = std::getenv("PPMG_RADIX");
+    const bool radix = np > 0 && (rx && rx[0] ? rx[0] == '1' : np >= RANK_RADIX_NP);
+    if (plan->key.ensure(sizeof(int) * (size_t)(np > 0 ? np : 1)) || plan->err.ensure(sizeof(int) * 4)) return PPMG_ERROR_FATAL;
+    if (!radix && (plan->slot.ensure(sizeof(int) * (size_t)(np > 0 ? np : 1)) ||
+                   plan->count.ensure(sizeof(int) * (size_t)ncells)))
         return PPMG_ERROR_FATAL;
-    if (fill_zero(plan->count.p, sizeof(int) * (size_t)ncells, s) || fill_zero(plan->err.p, sizeof(int) * 4, s))
+    if ((!radix && fill_zero(plan->count.p, sizeof(int) * (size_t)ncells, s)) || fill_zero(plan->err.p, sizeof(int) * 4, s))
         return PPMG_ERROR_FATAL;
     if (np > 0) {
         unsigned gr = nblk(np, 256);
         int* st = plan->err.as<int>();
+#define RANK_KEYS(D, T, S) hipLaunchKernelGGL((k_rank_keys<D, T, S>), dim3(gr), dim3(256), 0, s, (const T*)xp, np, g, \
+                                              plan->key.as<int>(), plan->slot.as<int>(), plan->count.as<int>(), st)
+#define RANK_KEYS_T(D, T)                      \
+    do {                                       \
+        if (radix) RANK_KEYS(D, T, false);     \
+        else RANK_KEYS(D, T, true);            \
+    } while (0)
+        const bool single = prec == PPMG_PREC_F32;
         if (g.dim == 3) {
-            if (prec == PPMG_PREC_F32)
-                hipLaunchKernelGGL((k_rank_keys<3, float>), dim3(gr), dim3(256), 0, s, (const float*)xp, np, g,
-                                   plan->key.as<int>(), plan->slot.as<int>(), plan->count.as<int>(), st);
-            else
-                hipLaunchKernelGGL((k_rank_keys<3, double>), dim3(gr), dim3(256), 0, s, (const double*)xp, np, g,
-                                   plan->key.as<int>(), plan->slot.as<int>(), plan->count.as<int>(), st);
+            if (single) RANK_KEYS_T(3, float);
+            else RANK_KEYS_T(3, double);
         } else {
-            if (prec == PPMG_PREC_F32)
-                hipLaunchKernelGGL((k_rank_keys<2, float>), dim3(gr), dim3(256), 0, s, (const float*)xp, np, g,
-                                   plan->key.as<int>(), plan->slot.as<int>(), plan->count.as<int>(), st);
-            else
-                hipLaunchKernelGGL((k_rank_keys<2, double>), dim3(gr), dim3(256), 0, s, (const double*)xp, np, g,
-                                   plan->key.as<int>(), plan->slot.as<int>(), plan->count.as<int>(), st);
+            if (single) RANK_KEYS_T(2, float);
+            else RANK_KEYS_T(2, double);
         }
+#undef RANK_KEYS_T
+#undef RANK_KEYS
         PPMG_HIP(hipGetLastError());
     }
     int stats[2] = {0, 0};
     PPMG_HIP(hipMemcpyAsync(stats, plan->err.p, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
     PPMG_HIP(hipStreamSynchronize(s));
     int64_t inside = np - stats[0];
-    if (exclusive_scan(plan->count.as<int>(), ncells, lhbx, plan->scan_tmp, inside, s)) return PPMG_ERROR_FATAL;
-    if (np > 0) {
-        hipLaunchKernelGGL(k_scatter<int>, dim3(nblk(np, 1024)), dim3(256), 0, s, plan->key.as<int>(),
-                           plan->slot.as<int>(), lhbx, np, lpdx);
-        hipLaunchKernelGGL(k_stabilize, dim3(nblk(ncells, 256)), dim3(256), 0, s, lhbx, ncells, lpdx);
-        hipLaunchKernelGGL(k_to_one_based, dim3(nblk(inside, 256)), dim3(256), 0, s, lpdx, inside);
+    if (radix) {
+        const int* ks = nullptr;
+        if (radix_sort(plan, plan->key.as<int>(), np, ncells + 1, lpdx, 1, inside, s, &ks)) return PPMG_ERROR_FATAL;
+        hipLaunchKernelGGL(k_heads, dim3(nblk(ncells, HEADS_CELLS)), dim3(256), 0, s, ks, np, ncells, lhbx, 1, 1,
+                           (int*)nullptr);
+    } else {
+        if (exclusive_scan(plan->count.as<int>(), ncells, lhbx, plan->scan_tmp, inside, s)) return PPMG_ERROR_FATAL;
+        if (np > 0) {
+            hipLaunchKernelGGL(k_scatter<int>, dim3(nblk(np, 1024)), dim3(256), 0, s, plan->key.as<int>(),
+                               plan->slot.as<int>(), lhbx, np, lpdx);
+            hipLaunchKernelGGL(k_stabilize, dim3(nblk(ncells, 256)), dim3(256), 0, s, lhbx, ncells, lpdx);
+            hipLaunchKernelGGL(k_to_one_based, dim3(nblk(inside, 256)), dim3(256), 0, s, lpdx, inside);
+        }
+        hipLaunchKernelGGL(k_to_one_based, dim3(nblk(ncells + 1, 256)), dim3(256), 0, s, lhbx, ncells + 1);
     }
-    hipLaunchKernelGGL(k_to_one_based, dim3(nblk(ncells + 1, 256)), dim3(256), 0, s, lhbx, ncells + 1);
     PPMG_HIP(hipGetLastError());
     // the binning's keys were overwritten: recomputed from its positions when read
     plan->keys_written = false;
