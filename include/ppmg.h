@@ -110,6 +110,9 @@ typedef struct ppmg_plan ppmg_plan;   /* device scratch + the forward sort (opaq
 /* ------------------------------------------------------------ plans -- */
 int ppmg_plan_create(ppmg_plan** plan);
 int ppmg_plan_destroy(ppmg_plan* plan);
+/* Device scratch the plan holds (its buffers grow with the largest call and
+ * are kept until the plan is destroyed). */
+int ppmg_plan_scratch_bytes(const ppmg_plan* plan, int64_t* bytes);
 
 /* ------------------------------------------------------------- core -- */
 /* P2M: replaces ppm_interp_p2m_{s,d}{s,v}_{2d,3d} (ppm_interp_p2m.f:127-162,

@@ -74,6 +74,12 @@ class Plan:
     def handle(self):
         return self._p
 
+    def scratch_bytes(self):
+        """Device scratch the plan holds."""
+        n = ctypes.c_int64()
+        check(lib().ppmg_plan_scratch_bytes(self._p, ctypes.byref(n)))
+        return n.value
+
     def set_timing(self, on=True):
         check(lib().ppmg_plan_set_timing(self._p, int(on)))
 

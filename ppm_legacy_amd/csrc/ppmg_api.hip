@@ -176,6 +176,15 @@ static int check_plan(ppmg_plan* plan) {
     return 0;
 }
 
+// Every device buffer of a plan.
+template <typename F>
+static void plan_buffers(ppmg_plan* plan, F f) {
+    DevBuf* bufs[] = {&plan->key, &plan->slot, &plan->count, &plan->start, &plan->perm, &plan->wsorted,
+                      &plan->usorted, &plan->scan_tmp, &plan->err, &plan->misc, &plan->misc2, &plan->gaps, &plan->multi, &plan->multi_n, &plan->ghost,
+                      &plan->table, &plan->rhist, &plan->work, &plan->work_cnt, &plan->rkey[0], &plan->rkey[1], &plan->rval[0], &plan->rval[1]};
+    for (DevBuf* b : bufs) f(*b);
+}
+
 }  // namespace ppmg
 
 using namespace ppmg;
@@ -213,13 +222,19 @@ int ppmg_plan_create(ppmg_plan** plan) {
 
 int ppmg_plan_destroy(ppmg_plan* plan) {
     if (!plan) return 0;
-    DevBuf* bufs[] = {&plan->key, &plan->slot, &plan->count, &plan->start, &plan->perm, &plan->wsorted,
-                      &plan->usorted, &plan->scan_tmp, &plan->err, &plan->misc, &plan->misc2, &plan->gaps, &plan->multi, &plan->multi_n, &plan->ghost,
-                      &plan->table, &plan->rhist, &plan->work, &plan->work_cnt, &plan->rkey[0], &plan->rkey[1], &plan->rval[0], &plan->rval[1]};
-    for (DevBuf* b : bufs) b->release();
+    plan_buffers(plan, [](DevBuf& b) { b.release(); });
+    host_slot_release(plan->host);
     if (plan->ev_init)
         for (auto& e : plan->ev) (void)hipEventDestroy(e);
     delete plan;
+    return 0;
+}
+
+int ppmg_plan_scratch_bytes(const ppmg_plan* plan, int64_t* bytes) {
+    if (!plan || !bytes) return fail(PPMG_ERROR_ERROR, PPMG_ERR_ARGUMENT, "plan or bytes is NULL");
+    int64_t n = 0;
+    plan_buffers(const_cast<ppmg_plan*>(plan), [&](DevBuf& b) { n += (int64_t)b.bytes; });
+    *bytes = n;
     return 0;
 }
 
@@ -377,7 +392,6 @@ int ppmg_m2p(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, const void
     const bool prebinned = plan->prebinned && plan->prebin_xp == xp && plan->prebin_np == np &&
                            plan->prebin_prec == prec && same_mesh(plan->prebin_mesh, m);
     plan->prebinned = false;
-    if (plan->err.ensure(sizeof(int) * 4) || fill_zero(plan->err.p, sizeof(int) * 4, s)) return g_status.info;
     mark(plan, s, true);
     const char* gen = std::getenv("PPMG_GENERAL");
     const bool force_general = gen && gen[0] && gen[0] != '0';
@@ -394,12 +408,11 @@ int ppmg_m2p(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, const void
         }
     }
     // the binning of the tiled path counts particles outside the sub in err[0]: start from zero
-    if (fill_zero(plan->err.p, sizeof(int) * 4, s)) return g_status.info;
+    if (plan->err.ensure(sizeof(int) * 4) || fill_zero(plan->err.p, sizeof(int) * 4, s)) return g_status.info;
     if (m2p_general(m, kernel, prec, np, xp, lda, fg, field->data, up, plan->err.as<int>(), s)) return g_status.info;
     mark(plan, s);
     int bad = 0;
-    PPMG_HIP(hipMemcpyAsync(&bad, plan->err.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, plan->err.as<int>(), 1, &bad, s)) return g_status.info;
     if (bad)
         return fail(PPMG_ERROR_ERROR, PPMG_ERR_FIELD_BOUNDS,
                     std::to_string(bad) + " particles read nodes outside the stored field");

@@ -467,6 +467,12 @@ struct ppmg_plan {
     int64_t prebin_np = 0, prebin_nbad = 0;
     int prebin_prec = 0;
     ppmg::DevMesh prebin_mesh{};
+    // pinned host words of read_back (ppmg_readback.hip) and its last ticket
+    uint32_t* host = nullptr;
+    uint32_t* host_dev = nullptr;
+    uint32_t ticket = 0;
+    bool host_tried = false;
+    bool lattice_flag_clear = false;   // err[6] (a lattice check's mismatch) is known to be zero
     int dim = 0, kernel = 0, prec = 0;
     ppmg::DevMesh mesh{};
     bool have_forward = false;
@@ -479,6 +485,12 @@ struct ppmg_plan {
 };
 
 namespace ppmg {
+// n device words, as the stream's work so far leaves them (waits for it);
+// pinned host slots of the plans.
+int read_back(ppmg_plan* plan, const int* src, int n, int* out, hipStream_t s);
+uint32_t* host_slot_acquire();
+void host_slot_release(uint32_t* slot);
+
 // Phase boundary marker of a timed plan (no-op unless timing is on).
 inline void mark(ppmg_plan* plan, hipStream_t s, bool first = false) {
     if (!plan || !plan->timing) return;

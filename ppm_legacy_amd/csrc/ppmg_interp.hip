@@ -653,6 +653,7 @@ static int adjoint_typed(ppmg_plan* plan, const DevMesh& m, int kernel, int64_t 
     const int KS = kernel == PPMG_KERNEL_MP4 ? 4 : 2;
     if (np <= 0) return 0;
     unsigned gr = nblk(np, 256);
+    plan->bin_xp = xp;   // the forward's positions, wherever they are held now
     if (materialize_perm(plan, s) || materialize_keys(plan, s)) return PPMG_ERROR_FATAL;
     const int* perm = plan->perm.as<int>();
     const int* key = plan->key.as<int>();
@@ -743,13 +744,12 @@ static int create_part_typed(ppmg_plan* plan, const DevMesh& m, const FieldGeom&
     PPMG_HIP(hipGetLastError());
     if (exclusive_scan(count, nb + 1, offs, plan->scan_tmp, 0, s)) return PPMG_ERROR_FATAL;
     int total = 0;
-    PPMG_HIP(hipMemcpyAsync(&total, offs + nb, sizeof(int), hipMemcpyDeviceToHost, s));
     if (a.maxnp > 0) CP_LDA(CP_WRITE);   // maxnp 0: the caller asks for the count only
 #undef CP_LDA
 #undef CP_WRITE
 #undef CP_MASK
     PPMG_HIP(hipGetLastError());
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, offs + nb, 1, &total, s)) return PPMG_ERROR_FATAL;
     *np_out = total;
     return 0;
 }

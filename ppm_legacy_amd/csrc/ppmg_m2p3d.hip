@@ -469,17 +469,16 @@ int m2p3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t 
 #undef TYPED
     };
     if (!plan->bin_lattice) return gather();
-    int* lat_err = plan->err.as<int>() + 6;
-    if (fill_zero(lat_err, sizeof(int), s)) return PPMG_ERROR_FATAL;
+    // (the binning cleared the mismatch flag)
     if (gather()) return PPMG_ERROR_FATAL;
     int off = 0;
-    PPMG_HIP(hipMemcpyAsync(&off, lat_err, sizeof(int), hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, plan->err.as<int>() + 6, 1, &off, s)) return PPMG_ERROR_FATAL;
     if (!off) {
         plan->lattice_checked = true;   // the plan's binning is the lattice (heads written on demand)
         return 0;
     }
     // not that lattice: bin and gather again (and bin the next 16 inputs)
+    plan->lattice_flag_clear = false;
     plan->lattice_pred = false;
     plan->lattice_skip = 16;
     if (bin_particles(plan, m, prec, np, xp, s, &nbad, periodic, false)) return PPMG_ERROR_FATAL;

@@ -23,14 +23,19 @@ static int g_next_topo = 1;
 static bool g_initialized = false;
 static int g_prec_mode = PPMG_PREC_F64;
 
-// Per-thread staging buffers and plan of the registry layer.
+// Per-thread staging buffers and plans of the registry layer.  M2P has a plan
+// of its own: a client's P2M and M2P bin particles in different orders
+// (advected ones, and often a fresh lattice), and one plan's predictions for
+// the one are wrong for the other (64^3: 90 us of a second binning per pass).
 struct Staging {
     ppmg_plan* plan = nullptr;
+    ppmg_plan* m2p_plan = nullptr;
     DevBuf xp, up, field, w[3], conv_up, conv_field, lp, lh;
     ~Staging() {
         DevBuf* b[] = {&xp, &up, &field, &w[0], &w[1], &w[2], &conv_up, &conv_field, &lp, &lh};
         for (DevBuf* x : b) x->release();
         if (plan) ppmg_plan_destroy(plan);
+        if (m2p_plan) ppmg_plan_destroy(m2p_plan);
     }
 };
 static thread_local Staging g_stage;
@@ -55,6 +60,11 @@ static int lookup(int topo_id, int mesh_id, Topo* out) {
 static ppmg_plan* stage_plan() {
     if (!g_stage.plan) ppmg_plan_create(&g_stage.plan);
     return g_stage.plan;
+}
+
+static ppmg_plan* stage_m2p_plan() {
+    if (!g_stage.m2p_plan) ppmg_plan_create(&g_stage.m2p_plan);
+    return g_stage.m2p_plan;
 }
 
 // Host arrays are copied to device scratch; device arrays pass through.
@@ -336,7 +346,7 @@ int ppmg_interp_m2p(const void* xp, int np, void* up, int lda, int topo_id, int 
     const size_t esz = single ? 4 : 8;
     ppmg_field f = padded_field(t, lda, g, nullptr);
     int64_t fcount = field_count(f);
-    ppmg_plan* plan = stage_plan();
+    ppmg_plan* plan = stage_m2p_plan();
     if (!plan) return current_info();
     const void *dxp = nullptr, *dfield = nullptr;
     void* dup = nullptr;

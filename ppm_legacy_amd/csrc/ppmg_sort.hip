@@ -648,23 +648,25 @@ __global__ void k_to_one_based(int* __restrict__ a, int64_t n) {
     if (i < n) a[i] += 1;
 }
 
-__global__ void k_fill_zero(uint32_t* __restrict__ p, int64_t n) {
+// Two ranges (the second may be empty) in one launch.
+__global__ void k_fill_zero(uint32_t* __restrict__ p, int64_t n, uint32_t* __restrict__ p2, int64_t n2) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) p[i] = 0u;
+    for (; i < n + n2; i += stride) (i < n ? p[i] : p2[i - n]) = 0u;
 }
 
 
 // Zero fill with a kernel (graph-capture safe, unlike hipMemsetAsync).
-int fill_zero(void* p, size_t bytes, hipStream_t s) {
-    int64_t n = (int64_t)(bytes / 4);
-    if (n <= 0) return 0;
-    int64_t g = (n + 255) / 256;
+static int fill_zero2(void* p, size_t bytes, void* p2, size_t bytes2, hipStream_t s) {
+    const int64_t n = (int64_t)(bytes / 4), n2 = (int64_t)(bytes2 / 4);
+    if (n + n2 <= 0) return 0;
+    int64_t g = (n + n2 + 255) / 256;
     if (g > 65536) g = 65536;
-    hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)g), dim3(256), 0, s, (uint32_t*)p, n);
+    hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)g), dim3(256), 0, s, (uint32_t*)p, n, (uint32_t*)p2, n2);
     PPMG_HIP(hipGetLastError());
     return 0;
 }
+int fill_zero(void* p, size_t bytes, hipStream_t s) { return fill_zero2(p, bytes, nullptr, 0, s); }
 
 // Keys of a binning that took the cell-order path (which writes none).
 template <int DIM, typename PosT>
@@ -990,8 +992,7 @@ static int heads_from_sorted(ppmg_plan* plan, const int* ks, int64_t np, int64_t
     hipLaunchKernelGGL(k_heads, dim3(g), dim3(256), 0, s, ks, np, ncells, plan->start.as<int>(), 0, stride, err);
     PPMG_HIP(hipGetLastError());
     int sample[128];
-    PPMG_HIP(hipMemcpyAsync(sample, err + 8, sizeof(sample), hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, err + 8, 128, sample, s)) return PPMG_ERROR_FATAL;
     int64_t crowd = 0, far = 0;
     for (int i = 0; i < 64; ++i) {
         crowd += sample[i];
@@ -1020,8 +1021,7 @@ static int bin_crowded(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, 
     }
     PPMG_HIP(hipGetLastError());
     int herr[2] = {0, 0};
-    PPMG_HIP(hipMemcpyAsync(herr, err, sizeof(herr), hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, err, 2, herr, s)) return PPMG_ERROR_FATAL;
     *nbad = herr[0];
     if (herr[0]) return 0;
     // input already in cell order: the keys are the sorted keys, the
@@ -1045,6 +1045,7 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     // byte-wide counts (count_word) come in whole blocks of 256 cells, and
     // the scan reads whole tiles of SCAN_TILE cells
     const size_t count_alloc = ((size_t)ncells + SCAN_TILE - 1) / SCAN_TILE * SCAN_TILE;
+    if (plan->err.bytes < sizeof(int) * ERR_WORDS) plan->lattice_flag_clear = false;   // about to be allocated
     if (plan->key.ensure(sizeof(int) * npb) || plan->slot.ensure(npb + 16) ||
         plan->perm.ensure(sizeof(int) * npb) || plan->count.ensure(count_alloc) ||
         plan->start.ensure(sizeof(int) * (size_t)(ncells + 1)) ||
@@ -1070,7 +1071,6 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
         plan->perm_written = true;
         return fill_zero(plan->start.p, sizeof(int) * (size_t)(ncells + 1), s);
     }
-    if (fill_zero(plan->err.p, sizeof(int) * ERR_WORDS, s)) return PPMG_ERROR_FATAL;
     // A lattice in cell order (particle p in cell p, np == ncells), as the last
     // binning of this plan found on the same mesh: for a reader that checks
     // every particle's cell itself (`lattice`), no pass at all; the reader
@@ -1082,6 +1082,8 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     }
     if (lattice && plan->lattice_pred && np == ncells && plan->lattice_prec == prec &&
         same_mesh(plan->lattice_mesh, m)) {
+        if (!plan->lattice_flag_clear && fill_zero(plan->err.p, sizeof(int) * ERR_WORDS, s)) return PPMG_ERROR_FATAL;
+        plan->lattice_flag_clear = true;
         plan->bin_lattice = true;
         plan->perm_identity = true;
         plan->perm_written = false;
@@ -1113,10 +1115,16 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     const bool radix = rx && rx[0] ? rx[0] == '1'
                                    : plan->crowded_cells * 64 > np ||
                                          (np >= FAR_MIN_NP && plan->far_particles * 4 > np);
-    if (!predict_sorted && radix && !arena_bound()) return bin_crowded(plan, m, prec, np, xp, s, nbad);
+    if (!predict_sorted && radix && !arena_bound()) {
+        if (fill_zero(plan->err.p, sizeof(int) * ERR_WORDS, s)) return PPMG_ERROR_FATAL;
+        plan->lattice_flag_clear = true;
+        return bin_crowded(plan, m, prec, np, xp, s, nbad);
+    }
     if (use_table && plan->table.ensure(sizeof(int) * TABLE_SLOTS * (size_t)ncells)) return PPMG_ERROR_FATAL;
     int* tab = use_table ? plan->table.as<int>() : nullptr;
-    if (!predict_sorted && fill_zero(plan->count.p, count_alloc, s)) return PPMG_ERROR_FATAL;
+    if (fill_zero2(plan->err.p, sizeof(int) * ERR_WORDS, plan->count.p, predict_sorted ? 0 : count_alloc, s))
+        return PPMG_ERROR_FATAL;
+    plan->lattice_flag_clear = true;
     int* key = plan->key.as<int>();
     uint8_t* slot8 = plan->slot.as<uint8_t>();
     uint32_t* count8 = plan->count.as<uint32_t>();
@@ -1148,8 +1156,7 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
         PPMG_HIP(hipGetLastError());
     }
     int herr[ERR_WORDS] = {};
-    PPMG_HIP(hipMemcpyAsync(herr, plan->err.p, sizeof(int) * ERR_WORDS, hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, err, ERR_WORDS, herr, s)) return PPMG_ERROR_FATAL;
     *nbad = herr[0];
     int64_t crowd = 0, far = 0;
     for (int i = 8; i < 72; ++i) {
@@ -1370,8 +1377,7 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
         PPMG_HIP(hipGetLastError());
     }
     int stats[2] = {0, 0};
-    PPMG_HIP(hipMemcpyAsync(stats, plan->err.p, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, plan->err.as<int>(), 2, stats, s)) return PPMG_ERROR_FATAL;
     int64_t inside = np - stats[0];
     if (radix) {
         const int* ks = nullptr;

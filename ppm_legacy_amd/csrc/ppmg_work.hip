@@ -153,8 +153,7 @@ int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, hipStream
                        plan->work.as<int4>());
     PPMG_HIP(hipGetLastError());
     int total = 0;
-    PPMG_HIP(hipMemcpyAsync(&total, offs + ncnt - 1, sizeof(int), hipMemcpyDeviceToHost, s));
-    PPMG_HIP(hipStreamSynchronize(s));
+    if (read_back(plan, offs + ncnt - 1, 1, &total, s)) return PPMG_ERROR_FATAL;
     *items = plan->work.as<int4>();
     *nitems = (unsigned)total;
     return 0;
