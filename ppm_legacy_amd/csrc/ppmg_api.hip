@@ -477,7 +477,7 @@ int ppmg_p2m_adjoint(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, co
     if (!force_general && adjoint3d_fast_applicable(m, kernel, fg)) {
         if (adjoint3d_fast(plan, m, prec, np, xp, lda, up, fg, g->data, grad_up, grad_xp, as_stream(stream)))
             return g_status.info;
-    } else if (adjoint_general(plan, m, kernel, prec, np, xp, lda, up, fg, g->data, grad_up, grad_xp,
+    } else if (adjoint_general(plan, m, kernel, prec, np, xp, lda, up, fg, g->data, grad_up, grad_xp, force_general,
                                as_stream(stream))) {
         return g_status.info;
     }

@@ -9,8 +9,11 @@ int p2m_general(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t
                 const void* up, const FieldGeom& fg, void* field, const void* const* wtab, hipStream_t s);
 int m2p_general(const DevMesh& m, int kernel, int prec, int64_t np, const void* xp, int lda, const FieldGeom& fg,
                 const void* field, void* up, int* err, hipStream_t s);
+// reference: every particle through the image search (used to cross-check the
+// specialised kernels)
 int adjoint_general(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp, int lda,
-                    const void* up, const FieldGeom& fg, const void* g, void* gu, void* gx, hipStream_t s);
+                    const void* up, const FieldGeom& fg, const void* g, void* gu, void* gx, bool reference,
+                    hipStream_t s);
 int comp_weights_general(const DevMesh& m, int kernel, int prec, int64_t np, const void* xp, void* w1, void* w2,
                          void* w3, hipStream_t s);
 int impose_bc_general(const DevMesh& m, int prec, int64_t np, void* xp, hipStream_t s);
