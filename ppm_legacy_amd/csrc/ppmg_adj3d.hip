@@ -87,7 +87,7 @@ template <int LDA, typename PosT, typename ValT, typename AccT, bool BOXED, bool
 __global__ void __launch_bounds__(A3_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
 k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ up, const ValT* __restrict__ g, FieldGeom fg,
-          ValT* __restrict__ grad_u, ValT* __restrict__ grad_x, int lda, int c0, int tz, const int4* __restrict__ items,
+          ValT* __restrict__ grad_u, ValT* __restrict__ grad_x, int lda, int c0, int tz, WorkList items,
           int accumulate_x) {
     __shared__ ValT ring[4 * LDA * A3_PL];   // [plane][c][ry][nx]
     const int tid = threadIdx.x;
@@ -388,11 +388,10 @@ static int launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, con
     // a step is long here: a chunk's three extra plane loads weigh little
     const int tz = pick_chunk((int64_t)tx * ty, m.N[2], res, 0.3, 0.3);
     unsigned grid = (unsigned)((int64_t)tx * ty * ((m.N[2] + tz - 1) / tz));
-    const int4* items = nullptr;   // crowded cells: workgroups from a work list
-    if (!TABLE && work_list_applies(plan)) {
-        const int rc = build_work(plan, m, {tx, ty, A3_TX, A3_TY, 0, 0, A3_TX, A3_TY, m.N[2]}, s, &items, &grid);
-        if (rc < 0) return rc;
-    }
+    WorkList items;   // crowded cells: workgroups from a work list
+    if (!TABLE && work_list_applies(plan, tz) &&
+        build_work(plan, m, {tx, ty, A3_TX, A3_TY, 0, 0, A3_TX, A3_TY, m.N[2], 0}, res.slots(), s, &items, &grid))
+        return PPMG_ERROR_FATAL;
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
     hipLaunchKernelGGL((k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>), dim3(grid), dim3(A3_THREADS), 0, s, m,
                        plan->start.as<int>(), tile_perm(plan), bt, xp, up, g, fg, gu, gx, lda, c0, tz, items, acc);

@@ -74,7 +74,7 @@ template <int KS, int LDA, typename PosT, typename ValT, typename AccT, int WPE,
 __global__ void __launch_bounds__(M3_THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ field, FieldGeom fg, ValT* __restrict__ up, int lda,
-          int c0, int tz, const int4* __restrict__ items, int* __restrict__ lat_err) {
+          int c0, int tz, WorkList items, int* __restrict__ lat_err) {
     static_assert(!(TABLE && LAT), "one binning form");
     constexpr int B = M3Geom<KS>::B, M3_TX = M3Geom<KS>::TX, M3_PL = M3Geom<KS>::PL;
     constexpr int RP = KS;                   // ring planes
@@ -383,11 +383,10 @@ static int launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, con
     unsigned grid = (unsigned)((int64_t)tx * ty * ((m.nbin[2] + tz - 1) / tz));
     // crowded cells: the workgroups come from a work list (clustered 512^3,
     // FP64, lda 3: 7.7 against 9.5 ms in 16-plane chunks)
-    const int4* items = nullptr;
-    if (!TABLE && !LAT && work_list_applies(plan)) {
-        const int rc = build_work(plan, m, {tx, ty, TX, M3_TY, 0, 0, TX, M3_TY, m.nbin[2]}, s, &items, &grid);
-        if (rc < 0) return rc;
-    }
+    WorkList items;
+    if (!TABLE && !LAT && work_list_applies(plan, tz) &&
+        build_work(plan, m, {tx, ty, TX, M3_TY, 0, 0, TX, M3_TY, m.nbin[2], 0}, res.slots(), s, &items, &grid))
+        return PPMG_ERROR_FATAL;
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(M3_THREADS), 0, s, m, plan->start.as<int>(),
                        tile_perm(plan), bt, xp, field, fg, up, fg.lda, c0, tz, items, plan->err.as<int>() + 6);

@@ -91,29 +91,47 @@ int sort_rows(int dim, int prec, int64_t np, void* xp, const int* lpdx1, const i
 // ------------------------------------------- work list (ppmg_work.hip) --
 // Tile columns of a 3D tile kernel: ntx x nty tiles of tx x ty, marching
 // `planes` planes; a tile's cells are the ncol x nrow ones starting at offset
-// (wx, wy) from its first.
+// (wx, wy) from its first.  halo: planes of particles a piece takes beyond its
+// own.
 struct TileWindow {
     int ntx, nty, tx, ty;
     int wx, wy, ncol, nrow;
-    int planes;
+    int planes, halo;
+};
+// Pieces of tile columns in WK_CLASSES classes, heaviest first: class k's lie
+// at items + k * cap and are workgroups end[k-1] .. end[k]-1; a piece is its
+// column and first plane * 64 + planes.
+constexpr int WK_CLASSES = 4;
+struct WorkList {
+    const int2* items = nullptr;
+    int64_t cap = 0;
+    unsigned end[WK_CLASSES] = {};
 };
 // The plan's last binning found crowded cells and left heads: launches take
-// their workgroups from a work list.
-bool work_list_applies(const ppmg_plan* plan);
-// Pieces (tile column, first plane, end plane) of all tile columns, heaviest
-// first, in the plan's scratch; 0, 1 (no list) or an error.
-int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, hipStream_t s, const int4** items,
+// their workgroups from a work list.  tz: the grid's chunk; single planes leave
+// nothing to cut (95 x 86 x 54, BSP2, half a particle a cell in blobs: deposit
+// 100 us, 144 with the list).
+bool work_list_applies(const ppmg_plan* plan, int tz);
+// The pieces of all tile columns, in the plan's scratch, and their number
+// (slots: resident workgroups of the kernel); the list stays empty where it
+// would take too much scratch.
+int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, int slots, hipStream_t s, WorkList* list,
                unsigned* nitems);
 // This workgroup's tile column and planes [z0, z1): from the work list, or
-// (items NULL) the grid's chunks of tz planes in XCD order.
-__device__ __forceinline__ void tile_piece(const int4* __restrict__ items, int ntx, int nty, int tz, int planes,
-                                           int& tx, int& ty, int& z0, int& z1) {
+// (no items) the grid's chunks of tz planes in XCD order.
+__device__ __forceinline__ void tile_piece(const WorkList& list, int ntx, int nty, int tz, int planes, int& tx,
+                                           int& ty, int& z0, int& z1) {
     int col;
-    if (items) {
-        const int4 it = items[blockIdx.x];
+    if (list.items) {
+        const unsigned b = blockIdx.x;
+        int64_t at = b;
+#pragma unroll
+        for (int k = 1; k < WK_CLASSES; ++k)
+            if (b >= list.end[k - 1]) at = k * list.cap + (b - list.end[k - 1]);
+        const int2 it = list.items[at];
         col = it.x;
-        z0 = it.y;
-        z1 = it.z;
+        z0 = it.y >> 6;
+        z1 = z0 + (it.y & 63);
     } else {
         const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
         const int64_t ncol = (int64_t)ntx * nty;
