@@ -208,9 +208,22 @@ __device__ __forceinline__ float row_shl(float v) {
 }
 
 // Value of lane ex + D of the same 16-lane row (D > 0: row_shl, D < 0: row_shr).
-template <int D, typename T>
+// W = 32: rows of 32 lanes, by whole-wavefront shifts of one lane (a lane at a
+// row's end reads the other row's, where a 16-lane row reads 0).
+template <int CTRL> __device__ __forceinline__ double wave_shift(double v) {
+    int lo = __double2loint(v), hi = __double2hiint(v);
+    lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, true);
+    hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+template <int CTRL> __device__ __forceinline__ float wave_shift(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int D, int W = 16, typename T>
 __device__ __forceinline__ T lane_from(T v) {
-    if constexpr (D > 0) return row_shl<D>(v);
+    if constexpr (W == 32 && D > 0) return lane_from<D - 1, W>(wave_shift<0x130>(v));
+    else if constexpr (W == 32 && D < 0) return lane_from<D + 1, W>(wave_shift<0x138>(v));
+    else if constexpr (D > 0) return row_shl<D>(v);
     else if constexpr (D < 0) return row_shr<-D>(v);
     else return v;
 }

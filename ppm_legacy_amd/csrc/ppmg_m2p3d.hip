@@ -7,18 +7,19 @@
 // (ghost_get) is the node map of the planes loaded around the tile
 // (stored_node).
 //
-// A workgroup (4 wavefronts, 16 rows of 16 lanes) owns the particles of a
-// 13 x 16 cell tile in x,y over 32 cell planes in z.  The 16 x 19 nodes those
-// cells read are kept for 4 node planes in an LDS ring (component-major, rows
-// of 16 nodes): cell plane cz reads node planes cz-1 .. cz+2, after which
-// plane cz-1 is replaced by plane cz+3, loaded with coalesced reads.
+// A workgroup (4 wavefronts, 16 rows of 16 lanes or 8 of 32) owns the
+// particles of a 13 x 16 or 29 x 8 cell tile in x,y over a chunk of cell planes
+// in z.  The nodes those cells read (three more rows, 16 or 32 to a row) are
+// kept for 4 node planes in an LDS ring (component-major): cell plane
+// cz reads node planes cz-1 .. cz+2, after which plane cz-1 is replaced by
+// plane cz+3, loaded with coalesced reads.
 //
 // Lane mapping: lane ex of row `row` stands for node column tx0-1+ex and for
-// cell (tx0+ex-1, ty0+row); lanes 1..13 carry the particles of their cell, one
+// cell (tx0+ex-1, ty0+row); lanes 1..13 (1..29) carry the particles of their cell, one
 // particle per round (particles are binned, so a cell's particles are
 // contiguous in the permutation).  Instead of every particle reading its
 // 4x4x4 stencil (192 scattered LDS reads for lda = 3), every lane reads ONE
-// 4x4 (y,z) column of its node column -- 16 lanes read 16 consecutive words,
+// 4x4 (y,z) column of its node column -- a row's lanes read consecutive words,
 // free of bank conflicts -- and contracts it with the (y,z) weights of the
 // four particles whose x-stencil covers that column; those weights come from
 // lanes ex+1, ex, ex-1, ex-2 by DPP row shifts, and the four partial sums go
@@ -35,18 +36,19 @@
 
 namespace ppmg {
 
-constexpr int M3_TY = 16;               // owned cell rows per tile (one 16-lane row each)
-constexpr int M3_THREADS = 16 * M3_TY;  // 256
+constexpr int M3_THREADS = 256;
 
 // Tile geometry for a stencil of KS nodes per axis (4: M'4, 2: BSP2): a
 // particle of cell c reads nodes c - B .. c - B + KS - 1.  Lane ex of a row
 // stands for node column tx0 - B + ex; the cells of lanes B .. B + TX - 1
 // carry particles.  The ring holds KS node planes of RY rows of 16 nodes.
-template <int KS> struct M3Geom {
+// W: lanes per row (16 or 32).
+template <int KS, int W> struct M3Geom {
     static constexpr int B = KS == 4 ? 1 : 0;
-    static constexpr int TX = 17 - KS;            // owned cells per tile along x (13 or 15)
-    static constexpr int RY = M3_TY + KS - 1;     // node rows in the ring
-    static constexpr int PL = RY * 16;            // node slots per ring plane and component
+    static constexpr int TX = W + 1 - KS;         // owned cells per tile along x
+    static constexpr int TY = M3_THREADS / W;     // owned cell rows per tile
+    static constexpr int RY = TY + KS - 1;        // node rows in the ring
+    static constexpr int PL = RY * W;             // node slots per ring plane and component
 };
 
 // Stored node read as stored: v itself on a stored box (clamped into it for
@@ -60,7 +62,7 @@ __device__ __forceinline__ int raw_node(const DevMesh& m, const FieldGeom& fg, i
 // WPE: minimum wavefronts per SIMD the register allocation must allow: 4 (at
 // most 128 VGPRs) where that needs no spills, else 3 (M'4 with four
 // components or the MIX form).  At 512^3, lda 3, FP64 the gather takes 2.94 ms
-// with 4 wavefronts against 3.18 ms with 3 (136 VGPRs unconstrained).
+// with 4 wavefronts against 3.18 ms with 3 (136 VGPRs unconstrained), in 16-lane rows.
 // MIX: some open axis beside a periodic axis stored as a box, where whether a
 // node takes the periodic node map depends on all three of its coordinates.
 // TABLE: the binning is a slot table (byte counts, particle r of cell c at
@@ -69,18 +71,19 @@ __device__ __forceinline__ int raw_node(const DevMesh& m, const FieldGeom& fg, i
 // c, one per cell) without having been computed: every particle's cell key
 // is checked against its cell, and a mismatch sets *lat_err (the caller then
 // bins and gathers again).
-template <int KS, int LDA, typename PosT, typename ValT, typename AccT, int WPE, bool OPEN, bool MIX, bool TABLE,
+template <int KS, int W, int LDA, typename PosT, typename ValT, typename AccT, int WPE, bool OPEN, bool MIX, bool TABLE,
           bool LAT>
 __global__ void __launch_bounds__(M3_THREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ field, FieldGeom fg, ValT* __restrict__ up, int lda,
           int c0, int tz, WorkList items, int* __restrict__ lat_err) {
     static_assert(!(TABLE && LAT), "one binning form");
-    constexpr int B = M3Geom<KS>::B, M3_TX = M3Geom<KS>::TX, M3_PL = M3Geom<KS>::PL;
+    using G = M3Geom<KS, W>;
+    constexpr int B = G::B, M3_TX = G::TX, M3_TY = G::TY, M3_PL = G::PL;
     constexpr int RP = KS;                   // ring planes
     __shared__ ValT ring[RP * LDA * M3_PL];  // [plane][c][ry][nx]
     const int tid = threadIdx.x;
-    const int ex = tid & 15, row = tid >> 4;
+    const int ex = tid & (W - 1), row = tid / W;
     // tiles cover the cells: N per periodic axis, N+1 (0..N) per open one
     const int Nx = m.nbin[0], Ny = m.nbin[1], Nz = m.nbin[2];
     const int ntx = (Nx + M3_TX - 1) / M3_TX, nty = (Ny + M3_TY - 1) / M3_TY;
@@ -105,7 +108,7 @@ k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 #pragma unroll
     for (int j = 0; j < NN; ++j) {
         const int node = tid + j * M3_THREADS;
-        const int nx = node & 15, ry = node >> 4;
+        const int nx = node & (W - 1), ry = node / W;
         const int gx = stored_node<OPEN>(m, fg, 0, tx0 - B + nx) - fg.lo[0];
         const int gy = stored_node<OPEN>(m, fg, 1, ty0 - B + ry) - fg.lo[1];
         soff[j] = (unsigned)(((gy * fg.ext[0] + gx) * lda + c0) * (int)sizeof(ValT));
@@ -114,7 +117,7 @@ k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     }
     // MIX: byte offset of node `node` of a plane read as stored
     auto raw_off = [&](int node) -> unsigned {
-        const int nx = node & 15, ry = node >> 4;
+        const int nx = node & (W - 1), ry = node / W;
         const int gx = raw_node<OPEN>(m, fg, 0, tx0 - B + nx) - fg.lo[0];
         const int gy = raw_node<OPEN>(m, fg, 1, ty0 - B + ry) - fg.lo[1];
         return (unsigned)(((gy * fg.ext[0] + gx) * lda + c0) * (int)sizeof(ValT));
@@ -264,11 +267,12 @@ k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
             AccT a[KS][KS], b[KS][KS];
 #pragma unroll
             for (int o = 0; o < KS; ++o) {
-                a[0][o] = lane_from<B>(wy[o]);     b[0][o] = lane_from<B>(wz[o]);
-                a[1][o] = lane_from<B - 1>(wy[o]); b[1][o] = lane_from<B - 1>(wz[o]);
+                a[0][o] = lane_from<B, W>(wy[o]);     b[0][o] = lane_from<B, W>(wz[o]);
+                a[1][o] = lane_from<B - 1, W>(wy[o]); b[1][o] = lane_from<B - 1, W>(wz[o]);
                 if constexpr (KS == 4) {
-                    a[2][o] = lane_from<B - 2>(wy[o]); b[2][o] = lane_from<B - 2>(wz[o]);
-                    a[3][o] = lane_from<B - 3>(wy[o]); b[3][o] = lane_from<B - 3>(wz[o]);
+                    a[2][o] = lane_from<B - 2, W>(wy[o]); b[2][o] = lane_from<B - 2, W>(wz[o]);
+                    a[3][o] = W == 32 ? lane_from<-1, W>(a[2][o]) : lane_from<B - 3, W>(wy[o]);
+                    b[3][o] = W == 32 ? lane_from<-1, W>(b[2][o]) : lane_from<B - 3, W>(wz[o]);
                 }
             }
             // per component: column partial sums Ck = sum_oz b_k[oz] * sum_oy a_k[oy] f(oz, oy)
@@ -282,10 +286,10 @@ k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                 for (int k = 0; k < KS; ++k) C[k] = AccT(0);
 #pragma unroll
                 for (int oz = 0; oz < KS; ++oz) {
-                    const ValT* f = ring + ((cz - B + oz) & (RP - 1)) * (LDA * M3_PL) + c * M3_PL + row * 16 + ex;
+                    const ValT* f = ring + ((cz - B + oz) & (RP - 1)) * (LDA * M3_PL) + c * M3_PL + row * W + ex;
                     AccT fv[KS];
 #pragma unroll
-                    for (int oy = 0; oy < KS; ++oy) fv[oy] = (AccT)f[16 * oy];
+                    for (int oy = 0; oy < KS; ++oy) fv[oy] = (AccT)f[W * oy];
 #pragma unroll
                     for (int k = 0; k < KS; ++k) {
                         AccT t = a[k][0] * fv[0];
@@ -295,11 +299,11 @@ k_m3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                     }
                 }
                 // x offset k of this lane's particle is the column of lane ex - B + k
-                AccT u = wx[0] * lane_from<-B>(C[0]);
-                u += wx[1] * lane_from<1 - B>(C[1]);
+                AccT u = wx[0] * lane_from<-B, W>(C[0]);
+                u += wx[1] * lane_from<1 - B, W>(C[1]);
                 if constexpr (KS == 4) {
-                    u += wx[2] * lane_from<2 - B>(C[2]);
-                    u += wx[3] * lane_from<3 - B>(C[3]);
+                    u += wx[2] * lane_from<2 - B, W>(C[2]);
+                    u += wx[3] * lane_from<3 - B, W>(C[3]);
                 }
                 res[c] = (ValT)u;
                 // one component at a time: keeps the column reads of the next
@@ -367,14 +371,13 @@ bool m2p3d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg) {
 // field's layout).
 bool m2p3d_table_applicable(const DevMesh& m) { return m.dim == 3 && m.periodic[0] && m.periodic[1] && m.periodic[2]; }
 
-// One launch of the gather for components c0 .. c0+LL-1.
-template <int KS, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool MIX, bool TABLE = false,
-          bool LAT = false>
-static int launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
-                           const ValT* field, ValT* up, hipStream_t s) {
-    constexpr int TX = M3Geom<KS>::TX;
+// One launch of the gather for components c0 .. c0+LL-1, rows of W lanes.
+template <int KS, int W, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool MIX, bool TABLE, bool LAT>
+static int launch_m3_rows(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
+                          const ValT* field, ValT* up, hipStream_t s) {
+    constexpr int TX = M3Geom<KS, W>::TX, M3_TY = M3Geom<KS, W>::TY;
     constexpr int WPE = KS == 4 && (LL == 4 || MIX) ? 3 : 4;
-    auto kernel = k_m3_tile<KS, LL, PosT, ValT, AccT, WPE, OPEN, MIX, TABLE, LAT>;
+    auto kernel = k_m3_tile<KS, W, LL, PosT, ValT, AccT, WPE, OPEN, MIX, TABLE, LAT>;
     static const Residency res = residency(kernel, M3_THREADS);
     const int tx = (m.nbin[0] + TX - 1) / TX, ty = (m.nbin[1] + M3_TY - 1) / M3_TY;
     // a chunk loads KS - 1 more planes before its first step: a plane's worth
@@ -391,6 +394,25 @@ static int launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, con
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(M3_THREADS), 0, s, m, plan->start.as<int>(),
                        tile_perm(plan), bt, xp, field, fg, up, fg.lda, c0, tz, items, plan->err.as<int>() + 6);
     return 0;
+}
+
+// Rows of 32 or 16 lanes.  The M'4 gather is bound by its FP64 instructions
+// (92% of the issue slots at 512^3), and of a row all but three lanes carry
+// particles: 29 of 32 where the longer rows cover the mesh with fewer lanes,
+// else 13 of 16.  lda 3, lattice: 512^3 FP64 3.09 -> 2.89 ms, 256^3 FP32c
+// 374 -> 345 us.  (BSP2, 31 of 32 against 15 of 16, has too little to gain.)
+template <int KS, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool MIX, bool TABLE = false,
+          bool LAT = false>
+static int launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
+                          const ValT* field, ValT* up, hipStream_t s) {
+    if constexpr (KS == 4) {
+        const int n = m.nbin[0];
+        constexpr int T16 = M3Geom<KS, 16>::TX, T32 = M3Geom<KS, 32>::TX;
+        if ((n + T32 - 1) / T32 * 32 < (n + T16 - 1) / T16 * 16)
+            return launch_m3_rows<KS, 32, LL, PosT, ValT, AccT, OPEN, MIX, TABLE, LAT>(plan, m, xp, fg, c0, field, up,
+                                                                                      s);
+    }
+    return launch_m3_rows<KS, 16, LL, PosT, ValT, AccT, OPEN, MIX, TABLE, LAT>(plan, m, xp, fg, c0, field, up, s);
 }
 
 // OPEN: some axis is open (a fully periodic mesh compiles without the clamp);

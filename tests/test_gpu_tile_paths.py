@@ -113,3 +113,41 @@ def test_crowded_work_list(core, monkeypatch, shape, bc, kernel):
             assert torch.equal(a, b)
     for a, b in zip(first, _general(monkeypatch, run)):
         assert ((a - b).abs().max() / b.abs().max()).item() < 1e-12
+
+
+@pytest.mark.parametrize("nx", [27, 29, 55, 58])
+@pytest.mark.parametrize("bc", [[1] * 6, [1, 1, 1, 1, 2, 2], [2] * 6], ids=["periodic", "open_z", "open"])
+@pytest.mark.parametrize("parts", ["lattice", "random", "blob"])
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_gather_wide_rows(core, monkeypatch, nx, bc, parts, prec):
+    """Meshes whose M'4 gather takes rows of 32 lanes (29 cells to a tile), on
+    every binning form: bitwise the same on all three passes of a plan, and
+    against the general path (64 terms: 1e-13 of the maximum in FP64, FP32c
+    with FP64 sums of FP32 nodes 1e-6)."""
+    shape = (nx, 19, 10)
+    rng = np.random.default_rng(nx)
+    if parts == "lattice":
+        i = np.arange(nx * 19 * 10)
+        x = (np.stack([i % nx, (i // nx) % 19, i // (nx * 19)], 1) + rng.uniform(0.05, 0.95, (len(i), 3))) / shape
+    elif parts == "random":
+        x = rng.uniform(0, 0.999, (nx * 190, 3))
+    else:
+        x = np.concatenate([rng.normal(0.5, 0.04, (4000, 3)).clip(0.01, 0.99), rng.uniform(0, 0.999, (500, 3))])
+    side = np.array(shape) / nx
+    mesh = core.Mesh(3, [n + 1 for n in shape], [0.0] * 3, list(side), bc)
+    xd = torch.as_tensor(x * side).to(core.POS_DTYPE[prec]).cuda()
+    vdt = core.VAL_DTYPE[prec]
+    for lda in (1, 3, 4):
+        f = torch.as_tensor(rng.normal(size=mesh.padded_shape(lda, [2] * 3))).to(vdt).cuda()
+
+        def m2p(plan=None):
+            out = torch.empty((len(x), lda), dtype=vdt, device="cuda")
+            core.m2p(mesh, xd, f, [-2] * 3, out, MP4, prec, plan=plan)
+            return out
+
+        plan = core.Plan()
+        got = m2p(plan)
+        for _ in range(2):
+            assert torch.equal(got, m2p(plan))
+        ref = _general(monkeypatch, m2p)
+        assert ((got - ref).abs().max() / ref.abs().max()).item() < (1e-13 if prec == F64 else 1e-6)
