@@ -28,12 +28,16 @@ namespace ppmg {
 constexpr int M2_RING = 8;   // node rows in the ring
 
 // TABLE: the binning is a slot table (byte counts, particle r of cell c at
-// bt.table[r * ncells + c]) instead of heads and a permutation.
-template <int KS, int LDA, typename PosT, typename ValT, typename AccT, bool OPEN, bool TABLE>
+// bt.table[r * ncells + c]) instead of heads and a permutation.  LAT: the
+// binning is taken to be a lattice in cell order, not computed: every
+// particle's cell is checked and a mismatch sets *lat_err (gather_checked).
+// At 8192^2 the binning pass it saves took 256 us beside a gather of 1010.
+template <int KS, int LDA, typename PosT, typename ValT, typename AccT, bool OPEN, bool TABLE, bool LAT>
 __global__ void __launch_bounds__(64)
 k_m2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ field, FieldGeom fg, ValT* __restrict__ up, int lda,
-          int c0, int ty) {
+          int c0, int ty, int* __restrict__ lat_err) {
+    static_assert(!(TABLE && LAT), "one binning form");
     constexpr int B = Stencil<KS>::B, TX = 17 - KS;
     constexpr int ROWV = 16 * LDA;                 // values per ring row: [c][nx]
     __shared__ ValT ring[M2_RING * ROWV];
@@ -81,7 +85,10 @@ k_m2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
         const int cy = y0 + 4 * st + erow;
         if (plane_lane && st < nsteps && cy < y1) {
             const int key = cx + Nx * cy;
-            if constexpr (TABLE) {
+            if constexpr (LAT) {
+                f = key;
+                n = 1;
+            } else if constexpr (TABLE) {
                 f = key;
                 n = (int)bt.count[count_word(key)];   // decoded where used: the load stays in flight
                 t = bt.table[key];
@@ -92,15 +99,18 @@ k_m2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
         }
     };
     auto count_of = [&](int f, int n) {
-        if constexpr (TABLE) return (int)(((unsigned)n >> count_shift(f)) & 255u);
+        if constexpr (LAT) return n;
+        else if constexpr (TABLE) return (int)(((unsigned)n >> count_shift(f)) & 255u);
         else return n - f;
     };
     auto lookup = [&](int f, int n, int t) {
-        if constexpr (TABLE) return count_of(f, n) > 0 ? t : 0;
+        if constexpr (LAT) return f;
+        else if constexpr (TABLE) return count_of(f, n) > 0 ? t : 0;
         else return n > f ? (perm ? perm[f] : f) : 0;
     };
     auto entry = [&](int f, int r) {
-        if constexpr (TABLE) return bt.table[(int64_t)r * bt.ncells + f];
+        if constexpr (LAT) return f + r;
+        else if constexpr (TABLE) return bt.table[(int64_t)r * bt.ncells + f];
         else return perm ? perm[f + r] : f + r;
     };
     auto position = [&](int p, int n, PosT (&x)[2]) {
@@ -118,6 +128,7 @@ k_m2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     position(pn, count_of(first_n, cnt_n), xn);
     wave_lds_sync();
 
+    bool lat_bad = false;   // (LAT) a particle found outside the cell it was taken for
     for (int st = 0; st < nsteps; ++st) {
         const int first = first_n, cnt = count_of(first_n, cnt_n);
         asm volatile("" ::"v"(first), "v"(cnt) : "memory");
@@ -135,9 +146,19 @@ k_m2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 #pragma unroll
             for (int o = 0; o < KS; ++o) wx[o] = wy[o] = AccT(0);
             if (has) {
-                int ci;
-                tile_weights<KS, AccT>((AccT)cell_offset<PosT>(x[0], (PosT)m.minv[0], (PosT)m.dxi[0], ci), wx);
-                tile_weights<KS, AccT>((AccT)cell_offset<PosT>(x[1], (PosT)m.minv[1], (PosT)m.dxi[1], ci), wy);
+                int ci[2];
+                tile_weights<KS, AccT>((AccT)cell_offset<PosT>(x[0], (PosT)m.minv[0], (PosT)m.dxi[0], ci[0]), wx);
+                tile_weights<KS, AccT>((AccT)cell_offset<PosT>(x[1], (PosT)m.minv[1], (PosT)m.dxi[1], ci[1]), wy);
+                if constexpr (LAT) {
+                    // the cell key's test on a periodic mesh (as in the 3D gather)
+                    const int cell[2] = {cx, y0 + 4 * st + erow};
+                    bool in = true;
+#pragma unroll
+                    for (int d = 0; d < 2; ++d)
+                        in = in && x[d] >= (PosT)m.minv[d] && x[d] <= (PosT)m.maxv[d] &&
+                             (ci[d] == cell[d] || (ci[d] == m.N[d] && cell[d] == 0));
+                    lat_bad = lat_bad || !in;
+                }
             }
             // y weights of the particle whose stencil takes this lane's column as
             // x offset k: that of lane ex + B - k
@@ -193,6 +214,9 @@ k_m2_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
         if (more) store_row(4 * st + 8 + erow, stage);
         wave_lds_sync();
     }
+    if constexpr (LAT) {
+        if (__ballot(lat_bad) != 0ull && lane == 0) *lat_err = 1;
+    }
 }
 
 // Per periodic axis the compact layout or a stored box holding the whole real
@@ -219,18 +243,19 @@ bool m2p2d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg) {
     return true;
 }
 
-template <int KS, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool TABLE = false>
+template <int KS, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool TABLE = false,
+          bool LAT = false>
 static void launch_m2_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
                            const ValT* field, ValT* up, hipStream_t s) {
     constexpr int TX = 17 - KS;
     static std::atomic<int> slots{0};
-    if (slots.load() == 0) slots.store(resident_workgroups(k_m2_tile<KS, LL, PosT, ValT, AccT, OPEN, TABLE>, 64));
+    if (slots.load() == 0) slots.store(resident_workgroups(k_m2_tile<KS, LL, PosT, ValT, AccT, OPEN, TABLE, LAT>, 64));
     const int tx = (m.nbin[0] + TX - 1) / TX;
     const int ty = pick_z_chunk(tx, m.nbin[1], slots.load(), 0);
     dim3 grid((unsigned)((int64_t)tx * ((m.nbin[1] + ty - 1) / ty)));
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
-    hipLaunchKernelGGL((k_m2_tile<KS, LL, PosT, ValT, AccT, OPEN, TABLE>), grid, dim3(64), 0, s, m,
-                       plan->start.as<int>(), tile_perm(plan), bt, xp, field, fg, up, fg.lda, c0, ty);
+    hipLaunchKernelGGL((k_m2_tile<KS, LL, PosT, ValT, AccT, OPEN, TABLE, LAT>), grid, dim3(64), 0, s, m,
+                       plan->start.as<int>(), tile_perm(plan), bt, xp, field, fg, up, fg.lda, c0, ty, plan->err.as<int>() + 6);
 }
 
 template <int KS, typename PosT, typename ValT, typename AccT>
@@ -242,7 +267,8 @@ static int m2p2d_typed(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const 
         const int L = lda - c0 < 4 ? lda - c0 : 4;
 #define TL(LL)                                                                                   \
     do {                                                                                         \
-        if (plan->bin_table) launch_m2_open<KS, LL, PosT, ValT, AccT, false, true>(plan, m, xp, fg, c0, field, up, s); \
+        if (plan->bin_lattice) launch_m2_open<KS, LL, PosT, ValT, AccT, false, false, true>(plan, m, xp, fg, c0, field, up, s); \
+        else if (plan->bin_table) launch_m2_open<KS, LL, PosT, ValT, AccT, false, true>(plan, m, xp, fg, c0, field, up, s); \
         else if (open) launch_m2_open<KS, LL, PosT, ValT, AccT, true>(plan, m, xp, fg, c0, field, up, s);  \
         else launch_m2_open<KS, LL, PosT, ValT, AccT, false>(plan, m, xp, fg, c0, field, up, s);      \
     } while (0)
@@ -262,11 +288,13 @@ static int m2p2d_typed(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const 
 int m2p2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp,
                const FieldGeom& fg, const void* field, void* up, hipStream_t s) {
     int64_t nbad = 0;
-    // a slot table on a periodic mesh
-    if (bin_particles(plan, m, prec, np, xp, s, &nbad, m.periodic[0] && m.periodic[1])) return PPMG_ERROR_FATAL;
+    // a slot table, or an unchecked lattice, on a periodic mesh
+    const bool periodic = m.periodic[0] && m.periodic[1];
+    if (bin_particles(plan, m, prec, np, xp, s, &nbad, periodic, periodic)) return PPMG_ERROR_FATAL;
     if (nbad > 0) return 1;
     mark(plan, s);
     if (np <= 0) return 0;
+    auto gather = [&]() -> int {
 #define TYPED(KS)                                                                                             \
     do {                                                                                                      \
         if (prec == PPMG_PREC_F64)                                                                            \
@@ -278,9 +306,11 @@ int m2p2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t 
         return m2p2d_typed<KS, float, float, double>(plan, m, (const float*)xp, fg, (const float*)field,      \
                                                      (float*)up, s);                                          \
     } while (0)
-    if (kernel == PPMG_KERNEL_BSP2) TYPED(2);
-    TYPED(4);
+        if (kernel == PPMG_KERNEL_BSP2) TYPED(2);
+        TYPED(4);
 #undef TYPED
+    };
+    return gather_checked(plan, m, prec, np, xp, periodic, s, gather);
 }
 
 }  // namespace ppmg

@@ -457,12 +457,6 @@ static int m2p3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const PosT
 // issues at the FP32 rate, so the FP32-compensated form keeps FP32 only where
 // it saves bytes (field in HBM and LDS, output) and sums its 64 products in
 // FP64 registers -- more accurate than compensated FP32 at no extra cost.
-//
-// A plan whose last binning found a lattice in cell order (particle p in
-// cell p, one per cell: a fresh lattice of remeshed particles) takes the
-// next one on the same mesh as that lattice without a binning pass: the
-// gather checks every particle's cell key and, should one differ, the call
-// bins and gathers again.
 int m2p3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp,
                const FieldGeom& fg, const void* field, void* up, bool prebinned, hipStream_t s) {
     const bool periodic = m2p3d_table_applicable(m);
@@ -489,22 +483,7 @@ int m2p3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t 
         TYPED(4);
 #undef TYPED
     };
-    if (!plan->bin_lattice) return gather();
-    // (the binning cleared the mismatch flag)
-    if (gather()) return PPMG_ERROR_FATAL;
-    int off = 0;
-    if (read_back(plan, plan->err.as<int>() + 6, 1, &off, s)) return PPMG_ERROR_FATAL;
-    if (!off) {
-        plan->lattice_checked = true;   // the plan's binning is the lattice (heads written on demand)
-        return 0;
-    }
-    // not that lattice: bin and gather again (and bin the next 16 inputs)
-    plan->lattice_flag_clear = false;
-    plan->lattice_pred = false;
-    plan->lattice_skip = 16;
-    if (bin_particles(plan, m, prec, np, xp, s, &nbad, periodic, false)) return PPMG_ERROR_FATAL;
-    if (nbad > 0) return 1;
-    return gather();
+    return gather_checked(plan, m, prec, np, xp, periodic, s, gather);
 }
 
 }  // namespace ppmg

@@ -88,6 +88,34 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
 int sort_rows(int dim, int prec, int64_t np, void* xp, const int* lpdx1, const int* lhbx1, int64_t nbox, int* npbx,
               DevBuf& tmp, hipStream_t s);
 
+// Runs a gather of the plan's binning.  A plan whose last binning found a
+// lattice in cell order (particle p in cell p, one per cell: a fresh lattice of
+// remeshed particles) takes the next one on the same mesh as that lattice
+// without a binning pass: the gather checks every particle's cell key and,
+// should one differ, the particles are binned (table: a slot table will do) and
+// gathered again.  Returns 1 when some particle then lies outside the sub.
+template <typename F>
+int gather_checked(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const void* xp, bool table, hipStream_t s,
+                   F&& gather) {
+    if (!plan->bin_lattice) return gather();
+    // (the binning cleared the mismatch flag)
+    if (gather()) return PPMG_ERROR_FATAL;
+    int off = 0;
+    if (read_back(plan, plan->err.as<int>() + 6, 1, &off, s)) return PPMG_ERROR_FATAL;
+    if (!off) {
+        plan->lattice_checked = true;   // the plan's binning is the lattice (heads written on demand)
+        return 0;
+    }
+    // not that lattice: bin and gather again (and bin the next 16 inputs)
+    plan->lattice_flag_clear = false;
+    plan->lattice_pred = false;
+    plan->lattice_skip = 16;
+    int64_t nbad = 0;
+    if (bin_particles(plan, m, prec, np, xp, s, &nbad, table, false)) return PPMG_ERROR_FATAL;
+    if (nbad > 0) return 1;
+    return gather();
+}
+
 // ------------------------------------------- work list (ppmg_work.hip) --
 // Tile columns of a 3D tile kernel: ntx x nty tiles of tx x ty, marching
 // `planes` planes; a tile's cells are the ncol x nrow ones starting at offset

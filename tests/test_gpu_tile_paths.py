@@ -151,3 +151,55 @@ def test_gather_wide_rows(core, monkeypatch, nx, bc, parts, prec):
             assert torch.equal(got, m2p(plan))
         ref = _general(monkeypatch, m2p)
         assert ((got - ref).abs().max() / ref.abs().max()).item() < (1e-13 if prec == F64 else 1e-6)
+
+
+@pytest.mark.parametrize("shape", [(4, 5), (30, 17), (65, 40)])
+@pytest.mark.parametrize("ghost", [0, 2])
+@pytest.mark.parametrize("kernel", [MP4, BSP2])
+@pytest.mark.parametrize("prec", [F64, F32])
+def test_plane_lattice_without_binning(core, shape, ghost, kernel, prec):
+    """2D: a plan that has seen a lattice in cell order gathers at the next one
+    without a binning pass.  One plan is fed the lattice (binned), two more
+    (no pass), one with two particles swapped and one with a NaN (checked, then
+    binned again), and a lattice after 16 binned ones: every output, or error,
+    is bitwise that of a fresh plan, and sort_view gives the identity."""
+    nx, ny = shape
+    n = nx * ny
+    rng = np.random.default_rng(nx + ghost)
+    i = np.arange(n)
+    side = np.array(shape) / max(shape)
+    mesh = core.Mesh(2, [nx + 1, ny + 1], [0.0] * 2, list(side))
+    vdt = core.VAL_DTYPE[prec]
+    fs = mesh.padded_shape(3, [ghost] * 2) if ghost else mesh.compact_shape(3)
+    f = torch.as_tensor(rng.normal(size=fs)).to(vdt).cuda()
+
+    def call(x, plan=None):
+        out = torch.zeros((n, 3), dtype=vdt, device="cuda")
+        try:
+            core.m2p(mesh, x, f, [-ghost] * 2, out, kernel, prec, plan=plan)
+        except RuntimeError as e:
+            return str(e)
+        return out
+
+    def lattice():
+        x = (np.stack([i % nx, i // nx], 1) + rng.uniform(0.05, 0.95, (n, 2))) / shape * side
+        return torch.as_tensor(x).to(core.POS_DTYPE[prec]).cuda()
+
+    plan = core.Plan()
+    for case in ["lattice"] * 3 + ["swapped", "lattice", "lattice"] + ["lattice"] * 16 + ["nan", "lattice"]:
+        x = lattice()
+        if case == "swapped":
+            x[[0, n - 1]] = x[[n - 1, 0]]
+        elif case == "nan":
+            x[n // 2, 1] = float("nan")
+        got, ref = call(x, plan), call(x)
+        assert type(got) is type(ref), case
+        if isinstance(ref, str):
+            assert got == ref
+            continue
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(ref)), case
+        if case == "lattice":
+            k, perm, start = plan.sort_view()
+            assert np.array_equal(start.cpu().numpy(), np.arange(n + 1))
+            assert np.array_equal(perm.cpu().numpy(), np.arange(n))
+            assert np.array_equal(k.cpu().numpy(), np.arange(n))
