@@ -25,9 +25,9 @@ constexpr int ERR_WORDS = 136;
 // than FAR_CELLS cells from their predecessor, is in no order: the slot atomics
 // and table writes of its key pass each touch a line of their own.
 constexpr int FAR_CELLS = 1024;
-constexpr int64_t FAR_MIN_NP = 1 << 21;
+constexpr int64_t FAR_MIN_NP = 3 << 19;
 // Particles from which util_rank sorts by radix.
-constexpr int64_t RANK_RADIX_NP = 1 << 20;
+constexpr int64_t RANK_RADIX_NP = 3 << 18;
 
 constexpr int SCAN_BLOCK = 256;
 constexpr int SCAN_ITEMS = 16;
@@ -693,7 +693,11 @@ __global__ void __launch_bounds__(256) k_keys_only(const PosT* __restrict__ xp, 
 //
 // A pass sorts by 8 or 9 bits, whichever takes fewer passes over the key's
 // bits (27 bits at 512^3: three passes of 9), with one thread per digit.
-constexpr int RS_ITEMS = 8;
+// RS_ITEMS pairs a thread: longer runs per digit to write and fewer tiles'
+// counts to scan, until a tile's LDS leaves too few workgroups (2^24 keys in
+// no order 471, 440, 460 us at 8, 16 and 24; clustered 2^26 2.03, 1.97, 1.94
+// and 2.45 ms at 8, 12, 16 and 24 with 9 bits).
+constexpr int RS_ITEMS = 16;
 template <int BITS> struct Radix {
     static constexpr int BUCKETS = 1 << BITS;
     static constexpr int THREADS = BUCKETS;                // one digit per thread in the tile loops
@@ -745,7 +749,8 @@ __device__ __forceinline__ uint64_t digit_peers(int d, bool live) {
 
 // Digit counts of every tile, digit-major: hist[d * ntiles + tile].  Tiles
 // are numbered XCD-contiguously (xcd_tile), as in k_rs_scatter: the tiles
-// one XCD sorts are neighbours, and so are their runs of each digit.
+// one XCD sorts are neighbours, and so are their runs of each digit.  2^24
+// keys: 17 us, 40 with the digit's lanes searched for every key.
 template <int BITS>
 __global__ void __launch_bounds__(Radix<BITS>::THREADS) k_rs_hist(const int* __restrict__ keys, int64_t n, int shift,
                                                                   int* __restrict__ hist, int64_t ntiles) {
@@ -766,83 +771,111 @@ __global__ void __launch_bounds__(Radix<BITS>::THREADS) k_rs_hist(const int* __r
     for (int j = 0; j < RS_ITEMS; ++j) {
         const bool live = t0 + j * R::THREADS + tid < n;
         const int d = (k[j] >> shift) & (R::BUCKETS - 1);
-        // one LDS add per digit and wavefront
-        const uint64_t peers = digit_peers<BITS>(d, live);
-        if (live && (int)__builtin_ctzll(peers) == lane) atomicAdd(&h[d], (int)__popcll(peers));
+        // one LDS add per lane, or, where many lanes hold the first lane's
+        // digit, one for all of those
+        const uint64_t same = __ballot(live && d == __builtin_amdgcn_readfirstlane(d));
+        if (__popcll(same) > 8) {
+            if (lane == 0) atomicAdd(&h[d], (int)__popcll(same));
+            if (live && !((same >> lane) & 1)) atomicAdd(&h[d], 1);
+        } else if (live) {
+            atomicAdd(&h[d], 1);
+        }
     }
     __syncthreads();
     hist[(int64_t)tid * ntiles + tile] = h[tid];
 }
 
-// One stable pass.  The pairs of a tile are first ordered by digit in LDS: a
-// tile is taken THREADS pairs a round in index order, and a pair's place
-// is its digit's start in the tile plus its rank among the tile's pairs of
-// that digit (the count from earlier rounds, earlier wavefronts of its round
-// and earlier lanes of its wavefront).  The tile then writes its digit runs
-// at their offsets (offs: the exclusive scan of hist), consecutive threads to
-// consecutive addresses.  vin nullptr: the values are the pairs' indices
-// (the first pass); vadd is added to the values written (1: one-based ranks).
-// vmax: values at positions from vmax on are not written.
+// One stable pass.  The pairs of a tile are first ordered by digit in LDS.  A
+// wavefront takes a run of 64 ITEMS pairs, 64 at a time in index order, and
+// counts its digits as it goes: a pair's place is its digit's start in the
+// tile, plus that digit's pairs in the wavefronts before, plus its rank among
+// this wavefront's (the count so far and the lanes below with the same digit).
+// The tile then writes its digit runs at their offsets (offs: the exclusive
+// scan of the tiles' counts), consecutive threads to consecutive addresses,
+// the keys first and the values through the same LDS.  Bound by memory with
+// runs of half a line: 2^24 pairs of 8 bits 73 us (268 MB), 116 with the
+// wavefronts in step, a barrier per 64 pairs.  vin nullptr: the values
+// are the pairs' indices (the first pass); vadd is added to the values written
+// (1: one-based ranks).  vmax: values at positions from vmax on are not written.
 template <int BITS>
 __global__ void __launch_bounds__(Radix<BITS>::THREADS)
 k_rs_scatter(const int* __restrict__ kin, const int* __restrict__ vin, int64_t n, int shift,
-             const int* __restrict__ hist, const int* __restrict__ offs, int64_t ntiles, int* __restrict__ kout,
-             int* __restrict__ vout, int vadd, int64_t vmax) {
+             const int* __restrict__ offs, int64_t ntiles, int* __restrict__ kout, int* __restrict__ vout, int vadd,
+             int64_t vmax) {
     using R = Radix<BITS>;
-    __shared__ int base[R::BUCKETS];     // next place of each digit in the tile's order
     __shared__ int shift_out[R::BUCKETS];   // global position minus place, per digit
     __shared__ int wcnt[R::NWAVE][R::BUCKETS];
-    __shared__ int sk[R::TILE], sv[R::TILE];
+    __shared__ int sk[R::TILE];
     __shared__ int64_t sh[R::NWAVE + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t tile = xcd_tile(blockIdx.x, (int64_t)gridDim.x);
     const int64_t t0 = tile * R::TILE;
     const int tn = (int)min((int64_t)R::TILE, n - t0);
+    const int w0 = wave * (64 * RS_ITEMS);
     int kk[RS_ITEMS], vv[RS_ITEMS];   // all loads in flight before the first round
 #pragma unroll
     for (int j = 0; j < RS_ITEMS; ++j) {
-        const int64_t i = t0 + j * R::THREADS + tid;
-        kk[j] = i < n ? kin[i] : 0;
-        vv[j] = i < n ? (vin ? vin[i] : (int)i) : 0;
+        const int q = w0 + j * 64 + lane;
+        kk[j] = q < tn ? kin[t0 + q] : 0;
+        vv[j] = q < tn ? (vin ? vin[t0 + q] : (int)(t0 + q)) : 0;
     }
-    // thread t = digit t: its start in the tile (exclusive scan of the tile's counts)
-    int64_t lb;
-    block_exclusive_scan<R::THREADS>((int64_t)hist[(int64_t)tid * ntiles + tile], sh, lb);
-    base[tid] = (int)lb;
-    shift_out[tid] = offs[(int64_t)tid * ntiles + tile] - (int)lb;
 #pragma unroll
     for (int w = 0; w < R::NWAVE; ++w) wcnt[w][tid] = 0;
     const uint64_t lt = lane ? ~0ull >> (64 - lane) : 0ull;   // lanes below this one
     __syncthreads();
+    int rank[RS_ITEMS];
 #pragma unroll
     for (int j = 0; j < RS_ITEMS; ++j) {
-        const bool live = t0 + j * R::THREADS + tid < n;
+        const bool live = w0 + j * 64 + lane < tn;
         const int d = (kk[j] >> shift) & (R::BUCKETS - 1);
         const uint64_t peers = digit_peers<BITS>(d, live);
-        if (live && (int)__builtin_ctzll(peers) == lane) wcnt[wave][d] = (int)__popcll(peers);
-        __syncthreads();
-        if (live) {
-            int r = base[d] + (int)__popcll(peers & lt);
-            for (int w = 0; w < wave; ++w) r += wcnt[w][d];
-            sk[r] = kk[j];
-            sv[r] = vv[j];
-        }
-        __syncthreads();
-        // thread t owns digit t: advance its place, clear its counts
-        int add = 0;
-#pragma unroll
-        for (int w = 0; w < R::NWAVE; ++w) {
-            add += wcnt[w][tid];
-            wcnt[w][tid] = 0;
-        }
-        base[tid] += add;
-        __syncthreads();
+        const int before = wcnt[wave][d];
+        rank[j] = before + (int)__popcll(peers & lt);
+        wave_lds_sync();
+        if (live && (peers & lt) == 0ull) wcnt[wave][d] = before + (int)__popcll(peers);
+        wave_lds_sync();
     }
-    for (int q = tid; q < tn; q += R::THREADS) {
-        const int k = sk[q];
-        const int o = shift_out[(k >> shift) & (R::BUCKETS - 1)] + q;
-        kout[o] = k;
-        if (o < vmax) vout[o] = sv[q] + vadd;
+    __syncthreads();
+    // thread t = digit t: its start in the tile, and each wavefront's in it
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < R::NWAVE; ++w) total += wcnt[w][tid];
+    int64_t lb;
+    block_exclusive_scan<R::THREADS>((int64_t)total, sh, lb);
+    shift_out[tid] = offs[(int64_t)tid * ntiles + tile] - (int)lb;
+    int run = (int)lb;
+#pragma unroll
+    for (int w = 0; w < R::NWAVE; ++w) {
+        const int c = wcnt[w][tid];
+        wcnt[w][tid] = run;
+        run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j) {
+        rank[j] += wcnt[wave][(kk[j] >> shift) & (R::BUCKETS - 1)];
+        if (w0 + j * 64 + lane < tn) sk[rank[j]] = kk[j];
+    }
+    __syncthreads();
+    int o[RS_ITEMS];
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j) {
+        const int q = j * R::THREADS + tid;
+        if (q < tn) {
+            const int k = sk[q];
+            o[j] = shift_out[(k >> shift) & (R::BUCKETS - 1)] + q;
+            kout[o[j]] = k;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j)
+        if (w0 + j * 64 + lane < tn) sk[rank[j]] = vv[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j) {
+        const int q = j * R::THREADS + tid;
+        if (q < tn && o[j] < vmax) vout[o[j]] = sk[q] + vadd;
     }
 }
 
@@ -964,8 +997,8 @@ static int radix_sort_bits(ppmg_plan* plan, const int* keys, int64_t n, int pass
         int* vo = last ? vout : plan->rval[pass & 1].as<int>();
         hipLaunchKernelGGL(k_rs_hist<BITS>, dim3((unsigned)ntiles), dim3(R::THREADS), 0, s, kin, n, shift, hist, ntiles);
         if (exclusive_scan(hist, R::BUCKETS * ntiles, offs, plan->scan_tmp, n, s)) return PPMG_ERROR_FATAL;
-        hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3((unsigned)ntiles), dim3(R::THREADS), 0, s, kin, vin, n, shift, hist,
-                           offs, ntiles, kout, vo, last ? vadd : 0, last ? vmax : n);
+        hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3((unsigned)ntiles), dim3(R::THREADS), 0, s, kin, vin, n, shift, offs,
+                           ntiles, kout, vo, last ? vadd : 0, last ? vmax : n);
         kin = kout;
         vin = vo;
     }
@@ -1106,8 +1139,8 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     if (table && !predict_sorted && plan->table_skip > 0) --plan->table_skip;
     // Crowded input (the last binning's sample found a cell of nine or more
     // particles per 64 particles), and large input in no order, is binned by the
-    // radix sort (16.8M particles of 256^3 cells in random order: 0.68 against
-    // 1.04 ms; the two meet at 2^21 particles, P2M 335 and 341 us); PPMG_RADIX=1
+    // radix sort (16.8M particles of 256^3 cells in random order: 0.49 against
+    // 1.04 ms; 2.1M 129 against 173 us, 1.03M 109 against 96); PPMG_RADIX=1
     // forces that path for input not predicted in cell order, PPMG_RADIX=0
     // rules it out (both for tests).  Allocation-free calls keep the counting
     // path (the sort needs four more int32 per particle).
@@ -1342,8 +1375,8 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
     if (materialize_heads(plan, s)) return PPMG_ERROR_FATAL;
     plan->prebinned = false;
     // Large input is ranked by the radix sort of its cell keys (2^24 particles in
-    // no order, eight to a box: 0.56 against 1.34 ms; 2^20: 122 against 135 us,
-    // 2^19: 119 against 107); slot
+    // no order, eight to a box: 0.46 against 1.34 ms; 10^6: 102 against 114 us,
+    // 2^19: 98 against 85); slot
     // atomics and per-cell sorts keep the small ones, whose counts stay in L2
     // and which have few launches (PPMG_RADIX forces either, as in the binning).
     const char* rx = std::getenv("PPMG_RADIX");
