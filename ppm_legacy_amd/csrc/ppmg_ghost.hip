@@ -137,6 +137,7 @@ struct GhostList {
     unsigned wg[27];
     int64_t per;                // elements per workgroup
     int N[3];                   // cells per axis (0: not an axis of the mesh)
+    int face[26];               // the only shifted axis of a face's block, else -1
     int nb;
 };
 constexpr int GHOST_WG = 256;   // threads per workgroup
@@ -228,9 +229,13 @@ __global__ void __launch_bounds__(GHOST_WG) k_ghost_pop(T* __restrict__ field, F
         bool other = false;   // another block's thread carries out this node's list
         if (get) {
             for (int d = 0; d < 3; ++d) n[d] += l.b[q].off[d];
-            // two images of the real range 0..N meet on the nodes 0 and N only
+            // Two images of the real range 0..N meet on the nodes 0 and N only,
+            // and a face's shares its own axis' node with the real range, no
+            // image: a third of a face's nodes need no search of the blocks (256^3
+            // box, ghost size 2, lda 3, FP64: 36 us, 69 with one for every seam node).
             bool seam = false;
-            for (int d = 0; d < 3; ++d) seam = seam || (l.N[d] && (n[d] == 0 || n[d] == l.N[d]));
+            for (int d = 0; d < 3; ++d)
+                seam = seam || (d != l.face[q] && l.N[d] && (n[d] == 0 || n[d] == l.N[d]));
             if (seam)
                 for (int p = q + 1; p < l.nb && !other; ++p) other = ghost_holds(l.b[p], n, true);
         } else {
@@ -270,6 +275,13 @@ static int ghost_typed(const DevMesh& m, T* field, const FieldGeom& fg, const Gh
     l.base[0] = 0;
     for (int q = 0; q < nb; ++q) {
         l.b[q] = b[q];
+        int shifted = 0, axis = -1;
+        for (int d = 0; d < 3; ++d)
+            if (b[q].off[d] != 0) {
+                ++shifted;
+                axis = d;
+            }
+        l.face[q] = shifted == 1 ? axis : -1;
         l.base[q + 1] = l.base[q] + (int64_t)b[q].size[0] * b[q].size[1] * b[q].size[2] * fg.lda;
     }
     if (l.base[nb] == 0) return 0;
