@@ -437,8 +437,8 @@ int ppmg_m2p_prebin(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, con
     int64_t nbad = 0;
     plan->have_forward = false;
     // the tiled gather checks a lattice taken without a pass (m2p3d_fast)
-    if (bin_particles(plan, m, prec, np, xp, as_stream(stream), &nbad, m2p3d_table_applicable(m),
-                      m2p3d_table_applicable(m)))
+    if (bin_particles(plan, m, prec, np, xp, as_stream(stream), &nbad, true,
+                      m2p3d_lattice_applicable(m)))
         return g_status.info;
     plan->prebinned = true;
     plan->prebin_xp = xp;

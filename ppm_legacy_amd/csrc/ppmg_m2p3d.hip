@@ -367,9 +367,8 @@ bool m2p3d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg) {
     return (int64_t)fg.ext[0] * fg.ext[1] * fg.lda * 8 < ((int64_t)1 << 31);
 }
 
-// The gather reads a slot-table binning on a periodic mesh (whatever the
-// field's layout).
-bool m2p3d_table_applicable(const DevMesh& m) { return m.dim == 3 && m.periodic[0] && m.periodic[1] && m.periodic[2]; }
+// The gather checks a lattice's cells on a periodic mesh.
+bool m2p3d_lattice_applicable(const DevMesh& m) { return m.dim == 3 && m.periodic[0] && m.periodic[1] && m.periodic[2]; }
 
 // One launch of the gather for components c0 .. c0+LL-1, rows of W lanes.
 template <int KS, int W, int LL, typename PosT, typename ValT, typename AccT, bool OPEN, bool MIX, bool TABLE, bool LAT>
@@ -420,17 +419,14 @@ static int launch_m3_open(ppmg_plan* plan, const DevMesh& m, const PosT* xp, con
 template <int KS, int LL, typename PosT, typename ValT, typename AccT>
 static int launch_m3(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const FieldGeom& fg, int c0,
                       const ValT* field, ValT* up, hipStream_t s) {
-    // a slot table or an unchecked lattice is binned on periodic meshes only (m2p3d_fast)
-    if (plan->bin_lattice)
-        return launch_m3_open<KS, LL, PosT, ValT, AccT, false, false, false, true>(plan, m, xp, fg, c0, field, up, s);
-    else if (plan->bin_table)
-        return launch_m3_open<KS, LL, PosT, ValT, AccT, false, false, true>(plan, m, xp, fg, c0, field, up, s);
-    else if (m.periodic[0] && m.periodic[1] && m.periodic[2])
-        return launch_m3_open<KS, LL, PosT, ValT, AccT, false, false>(plan, m, xp, fg, c0, field, up, s);
-    else if (fg.swap[0] || fg.swap[1] || fg.swap[2])
-        return launch_m3_open<KS, LL, PosT, ValT, AccT, true, true>(plan, m, xp, fg, c0, field, up, s);
-    else
-        return launch_m3_open<KS, LL, PosT, ValT, AccT, true, false>(plan, m, xp, fg, c0, field, up, s);
+    // an unchecked lattice is binned on periodic meshes only (m2p3d_fast)
+    const bool open = !(m.periodic[0] && m.periodic[1] && m.periodic[2]);
+    const bool mix = open && (fg.swap[0] || fg.swap[1] || fg.swap[2]);
+#define M3(...) launch_m3_open<KS, LL, PosT, ValT, AccT, __VA_ARGS__>(plan, m, xp, fg, c0, field, up, s)
+    if (plan->bin_lattice) return M3(false, false, false, true);
+    if (plan->bin_table) return !open ? M3(false, false, true) : mix ? M3(true, true, true) : M3(true, false, true);
+    return !open ? M3(false, false) : mix ? M3(true, true) : M3(true, false);
+#undef M3
 }
 
 template <int KS, typename PosT, typename ValT, typename AccT>
@@ -459,12 +455,10 @@ static int m2p3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const PosT
 // FP64 registers -- more accurate than compensated FP32 at no extra cost.
 int m2p3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp,
                const FieldGeom& fg, const void* field, void* up, bool prebinned, hipStream_t s) {
-    const bool periodic = m2p3d_table_applicable(m);
     int64_t nbad = prebinned ? plan->prebin_nbad : 0;
-    if (!prebinned && bin_particles(plan, m, prec, np, xp, s, &nbad, periodic, periodic)) return PPMG_ERROR_FATAL;
+    if (!prebinned && bin_particles(plan, m, prec, np, xp, s, &nbad, true, m2p3d_lattice_applicable(m)))
+        return PPMG_ERROR_FATAL;
     if (nbad > 0) return 1;
-    // (a prebinning of a mesh the gather cannot read as a table or check as a lattice)
-    if ((plan->bin_table || plan->bin_lattice) && !periodic && materialize_heads(plan, s)) return PPMG_ERROR_FATAL;
     mark(plan, s);
     if (np <= 0) return 0;
     auto gather = [&]() -> int {
@@ -483,7 +477,7 @@ int m2p3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t 
         TYPED(4);
 #undef TYPED
     };
-    return gather_checked(plan, m, prec, np, xp, periodic, s, gather);
+    return gather_checked(plan, m, prec, np, xp, true, s, gather);
 }
 
 }  // namespace ppmg
