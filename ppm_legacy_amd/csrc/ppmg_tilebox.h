@@ -25,35 +25,48 @@ template <typename ValT> struct WTab {
 // tiles wrote there.  Enumerated as the face i = N, then j = N (i < N), then
 // k = N (i, j < N), over the real nodes (r per axis, b = 1 where node N is a
 // copy).
+struct BoxDup {
+    int3 n, r, b;
+    int64_t ndup;
+    unsigned wg;   // workgroups of 256 nodes
+};
 template <typename ValT>
-__global__ void __launch_bounds__(256) k_box_dup(FieldGeom fg, int3 n, int3 r, int3 b, ValT* __restrict__ field,
-                                                int64_t ndup) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ndup) return;
-    const int64_t fx = b.x ? (int64_t)r.y * r.z : 0;
-    const int64_t fy = b.y ? (int64_t)(r.x - b.x) * r.z : 0;
+__device__ __forceinline__ void box_dup(const FieldGeom& fg, const BoxDup& d, ValT* __restrict__ field, int64_t tt) {
+    if (tt >= d.ndup) return;
     int i, j, k;
-    if (t < fx) {
-        i = n.x;
-        j = (int)(t % r.y);
-        k = (int)(t / r.y);
-    } else if (t < fx + fy) {
-        const int64_t q = t - fx;
-        i = (int)(q % (r.x - b.x));
-        j = n.y;
-        k = (int)(q / (r.x - b.x));
-    } else {
-        const int64_t q = t - fx - fy;
-        i = (int)(q % (r.x - b.x));
-        j = (int)((q / (r.x - b.x)) % (r.y - b.y));
-        k = n.z;
-    }
+    auto locate = [&](auto t) {   // 32-bit divisions wherever the node count fits
+        using U = decltype(t);
+        const U fx = d.b.x ? (U)d.r.y * (U)d.r.z : 0;
+        const U wx = (U)(d.r.x - d.b.x), wy = (U)(d.r.y - d.b.y);
+        const U fy = d.b.y ? wx * (U)d.r.z : 0;
+        if (t < fx) {
+            i = d.n.x;
+            j = (int)(t % (U)d.r.y);
+            k = (int)(t / (U)d.r.y);
+        } else if (t < fx + fy) {
+            t -= fx;
+            i = (int)(t % wx);
+            j = d.n.y;
+            k = (int)(t / wx);
+        } else {
+            t -= fx + fy;
+            i = (int)(t % wx);
+            j = (int)((t / wx) % wy);
+            k = d.n.z;
+        }
+    };
+    if ((uint64_t)d.ndup >> 32) locate((uint64_t)tt);
+    else locate((uint32_t)tt);
     auto at = [&](int x, int y, int z) {
         return (((int64_t)(z - fg.lo[2]) * fg.ext[1] + (y - fg.lo[1])) * fg.ext[0] + (x - fg.lo[0])) * fg.lda;
     };
     const int64_t dst = at(i, j, k);
-    const int64_t src = at(i == n.x ? 0 : i, j == n.y ? 0 : j, k == n.z ? 0 : k);
+    const int64_t src = at(i == d.n.x ? 0 : i, j == d.n.y ? 0 : j, k == d.n.z ? 0 : k);
     for (int c = 0; c < fg.lda; ++c) field[dst + c] = field[src + c];
+}
+template <typename ValT>
+__global__ void __launch_bounds__(256) k_box_dup(FieldGeom fg, BoxDup dup, ValT* __restrict__ field) {
+    box_dup<ValT>(fg, dup, field, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // Stored nodes outside 0..N on some axis (ghost layers): the raw sum of the
@@ -73,7 +86,9 @@ __global__ void __launch_bounds__(256) k_box_dup(FieldGeom fg, int3 n, int3 r, i
 // node, cell j going to lane j mod 4; a lane has the heads of four cells and
 // then their first particles in flight at once, so a node takes one pass of the
 // chain, and the short register list leaves many wavefronts resident.  The
-// four partial sums are added in a fixed order.  (One lane per node, 16 heads
+// four partial sums are added in a fixed order.  The first dup.wg workgroups
+// make node N's copies (box_dup), so that a small box has one launch fewer
+// (3 us of 82 for a step on 32^3 cells).  (One lane per node, 16 heads
 // and then four batches of four particles, against this: 115 and 84 us at
 // 256^3, ghost size 2, lda 3, FP32c; 40 and 11 us at 64^3, FP64.)
 constexpr int SHELL_LANES = 4;   // lanes per node (a DPP quad)
@@ -97,9 +112,13 @@ __global__ void __launch_bounds__(256) k_box_shell(DevMesh m, FieldGeom fg, int3
                                                   const int* __restrict__ perm, BinTable bt,
                                                   const PosT* __restrict__ xp, const ValT* __restrict__ up, int c0,
                                                   ValT* __restrict__ field, int64_t t0, int64_t nshell,
-                                                  WTab<ValT> wt) {
+                                                  WTab<ValT> wt, BoxDup dup) {
+    if (blockIdx.x < dup.wg) {
+        box_dup<ValT>(fg, dup, field, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
+        return;
+    }
     const int sub = threadIdx.x & (SHELL_LANES - 1);
-    const int64_t tq = t0 + ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / SHELL_LANES;
+    const int64_t tq = t0 + ((int64_t)(blockIdx.x - dup.wg) * blockDim.x + threadIdx.x) / SHELL_LANES;
     const bool live = tq < nshell;   // a quad past the end works on the last node and stores nothing
     const int64_t t = live ? tq : nshell - 1;
     const int e0 = fg.ext[0], e1 = fg.ext[1], e2 = fg.ext[2];
@@ -242,10 +261,9 @@ int fill_stored_box(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const Val
     const int3 n3 = make_int3(D[0], D[1], D[2]), r3 = make_int3(R[0], R[1], R[2]),
                b3 = make_int3(B[0], B[1], B[2]);
     const int64_t ndup = (int64_t)R[0] * R[1] * R[2] - (int64_t)(R[0] - B[0]) * (R[1] - B[1]) * (R[2] - B[2]);
-    if (ndup > 0)
-        hipLaunchKernelGGL(k_box_dup<ValT>, dim3((unsigned)((ndup + 255) / 256)), dim3(256), 0, s, fg, n3, r3, b3,
-                           field, ndup);
     const int64_t nshell = (int64_t)fg.ext[0] * fg.ext[1] * fg.ext[2] - (int64_t)R[0] * R[1] * R[2];
+    BoxDup dup{n3, r3, b3, ndup, (unsigned)((ndup + 255) / 256)};
+    if (ndup > 0 && nshell == 0) hipLaunchKernelGGL(k_box_dup<ValT>, dim3(dup.wg), dim3(256), 0, s, fg, dup, field);
     if (nshell > 0) {
         const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
         const bool table = plan->bin_table;
@@ -257,8 +275,9 @@ int fill_stored_box(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const Val
     for (int64_t t0 = 0; t0 < nshell; t0 += (int64_t)1 << 28) {                                                       \
         const int64_t nt = nshell - t0 < ((int64_t)1 << 28) ? nshell - t0 : (int64_t)1 << 28;                          \
         hipLaunchKernelGGL((k_box_shell<DIM, KS, PosT, ValT, LL, TB>),                                                \
-                           dim3((unsigned)((nt * SHELL_LANES + 255) / 256)), dim3(256), 0, s, m, fg, r3,              \
-                           plan->start.as<int>(), tile_perm(plan), bt, xp, up, c0, field, t0, t0 + nt, wt);           \
+                           dim3((unsigned)((nt * SHELL_LANES + 255) / 256) + dup.wg), dim3(256), 0, s, m, fg, r3,     \
+                           plan->start.as<int>(), tile_perm(plan), bt, xp, up, c0, field, t0, t0 + nt, wt, dup);      \
+        dup.wg = 0;   /* (the copies are of all components) */                                                       \
     }
 #define SHL(LL)                      \
     do {                             \
