@@ -297,8 +297,8 @@ int ppmg_map_field_ghost_kind(const ppmg_mesh* mesh, int kind, const ppmg_field*
 int ppmg_plan_sort_view(const ppmg_plan* plan, const int** key, const int** perm, const int** start, int64_t* np,
                         int64_t* ncells) {
     if (!plan) return fail(PPMG_ERROR_ERROR, PPMG_ERR_ARGUMENT, "plan is NULL");
-    if ((perm || start) && plan->bin_table) {
-        // the binning left a slot table: build the heads and the permutation
+    if ((perm || start) && (plan->bin_table || plan->bin_lattice)) {
+        // the binning left a slot table or a lattice: build the heads and the permutation
         ppmg_plan* w = const_cast<ppmg_plan*>(plan);
         if (materialize_heads(w, w->bin_stream)) return g_status.info;
         PPMG_HIP(hipStreamSynchronize(w->bin_stream));

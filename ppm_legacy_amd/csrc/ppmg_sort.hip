@@ -1079,14 +1079,16 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     // the scan reads whole tiles of SCAN_TILE cells
     const size_t count_alloc = ((size_t)ncells + SCAN_TILE - 1) / SCAN_TILE * SCAN_TILE;
     if (plan->err.bytes < sizeof(int) * ERR_WORDS) plan->lattice_flag_clear = false;   // about to be allocated
-    if (plan->key.ensure(sizeof(int) * npb) || plan->slot.ensure(npb + 16) ||
-        plan->perm.ensure(sizeof(int) * npb) || plan->count.ensure(count_alloc) ||
-        plan->start.ensure(sizeof(int) * (size_t)(ncells + 1)) ||
-        plan->gaps.ensure(sizeof(int4) * (size_t)gapcap) ||
-        plan->multi.ensure(sizeof(int) * (size_t)nblk(np, KEYS_BLOCK) * KEYS_BLOCK) ||
-        plan->multi_n.ensure(sizeof(int) * (size_t)nblk(np, KEYS_BLOCK)) ||
-        plan->err.ensure(sizeof(int) * ERR_WORDS))
-        return PPMG_ERROR_FATAL;
+    if (plan->err.ensure(sizeof(int) * ERR_WORDS)) return PPMG_ERROR_FATAL;
+    // Keys, permutation and heads are allocated where they are used: a slot
+    // table or a checked lattice goes without (14 bytes per particle and 4 per
+    // cell; materialize_heads and the like allocate them should they be asked
+    // for after all).
+    auto sorted_lists = [&]() {
+        return plan->key.ensure(sizeof(int) * npb) || plan->slot.ensure(npb + 16) ||
+               plan->perm.ensure(sizeof(int) * npb) || plan->start.ensure(sizeof(int) * (size_t)(ncells + 1)) ||
+               plan->gaps.ensure(sizeof(int4) * (size_t)gapcap);
+    };
     plan->bin_stream = s;
     plan->prebinned = false;   // a binning left by ppmg_m2p_prebin is overwritten
     plan->bin_table = false;
@@ -1102,6 +1104,7 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     if (np == 0) {
         plan->perm_identity = true;
         plan->perm_written = true;
+        if (sorted_lists()) return PPMG_ERROR_FATAL;
         return fill_zero(plan->start.p, sizeof(int) * (size_t)(ncells + 1), s);
     }
     // A lattice in cell order (particle p in cell p, np == ncells), as the last
@@ -1149,11 +1152,17 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
                                    : plan->crowded_cells * 64 > np ||
                                          (np >= FAR_MIN_NP && plan->far_particles * 4 > np);
     if (!predict_sorted && radix && !arena_bound()) {
+        if (sorted_lists()) return PPMG_ERROR_FATAL;
         if (fill_zero(plan->err.p, sizeof(int) * ERR_WORDS, s)) return PPMG_ERROR_FATAL;
         plan->lattice_flag_clear = true;
         return bin_crowded(plan, m, prec, np, xp, s, nbad);
     }
-    if (use_table && plan->table.ensure(sizeof(int) * TABLE_SLOTS * (size_t)ncells)) return PPMG_ERROR_FATAL;
+    if (use_table ? plan->table.ensure(sizeof(int) * TABLE_SLOTS * (size_t)ncells) : sorted_lists())
+        return PPMG_ERROR_FATAL;
+    if (plan->count.ensure(count_alloc) ||
+        plan->multi.ensure(sizeof(int) * (size_t)nblk(np, KEYS_BLOCK) * KEYS_BLOCK) ||
+        plan->multi_n.ensure(sizeof(int) * (size_t)nblk(np, KEYS_BLOCK)))
+        return PPMG_ERROR_FATAL;
     int* tab = use_table ? plan->table.as<int>() : nullptr;
     if (fill_zero2(plan->err.p, sizeof(int) * ERR_WORDS, plan->count.p, predict_sorted ? 0 : count_alloc, s))
         return PPMG_ERROR_FATAL;
@@ -1277,6 +1286,7 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
 
 int materialize_keys(ppmg_plan* plan, hipStream_t s) {
     if (!plan->keys_written && plan->np > 0) {
+        if (plan->key.ensure(sizeof(int) * (size_t)plan->np)) return PPMG_ERROR_FATAL;
         const unsigned g = nblk(plan->np, 256);
         const DevMesh& m = plan->bin_mesh;
         int* key = plan->key.as<int>();
@@ -1302,6 +1312,7 @@ int materialize_heads(ppmg_plan* plan, hipStream_t s) {
                                  false);
         }
         // a checked lattice: cell c holds particle c
+        if (plan->start.ensure(sizeof(int) * (size_t)(plan->ncells + 1))) return PPMG_ERROR_FATAL;
         hipLaunchKernelGGL(k_iota, dim3(nblk(plan->ncells + 1, 256)), dim3(256), 0, s, plan->start.as<int>(),
                            plan->ncells + 1);
         PPMG_HIP(hipGetLastError());
@@ -1310,6 +1321,8 @@ int materialize_heads(ppmg_plan* plan, hipStream_t s) {
     }
     if (!plan->bin_table) return 0;
     const int64_t ncells = plan->ncells, np = plan->np;
+    if (plan->start.ensure(sizeof(int) * (size_t)(ncells + 1)) || plan->perm.ensure(sizeof(int) * (size_t)np))
+        return PPMG_ERROR_FATAL;
     int* start = plan->start.as<int>();
     const uint32_t* count8 = plan->count.as<uint32_t>();
     if (exclusive_scan_u8(count8, ncells, start, plan->scan_tmp, np, s)) return PPMG_ERROR_FATAL;
@@ -1325,6 +1338,7 @@ int materialize_heads(ppmg_plan* plan, hipStream_t s) {
 int materialize_perm(ppmg_plan* plan, hipStream_t s) {
     if (materialize_heads(plan, s)) return PPMG_ERROR_FATAL;
     if (plan->perm_identity && !plan->perm_written && plan->np > 0) {
+        if (plan->perm.ensure(sizeof(int) * (size_t)plan->np)) return PPMG_ERROR_FATAL;
         hipLaunchKernelGGL(k_identity, dim3(nblk(plan->np, 256)), dim3(256), 0, s, plan->np, plan->perm.as<int>());
         PPMG_HIP(hipGetLastError());
     }
