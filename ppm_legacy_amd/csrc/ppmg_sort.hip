@@ -146,9 +146,22 @@ __global__ void __launch_bounds__(SUMS_THREADS) k_scan_sums(int64_t* __restrict_
     }
 }
 
+// Up to FEW_SUMS block sums are not scanned by a launch of their own: each
+// block of the last pass adds up the sums before its own (ranking of 2^24
+// particles, three scans: 418 -> 411 us).
+constexpr int64_t FEW_SUMS = 1024;
+
+// Prefix of this workgroup: its scanned sum, or (few) the plain sums before it.
+__device__ __forceinline__ int64_t block_prefix(const int64_t* __restrict__ sums, bool few, int64_t* sh) {
+    if (!few) return sums[blockIdx.x];
+    int64_t v = 0, excl;
+    for (unsigned b = threadIdx.x; b < blockIdx.x; b += SCAN_BLOCK) v += sums[b];
+    return block_exclusive_scan(v, sh, excl);
+}
+
 template <bool VEC>
 __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_down(const int* __restrict__ in, int64_t n,
-                                                          const int64_t* __restrict__ offs,
+                                                          const int64_t* __restrict__ sums, bool few,
                                                           int* __restrict__ out, int64_t total_out) {
     __shared__ int64_t sh[SCAN_BLOCK / 64 + 1];
     int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
@@ -158,8 +171,9 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_down(const int* __restrict_
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) s += vals[i];
     int64_t excl;
+    const int64_t prefix = block_prefix(sums, few, sh);
     block_exclusive_scan(s, sh, excl);
-    int64_t run = offs[blockIdx.x] + excl;
+    int64_t run = prefix + excl;
     int o[SCAN_ITEMS];
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) {
@@ -187,9 +201,10 @@ int exclusive_scan(const int* in, int64_t n, int* out, DevBuf& tmp, int64_t tota
     const bool vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
     if (vec) hipLaunchKernelGGL(k_scan_reduce<true>, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums);
     else hipLaunchKernelGGL(k_scan_reduce<false>, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SUMS_THREADS), 0, s, sums, nb);
-    if (vec) hipLaunchKernelGGL(k_scan_down<true>, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, out, total);
-    else hipLaunchKernelGGL(k_scan_down<false>, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, out, total);
+    const bool few = nb <= FEW_SUMS;
+    if (!few) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SUMS_THREADS), 0, s, sums, nb);
+    if (vec) hipLaunchKernelGGL(k_scan_down<true>, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, few, out, total);
+    else hipLaunchKernelGGL(k_scan_down<false>, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, few, out, total);
     PPMG_HIP(hipGetLastError());
     return 0;
 }
@@ -224,8 +239,8 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_reduce_u8(const uint32_t* _
 }
 
 __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_down_u8(const uint32_t* __restrict__ in, int64_t n,
-                                                             const int64_t* __restrict__ offs, int* __restrict__ out,
-                                                             int64_t total_out) {
+                                                             const int64_t* __restrict__ sums, bool few,
+                                                             int* __restrict__ out, int64_t total_out) {
     __shared__ int64_t sh[SCAN_BLOCK / 64 + 1];
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     int c[SCAN_ITEMS];
@@ -234,8 +249,9 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_down_u8(const uint32_t* __r
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) sum += c[i];
     int64_t excl;
+    const int64_t prefix = block_prefix(sums, few, sh);
     block_exclusive_scan(sum, sh, excl);
-    int run = (int)(offs[blockIdx.x] + excl);
+    int run = (int)(prefix + excl);
     int o[SCAN_ITEMS];
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i) {
@@ -263,8 +279,9 @@ static int exclusive_scan_u8(const uint32_t* in, int64_t n, int* out, DevBuf& tm
     if (tmp.ensure(sizeof(int64_t) * (size_t)nb)) return PPMG_ERROR_FATAL;
     int64_t* sums = tmp.as<int64_t>();
     hipLaunchKernelGGL(k_scan_reduce_u8, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SUMS_THREADS), 0, s, sums, nb);
-    hipLaunchKernelGGL(k_scan_down_u8, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, out, total);
+    const bool few = nb <= FEW_SUMS;
+    if (!few) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SUMS_THREADS), 0, s, sums, nb);
+    hipLaunchKernelGGL(k_scan_down_u8, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, few, out, total);
     PPMG_HIP(hipGetLastError());
     return 0;
 }
