@@ -8,8 +8,8 @@
 // binning (permutation, cell heads) is reused.
 //
 // Layout and lane mapping as the M2P tile: a workgroup (4 wavefronts, 16
-// rows of 16 lanes) owns 13 x 16 cells in x,y and marches a z chunk; an LDS
-// ring holds 4 planes of g (16 x 19 nodes, component-major).  Lane ex of row
+// rows of 16 lanes or 8 of 32) owns 13 x 16 or 29 x 8 cells in x,y and marches
+// a z chunk; an LDS ring holds 4 planes of g (component-major).  Lane ex of row
 // `row` reads the 4x4 (y,z) column of node column tx0-1+ex and contracts it,
 // for the particles of lanes ex+1, ex, ex-1, ex-2 (k = 0..3), three ways:
 //   C0_k = sum wy wz g,   Cy_k = sum dwy wz g,   Cz_k = sum wy dwz g
@@ -26,11 +26,26 @@
 
 namespace ppmg {
 
-constexpr int A3_TX = 13;
-constexpr int A3_TY = 16;
-constexpr int A3_RY = A3_TY + 3;
-constexpr int A3_PL = A3_RY * 16;
-constexpr int A3_THREADS = 16 * A3_TY;
+constexpr int A3_THREADS = 256;
+
+// Tile geometry with W lanes per row (16 or 32).
+template <int W> struct A3Geom {
+    static constexpr int TX = W - 3, TY = A3_THREADS / W;   // owned cells
+    static constexpr int RY = TY + 3, PL = RY * W;          // node rows and slots of a ring plane
+};
+
+// Weight of the particle whose x offset k is this lane's column: v of lane
+// ex + 1 - k; prev: the value for k - 1 (32-lane rows shift it once more).
+template <int W, typename T>
+__device__ __forceinline__ T from_offset(int k, T v, T prev) {
+    if (k == 3 && W == 32) return lane_from<-1, W>(prev);
+    return k == 0 ? lane_from<1, W>(v) : k == 1 ? v : k == 2 ? lane_from<-1, W>(v) : lane_from<-2, W>(v);
+}
+// Sum back to its particle: that of lane P - 1 + k.
+template <int W, typename T>
+__device__ __forceinline__ T to_offset(int k, T v) {
+    return k == 0 ? lane_from<-1, W>(v) : k == 1 ? v : k == 2 ? lane_from<1, W>(v) : lane_from<2, W>(v);
+}
 
 // Cotangent of stencil node u (unwrapped, periodic axes) when the forward
 // wrote a stored box: the forward's value at a stored node real on every axis
@@ -83,15 +98,16 @@ __device__ __forceinline__ double box_cotangent(const DevMesh& m, const FieldGeo
 // through box_cotangent.  Otherwise it is the compact layout.
 // TABLE: the forward's binning is a slot table (byte counts, particle r of
 // cell c at bt.table[r * ncells + c]) instead of heads and a permutation.
-template <int LDA, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE>
+template <int W, int LDA, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE>
 __global__ void __launch_bounds__(A3_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
 k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm, BinTable bt,
           const PosT* __restrict__ xp, const ValT* __restrict__ up, const ValT* __restrict__ g, FieldGeom fg,
           ValT* __restrict__ grad_u, ValT* __restrict__ grad_x, int lda, int c0, int tz, WorkList items,
           int accumulate_x) {
+    constexpr int A3_TX = A3Geom<W>::TX, A3_TY = A3Geom<W>::TY, A3_RY = A3Geom<W>::RY, A3_PL = A3Geom<W>::PL;
     __shared__ ValT ring[4 * LDA * A3_PL];   // [plane][c][ry][nx]
     const int tid = threadIdx.x;
-    const int ex = tid & 15, row = tid >> 4;
+    const int ex = tid & (W - 1), row = tid / W;
     const int Nx = m.N[0], Ny = m.N[1], Nz = m.N[2];
     const int ntx = (Nx + A3_TX - 1) / A3_TX, nty = (Ny + A3_TY - 1) / A3_TY;
     int tx0, ty0, z0, z1;
@@ -110,7 +126,7 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     // copy) and take the same staged fetch as the compact layout.  Other
     // planes of a BOXED tile are read through box_cotangent between the
     // barriers.
-    const bool box_pipe = BOXED && tx0 - 1 > 0 && tx0 + 14 < Nx && ty0 - 1 > 0 && ty0 + A3_RY - 2 < Ny &&
+    const bool box_pipe = BOXED && tx0 - 1 > 0 && tx0 + W - 2 < Nx && ty0 - 1 > 0 && ty0 + A3_RY - 2 < Ny &&
                           (int64_t)fg.ext[0] * fg.ext[1] * fg.lda * (int64_t)sizeof(ValT) < ((int64_t)1 << 31);
     auto staged = [&](int n) { return !BOXED || (box_pipe && n > 0 && n < Nz); };
     ValT stage[NN][LDA];
@@ -121,7 +137,7 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 #pragma unroll
     for (int j = 0; j < NN; ++j) {
         const int node = tid + j * A3_THREADS;
-        const int nx = node & 15, ry = node >> 4;
+        const int nx = node & (W - 1), ry = node / W;
         if constexpr (BOXED) {
             soff[j] = box_pipe ? (unsigned)((((int64_t)(ty0 - 1 + ry - fg.lo[1]) * fg.ext[0] + (tx0 - 1 + nx - fg.lo[0])) *
                                                  fg.lda + c0) * (int64_t)sizeof(ValT))
@@ -159,20 +175,20 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     // (tiles on the periodic faces) every node goes through box_cotangent.
     auto fetch_store_boxed = [&](int n) {
         ValT* dst = ring + (n & 3) * (LDA * A3_PL);
-        const bool inner = tx0 - 1 > 0 && tx0 + 14 < m.N[0] && ty0 - 1 > 0 && ty0 + A3_RY - 2 < m.N[1] && n > 0 &&
+        const bool inner = tx0 - 1 > 0 && tx0 + W - 2 < m.N[0] && ty0 - 1 > 0 && ty0 + A3_RY - 2 < m.N[1] && n > 0 &&
                            n < m.N[2];
         if (inner) {
             const ValT* src = g + (((int64_t)(n - fg.lo[2]) * fg.ext[1] + (ty0 - 1 - fg.lo[1])) * fg.ext[0] +
                                    (tx0 - 1 - fg.lo[0])) * fg.lda + c0;
             for (int i = tid; i < A3_PL * LDA; i += A3_THREADS) {
                 const int node = i / LDA;
-                dst[(i % LDA) * A3_PL + node] = src[((int64_t)(node >> 4) * fg.ext[0] + (node & 15)) * fg.lda + i % LDA];
+                dst[(i % LDA) * A3_PL + node] = src[((int64_t)(node / W) * fg.ext[0] + (node & (W - 1))) * fg.lda + i % LDA];
             }
             return;
         }
         for (int i = tid; i < A3_PL * LDA; i += A3_THREADS) {
             const int node = i / LDA;
-            const int u[3] = {tx0 - 1 + (node & 15), ty0 - 1 + (node >> 4), n};
+            const int u[3] = {tx0 - 1 + (node & (W - 1)), ty0 - 1 + node / W, n};
             dst[(i % LDA) * A3_PL + node] = (ValT)box_cotangent<ValT>(m, fg, g, c0 + i % LDA, u);
         }
     };
@@ -303,23 +319,23 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
 #pragma unroll
             for (int c = 0; c < LDA; ++c) gu[c] = AccT(0);
             AccT gx0 = AccT(0), gx1 = AccT(0), gx2 = AccT(0);
+            AccT a[4], da[4], b[4], db[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                AccT a[4], da[4], b[4], db[4];
 #pragma unroll
                 for (int o = 0; o < 4; ++o) {
-                    a[o] = k == 0 ? row_shl<1>(wy[o]) : k == 1 ? wy[o] : k == 2 ? row_shr<1>(wy[o]) : row_shr<2>(wy[o]);
-                    da[o] = k == 0 ? row_shl<1>(dy[o]) : k == 1 ? dy[o] : k == 2 ? row_shr<1>(dy[o]) : row_shr<2>(dy[o]);
-                    b[o] = k == 0 ? row_shl<1>(wz[o]) : k == 1 ? wz[o] : k == 2 ? row_shr<1>(wz[o]) : row_shr<2>(wz[o]);
-                    db[o] = k == 0 ? row_shl<1>(dz[o]) : k == 1 ? dz[o] : k == 2 ? row_shr<1>(dz[o]) : row_shr<2>(dz[o]);
+                    a[o] = from_offset<W>(k, wy[o], a[o]);
+                    da[o] = from_offset<W>(k, dy[o], da[o]);
+                    b[o] = from_offset<W>(k, wz[o], b[o]);
+                    db[o] = from_offset<W>(k, dz[o], db[o]);
                 }
 #pragma unroll
                 for (int c = 0; c < LDA; ++c) {
                     AccT C0 = AccT(0), Cy = AccT(0), Cz = AccT(0);
 #pragma unroll
                     for (int oz = 0; oz < 4; ++oz) {
-                        const ValT* f = ring + ((cz - 1 + oz) & 3) * (LDA * A3_PL) + c * A3_PL + row * 16 + ex;
-                        const AccT g0 = (AccT)f[0], g1 = (AccT)f[16], g2 = (AccT)f[32], g3 = (AccT)f[48];
+                        const ValT* f = ring + ((cz - 1 + oz) & 3) * (LDA * A3_PL) + c * A3_PL + row * W + ex;
+                        const AccT g0 = (AccT)f[0], g1 = (AccT)f[W], g2 = (AccT)f[2 * W], g3 = (AccT)f[3 * W];
                         AccT t = a[0] * g0;
                         t += a[1] * g1;
                         t += a[2] * g2;
@@ -333,9 +349,9 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
                         Cy += b[oz] * td;
                     }
                     // back to the particle: the sums of lane P-1+k
-                    const AccT s0 = k == 0 ? row_shr<1>(C0) : k == 1 ? C0 : k == 2 ? row_shl<1>(C0) : row_shl<2>(C0);
-                    const AccT sy = k == 0 ? row_shr<1>(Cy) : k == 1 ? Cy : k == 2 ? row_shl<1>(Cy) : row_shl<2>(Cy);
-                    const AccT sz = k == 0 ? row_shr<1>(Cz) : k == 1 ? Cz : k == 2 ? row_shl<1>(Cz) : row_shl<2>(Cz);
+                    const AccT s0 = to_offset<W>(k, C0);
+                    const AccT sy = to_offset<W>(k, Cy);
+                    const AccT sz = to_offset<W>(k, Cz);
                     gu[c] += wx[k] * s0;
                     gx0 += u[c] * dx[k] * s0;
                     gx1 += u[c] * wx[k] * sy;
@@ -380,22 +396,36 @@ k_a3_tile(DevMesh m, const int* __restrict__ start, const int* __restrict__ perm
     }
 }
 
-template <int LL, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE = false>
-static int launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
-                           const FieldGeom& fg, ValT* gu, ValT* gx, int lda, int c0, int acc, hipStream_t s) {
-    static const Residency res = residency(k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>, A3_THREADS);
-    const int tx = (m.N[0] + A3_TX - 1) / A3_TX, ty = (m.N[1] + A3_TY - 1) / A3_TY;
+template <int W, int LL, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE>
+static int launch_a3_rows(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
+                          const FieldGeom& fg, ValT* gu, ValT* gx, int lda, int c0, int acc, hipStream_t s) {
+    auto kernel = k_a3_tile<W, LL, PosT, ValT, AccT, BOXED, TABLE>;
+    constexpr int TX = A3Geom<W>::TX, TY = A3Geom<W>::TY;
+    static const Residency res = residency(kernel, A3_THREADS);
+    const int tx = (m.N[0] + TX - 1) / TX, ty = (m.N[1] + TY - 1) / TY;
     // a step is long here: a chunk's three extra plane loads weigh little
     const int tz = pick_chunk((int64_t)tx * ty, m.N[2], res, 0.3, 0.3);
     unsigned grid = (unsigned)((int64_t)tx * ty * ((m.N[2] + tz - 1) / tz));
     WorkList items;   // crowded cells: workgroups from a work list
     if (!TABLE && work_list_applies(plan, tz) &&
-        build_work(plan, m, {tx, ty, A3_TX, A3_TY, 0, 0, A3_TX, A3_TY, m.N[2], 0}, res.slots(), s, &items, &grid))
+        build_work(plan, m, {tx, ty, TX, TY, 0, 0, TX, TY, m.N[2], 0}, res.slots(), s, &items, &grid))
         return PPMG_ERROR_FATAL;
     const BinTable bt{plan->count.as<uint32_t>(), plan->table.as<int>(), plan->ncells};
-    hipLaunchKernelGGL((k_a3_tile<LL, PosT, ValT, AccT, BOXED, TABLE>), dim3(grid), dim3(A3_THREADS), 0, s, m,
-                       plan->start.as<int>(), tile_perm(plan), bt, xp, up, g, fg, gu, gx, lda, c0, tz, items, acc);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(A3_THREADS), 0, s, m, plan->start.as<int>(), tile_perm(plan), bt, xp,
+                       up, g, fg, gu, gx, lda, c0, tz, items, acc);
     return 0;
+}
+
+// Rows of 32 lanes where they cover the mesh with fewer lanes, as in the
+// gather (75% of the issue slots at 512^3).  FP64, lda 3: 512^3 9.46 -> 8.85
+// ms, 200^3 635 -> 575 us, stored boxes 200^3 775 -> 745 us, 58^3 33 -> 29 us.
+template <int LL, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE = false>
+static int launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,
+                           const FieldGeom& fg, ValT* gu, ValT* gx, int lda, int c0, int acc, hipStream_t s) {
+    constexpr int T16 = A3Geom<16>::TX, T32 = A3Geom<32>::TX;
+    if ((m.N[0] + T32 - 1) / T32 * 32 < (m.N[0] + T16 - 1) / T16 * 16)
+        return launch_a3_rows<32, LL, PosT, ValT, AccT, BOXED, TABLE>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
+    return launch_a3_rows<16, LL, PosT, ValT, AccT, BOXED, TABLE>(plan, m, xp, up, g, fg, gu, gx, lda, c0, acc, s);
 }
 
 // The compact layout of every axis, or a stored box on some axis.

@@ -246,3 +246,36 @@ def test_slot_table_on_open_axes(core, monkeypatch, shape, bc, kernel, prec):
     monkeypatch.delenv("PPMG_NO_TABLE")
     for a, b in zip(got, _general(monkeypatch, run)):
         assert ((a - b).abs().max() / b.abs().max()).item() < (1e-13 if prec == F64 else 2e-5)
+
+
+@pytest.mark.parametrize("nx", [27, 29, 55, 58])
+@pytest.mark.parametrize("ghost", [0, 2])
+@pytest.mark.parametrize("prec", [F64, F32C])
+def test_adjoint_wide_rows(core, monkeypatch, nx, ghost, prec):
+    """Meshes whose M'4 adjoint takes rows of 32 lanes, on the slot table and on
+    heads (bitwise the same), and against the general path (64 terms: 1e-13 of
+    the maximum in FP64; FP32c 2e-5)."""
+    shape = (nx, 19, 10)
+    rng = np.random.default_rng(nx + ghost)
+    x = np.concatenate([rng.uniform(0, 0.999, (nx * 190, 3)), 0.5 + 0.03 * rng.uniform(0, 1, (6, 3))])
+    side = np.array(shape) / nx
+    mesh = core.Mesh(3, [n + 1 for n in shape], [0.0] * 3, list(side))
+    vdt = core.VAL_DTYPE[prec]
+    xd = torch.as_tensor(x * side).to(core.POS_DTYPE[prec]).cuda()
+    for lda in (1, 3, 4):
+        u = torch.as_tensor(rng.normal(size=(len(x), lda))).to(vdt).cuda()
+        fs = mesh.padded_shape(lda, [ghost] * 3) if ghost else mesh.compact_shape(lda)
+        g = torch.as_tensor(rng.normal(size=fs)).to(vdt).cuda()
+
+        def run():
+            f = torch.empty_like(g)
+            plan = core.p2m(mesh, xd, u, f, [-ghost] * 3, MP4, prec)
+            return core.p2m_adjoint(mesh, xd, u, g, [-ghost] * 3, plan, MP4, prec)
+
+        got = run()
+        monkeypatch.setenv("PPMG_NO_TABLE", "1")
+        for a, b in zip(run(), got):
+            assert torch.equal(a, b)
+        monkeypatch.delenv("PPMG_NO_TABLE")
+        for a, b in zip(got, _general(monkeypatch, run)):
+            assert ((a - b).abs().max() / b.abs().max()).item() < (1e-13 if prec == F64 else 2e-5)
