@@ -398,12 +398,14 @@ int ppmg_m2p(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, const void
     const bool tiled3 = !force_general && m2p3d_fast_applicable(m, kernel, fg);
     const bool tiled2 = !force_general && !tiled3 && m2p2d_fast_applicable(m, kernel, fg);
     if (tiled3 || tiled2) {
+        // the binning below replaces the forward's, also where a particle
+        // outside the sub leaves the gather to the general path
+        plan->have_forward = false;
         int rc = tiled3 ? m2p3d_fast(plan, m, kernel, prec, np, xp, fg, field->data, up, prebinned, s)
                         : m2p2d_fast(plan, m, kernel, prec, np, xp, fg, field->data, up, s);
         if (rc < 0) return g_status.info;
         if (rc == 0) {
             mark(plan, s);
-            plan->have_forward = false;   // the binning now describes these particles
             return 0;
         }
     }

@@ -1,0 +1,66 @@
+"""What a plan answers after a call that failed, or that replaced its binning."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+MP4, BSP2 = 2, 1
+
+
+@pytest.fixture(scope="module")
+def core():
+    from ppm_legacy_amd import core as c
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    return c
+
+
+def _forward(core, dim, kernel, N=12, n=700):
+    """P2M of unordered particles into a stored box on a new plan (a slot
+    table): mesh, positions, strengths, field, plan."""
+    rng = np.random.default_rng(dim + 10 * kernel)
+    mesh = core.Mesh(dim, N + 1)
+    x = torch.as_tensor(rng.uniform(0, 1, (n, dim))).cuda()
+    u = torch.as_tensor(rng.normal(size=(n, 2))).cuda()
+    f = torch.zeros(mesh.padded_shape(2, [2] * dim), dtype=torch.float64, device="cuda")
+    return mesh, x, u, f, core.p2m(mesh, x, u, f, [-2] * dim, kernel)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("kernel", [MP4, BSP2])
+@pytest.mark.parametrize("where", ["ghost", "far"])
+def test_adjoint_refused_after_m2p_with_particle_outside(core, dim, kernel, where):
+    """M2P of as many particles, one of them outside the sub (on a ghost node,
+    where the general path answers, or beyond the stored box, where it fails):
+    the plan no longer holds the forward's binning, and the adjoint says so
+    before any launch.  A new forward makes the plan good again."""
+    from ppm_legacy_amd import _lib
+    mesh, x, u, f, plan = _forward(core, dim, kernel)
+    want = core.p2m_adjoint(mesh, x, u, f, [-2] * dim, plan, kernel)
+    y = x.clone()
+    y[5, 0] = 1.0 + 0.5 / 12 if where == "ghost" else 3.0
+    out = torch.empty_like(u)
+    if where == "ghost":
+        core.m2p(mesh, y, f, [-2] * dim, out, kernel, plan=plan)
+    else:
+        with pytest.raises(_lib.PpmgError):
+            core.m2p(mesh, y, f, [-2] * dim, out, kernel, plan=plan)
+    with pytest.raises(_lib.PpmgError) as e:
+        core.p2m_adjoint(mesh, x, u, f, [-2] * dim, plan, kernel)
+    assert e.value.code == _lib.ERR_ARGUMENT
+    g = f.clone()
+    core.p2m(mesh, x, u, f, [-2] * dim, kernel, plan=plan)
+    assert torch.equal(f, g)
+    got = core.p2m_adjoint(mesh, x, u, f, [-2] * dim, plan, kernel)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_adjoint_after_m2p_without_binning(core, monkeypatch):
+    """M2P on the general path bins nothing: the forward's binning stays."""
+    mesh, x, u, f, plan = _forward(core, 3, MP4)
+    want = core.p2m_adjoint(mesh, x, u, f, [-2] * 3, plan)
+    monkeypatch.setenv("PPMG_GENERAL", "1")
+    core.m2p(mesh, x, f, [-2] * 3, torch.empty_like(u), plan=plan)
+    monkeypatch.delenv("PPMG_GENERAL")
+    got = core.p2m_adjoint(mesh, x, u, f, [-2] * 3, plan)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
