@@ -66,6 +66,7 @@ int DevBuf::ensure(size_t n) {
     }
     hipError_t e = injected_alloc_failure(want) ? hipErrorOutOfMemory : hipMalloc(&p, want);
     if (e != hipSuccess) {
+        (void)hipGetLastError();   // reported here, not again by the next call's launch check
         p = nullptr;
         bytes = 0;
         set_error(PPMG_ERROR_FATAL, PPMG_ERR_ALLOC, std::string("hipMalloc of device scratch failed: ") + hipGetErrorString(e));

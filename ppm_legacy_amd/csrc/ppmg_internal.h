@@ -388,10 +388,13 @@ void set_error(int severity, int code, const std::string& msg);
 void clear_error();
 int debug_level();
 
+// HIP keeps the error of a failed call until it is asked for: it is taken here,
+// with the failure it belongs to.
 #define PPMG_HIP(call)                                                                   \
     do {                                                                                 \
         hipError_t e_ = (call);                                                          \
         if (e_ != hipSuccess) {                                                          \
+            (void)hipGetLastError();                                                     \
             ::ppmg::set_error(PPMG_ERROR_FATAL, PPMG_ERR_DEVICE,                         \
                               std::string(#call) + ": " + hipGetErrorString(e_));        \
             return PPMG_ERROR_FATAL;                                                     \

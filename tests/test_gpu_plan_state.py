@@ -64,3 +64,54 @@ def test_adjoint_after_m2p_without_binning(core, monkeypatch):
     monkeypatch.delenv("PPMG_GENERAL")
     got = core.p2m_adjoint(mesh, x, u, f, [-2] * 3, plan)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _refused(core, plan):
+    """A call on `plan` whose scratch no device holds (its lda is 2^28, of
+    which nothing is read: the allocation comes before any launch)."""
+    import ctypes
+
+    from ppm_legacy_amd import _lib
+    mesh = core.Mesh(3, 9)
+    field = torch.zeros(mesh.padded_shape(1, [2, 2, 2]), dtype=torch.float64, device="cuda")
+    f = core.field_desc(mesh, field, [-2] * 3)
+    f.lda = 1 << 28
+    g = (ctypes.c_int * 3)(2, 2, 2)
+    _lib.check(_lib.lib().ppmg_map_field_ghost(mesh.ref(), core.PREC_F64, ctypes.byref(f), g, _lib.MAP_GHOST_GET,
+                                               plan.handle, None))
+
+
+def test_refused_allocation_is_reported_once(core):
+    """A device allocation that HIP itself refuses fails its own call and
+    leaves nothing behind that a later call would report."""
+    from ppm_legacy_amd import _lib
+    plan = core.Plan()
+    with pytest.raises(_lib.PpmgError) as e:
+        _refused(core, plan)
+    assert e.value.code == _lib.ERR_ALLOC
+    mesh, x, u, f, plan = _forward(core, 3, MP4)
+    assert abs(f[2:-3, 2:-3, 2:-3].sum().item() - u.sum().item()) < 1e-9 * u.abs().sum().item()
+
+
+def test_graph_plan_retry_after_refused_allocation(core, monkeypatch):
+    """A forward whose scratch HIP refuses gives the pooled plans back and
+    runs again."""
+    from ppm_legacy_amd import autograd
+    mesh, x, u, _, _ = _forward(core, 3, MP4)
+    autograd.release_plans()
+    u.requires_grad_(True)
+    want = autograd.p2m(x, u, mesh)
+    keep = autograd.p2m(x, u, mesh)
+    del keep                                   # its plan is in the pool
+    real, calls = core.p2m, []
+
+    def refusing(mesh_, x_, u_, f_, lo, kernel, prec, plan):
+        calls.append(plan)
+        if len(calls) == 1:
+            autograd._pool.setdefault(0, []).append((core.Plan(), torch.cuda.Event(), 0, 0))
+            _refused(core, plan)
+        return real(mesh_, x_, u_, f_, lo, kernel, prec, plan)
+
+    monkeypatch.setattr(core, "p2m", refusing)
+    got = autograd.p2m(x, u, mesh)
+    assert len(calls) == 2 and torch.equal(got, want)
