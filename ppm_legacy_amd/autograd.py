@@ -25,7 +25,7 @@ from ._lib import ERR_ALLOC, KERNEL_MP4, PREC_F64, PpmgError
 
 POOL_BYTES = 2 << 30
 _lock = threading.RLock()   # a collection inside it may run another plan's __del__
-_pool = {}    # device index -> [(plan, event, stream handle, scratch bytes)]
+_pool = {}    # device index -> [(plan, event, (device, stream) of its last use, scratch bytes)]
 
 
 def release_plans(device=None):
@@ -39,30 +39,38 @@ def release_plans(device=None):
 
 
 class _GraphPlan:
-    """The plan of one forward, back in the pool when the graph lets go of it."""
+    """The plan of one forward, back in the pool when the graph lets go of it.
+    Its scratch and work are those of the device and stream that are current
+    (core._stream), whatever device the tensors are on: the plan is filed under
+    that device, and a stream is told by its device too (every device's default
+    stream has the handle 0)."""
 
-    def __init__(self, device):
-        self.device = device.index if device.index is not None else torch.cuda.current_device()
-        self.event = self.plan = None
-        stream = torch.cuda.current_stream(self.device)
+    def __init__(self):
+        self.device = torch.cuda.current_device()
+        self.plan = self.event = self.last = None
+        stream = torch.cuda.current_stream()
+        here = (self.device, stream.cuda_stream)
         with _lock:
             free = _pool.get(self.device, [])
             # the most recently used one, of this stream where there is one
-            at = next((i for i in reversed(range(len(free))) if free[i][2] == stream.cuda_stream), len(free) - 1)
+            at = next((i for i in reversed(range(len(free))) if free[i][2] == here), len(free) - 1)
             entry = free.pop(at) if free else None
         if entry is None:
-            self.plan, self.event = core.Plan(), torch.cuda.Event()
+            self.plan = core.Plan()
         else:
-            self.plan, self.event = entry[0], entry[1]
-            if entry[2] != stream.cuda_stream:
+            self.plan, self.event, self.last, _ = entry
+            if self.last != here:
                 stream.wait_event(self.event)
         self.used()
 
     def used(self):
         """Marks the current stream's work so far as the plan's last use."""
-        stream = torch.cuda.current_stream(self.device)
+        stream = torch.cuda.current_stream()
+        here = (torch.cuda.current_device(), stream.cuda_stream)
+        if self.event is None or self.last[0] != here[0]:   # an event belongs to one device
+            self.event = torch.cuda.Event()
         self.event.record(stream)
-        self.stream = stream.cuda_stream
+        self.last = here
 
     def __del__(self):
         if self.plan is None or sys.is_finalizing():
@@ -72,7 +80,7 @@ class _GraphPlan:
             with _lock:
                 free = _pool.setdefault(self.device, [])
                 if n + sum(e[3] for e in free) <= POOL_BYTES:
-                    free.append((self.plan, self.event, self.stream, n))
+                    free.append((self.plan, self.event, self.last, n))
                     self.plan = None
             if self.plan is not None:
                 self.plan.close()
@@ -85,7 +93,7 @@ class P2MFunction(torch.autograd.Function):
     def forward(ctx, xp, up, mesh, kernel, prec):
         lda = up.shape[1]
         field = torch.empty(mesh.compact_shape(lda), dtype=core.VAL_DTYPE[prec], device=up.device)
-        held = _GraphPlan(up.device)
+        held = _GraphPlan()
         x, u = xp.contiguous(), up.contiguous()
         try:
             core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)

@@ -1,0 +1,122 @@
+"""The pool of the autograd P2M's plans, with the device taken out: which plan
+a graph gets, what it waits for and what goes back."""
+import types
+
+import pytest
+import torch
+
+from ppm_legacy_amd import _lib, autograd, core
+
+
+class Stream:
+    def __init__(self, device, handle=0):
+        self.device_index, self.cuda_stream, self.waits = device, handle, []
+
+    def wait_event(self, event):
+        self.waits.append(event)
+
+
+class Event:
+    def __init__(self):
+        self.stream = None
+
+    def record(self, stream):
+        # an event belongs to the device it is first recorded on
+        assert self.stream is None or self.stream.device_index == stream.device_index
+        self.stream = stream
+
+    def synchronize(self):
+        pass
+
+
+class Plan:
+    def __init__(self):
+        self.closed = False
+
+    def scratch_bytes(self):
+        return 100
+
+    def close(self):
+        self.closed = True
+
+
+class Device:
+    """Stands for torch.cuda: current device and its current stream."""
+
+    def __init__(self, monkeypatch):
+        self.streams = {d: Stream(d) for d in (0, 1)}
+        self.current = 0
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: self.current)
+        monkeypatch.setattr(torch.cuda, "current_stream",
+                            lambda d=None: self.streams[self.current if d is None else torch.device("cuda", d).index
+                                                        if not isinstance(d, torch.device) else d.index or 0])
+        monkeypatch.setattr(torch.cuda, "Event", Event)
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (1 << 40, 1 << 40), raising=False)
+        monkeypatch.setattr(core, "Plan", Plan)
+
+
+@pytest.fixture
+def dev(monkeypatch):
+    d = Device(monkeypatch)
+    monkeypatch.setattr(autograd, "_pool", {})
+    plans = []
+    monkeypatch.setattr(core, "p2m", lambda mesh, x, u, f, lo, k, p, plan: (plans.append(plan), f.zero_()))
+    monkeypatch.setattr(core, "p2m_adjoint", lambda mesh, x, u, g, lo, plan, k, p, want_u, want_x:
+                        (plans.append(plan), (torch.zeros_like(u), torch.zeros_like(x)))[1])
+    d.plans = plans
+    return d
+
+
+def _graph(mesh=core.Mesh(2, 9)):
+    x = torch.rand((5, 2), dtype=torch.float64).requires_grad_(True)
+    u = torch.ones((5, 1), dtype=torch.float64).requires_grad_(True)
+    return autograd.p2m(x, u, mesh), (x, u)
+
+
+def test_filed_under_the_device_the_work_ran_on(dev, monkeypatch):
+    """The library works on the current device, wherever the tensors are: here
+    on device 0 with device 1 current."""
+    dev.current = 1
+    ctx = types.SimpleNamespace(save_for_backward=lambda *a: None)
+    up = types.SimpleNamespace(shape=(5, 1), device=torch.device("cuda", 0), contiguous=lambda: None)
+    with monkeypatch.context() as m:
+        empty = torch.empty
+        m.setattr(torch, "empty", lambda *a, device=None, **k: empty(*a, **k))
+        autograd.P2MFunction.forward(ctx, up, up, core.Mesh(2, 9), core.L.KERNEL_MP4, core.PREC_F64)
+    del ctx
+    assert not autograd._pool.get(0)
+    (plan, event), = [e[:2] for e in autograd._pool[1]]
+    assert plan is dev.plans[0] and event.stream is dev.streams[1]
+    dev.current = 0
+    f, _ = _graph()
+    assert dev.plans[1] is not plan
+    dev.current = 1
+    g, _ = _graph()
+    assert dev.plans[2] is plan
+
+
+def test_default_streams_of_two_devices_differ(dev):
+    """Both devices' default streams have the handle 0: a plan last used on
+    the other device is waited for."""
+    f, xu = _graph()
+    dev.current = 1
+    torch.autograd.grad(f.sum(), xu)     # the adjoint with device 1 current
+    del f
+    dev.current = 0
+    (_, event), = [e[:2] for e in autograd._pool[0]]
+    assert event.stream is dev.streams[1]
+    g, _ = _graph()
+    assert dev.plans[-1] is dev.plans[0] and dev.streams[0].waits == [event]
+
+
+def test_streams_of_one_device(dev):
+    """Of the pooled plans, the stream's own without a wait; another stream's
+    with one."""
+    f, _ = _graph()
+    del f
+    g, _ = _graph()
+    assert dev.plans[1] is dev.plans[0] and not dev.streams[0].waits
+    del g
+    dev.streams[0] = Stream(0, 7)
+    h, _ = _graph()
+    assert dev.plans[2] is dev.plans[0] and len(dev.streams[0].waits) == 1
