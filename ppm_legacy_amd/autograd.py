@@ -72,6 +72,12 @@ class _GraphPlan:
         self.event.record(stream)
         self.last = here
 
+    def drop(self):
+        """Frees the plan: a failed call may have left work running that no
+        event covers (freeing device memory waits for it)."""
+        plan, self.plan = self.plan, None
+        plan.close()
+
     def __del__(self):
         if self.plan is None or sys.is_finalizing():
             return
@@ -96,13 +102,17 @@ class P2MFunction(torch.autograd.Function):
         held = _GraphPlan()
         x, u = xp.contiguous(), up.contiguous()
         try:
-            core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)
-        except PpmgError as e:
-            if e.code != ERR_ALLOC or not _pool:
-                raise
-            release_plans()
-            core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)
-        held.used()
+            try:
+                core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)
+            except PpmgError as e:
+                if e.code != ERR_ALLOC or not _pool:
+                    raise
+                release_plans()
+                core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)
+            held.used()
+        except BaseException:
+            held.drop()
+            raise
         ctx.save_for_backward(xp, up)
         ctx.mesh, ctx.kernel, ctx.prec, ctx.plan = mesh, kernel, prec, held
         return field
@@ -114,9 +124,11 @@ class P2MFunction(torch.autograd.Function):
         if not (want_x or want_u):
             return None, None, None, None, None
         g = gfield.to(core.VAL_DTYPE[ctx.prec]).contiguous()
-        gu, gx = core.p2m_adjoint(ctx.mesh, xp.contiguous(), up.contiguous(), g, [0] * ctx.mesh.dim, ctx.plan.plan,
-                                  ctx.kernel, ctx.prec, want_u=want_u, want_x=want_x)
-        ctx.plan.used()
+        try:
+            gu, gx = core.p2m_adjoint(ctx.mesh, xp.contiguous(), up.contiguous(), g, [0] * ctx.mesh.dim, ctx.plan.plan,
+                                      ctx.kernel, ctx.prec, want_u=want_u, want_x=want_x)
+        finally:
+            ctx.plan.used()   # a failed call's launches too
         if gx is not None:
             gx = gx.to(xp.dtype)
         return gx, gu, None, None, None

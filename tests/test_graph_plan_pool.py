@@ -120,3 +120,33 @@ def test_streams_of_one_device(dev):
     dev.streams[0] = Stream(0, 7)
     h, _ = _graph()
     assert dev.plans[2] is dev.plans[0] and len(dev.streams[0].waits) == 1
+
+
+def test_plan_of_a_failed_forward_is_not_pooled(dev, monkeypatch):
+    """What a failed call has left running is not covered by the plan's event."""
+    plans = []
+
+    def failing(mesh, x, u, f, lo, k, p, plan):
+        plans.append(plan)
+        raise _lib.PpmgError(-1, _lib.ERR_PART_UNASS, "particles lie in no sub")
+
+    monkeypatch.setattr(core, "p2m", failing)
+    with pytest.raises(_lib.PpmgError):
+        _graph()
+    assert plans[0].closed and not autograd._pool.get(0)
+
+
+def test_failed_backward_is_covered(dev, monkeypatch):
+    """The event covers what a failed adjoint launched."""
+    f, xu = _graph()
+    other = Stream(0, 9)
+
+    def failing(*a, **k):
+        dev.streams[0] = other
+        raise _lib.PpmgError(-1, _lib.ERR_DEVICE, "failed")
+
+    monkeypatch.setattr(core, "p2m_adjoint", failing)
+    with pytest.raises(_lib.PpmgError):
+        torch.autograd.grad(f.sum(), xu)
+    del f
+    assert autograd._pool[0][0][1].stream is other
