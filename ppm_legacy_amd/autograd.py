@@ -12,8 +12,12 @@ A plan's scratch is a dozen device allocations, which an optimisation loop
 would make and free in every step (2.0 of 2.5 ms at 128^3, lda 3, on an
 MI355X).  A graph's plan therefore goes back to a pool when the graph is
 freed, and the next forward takes it from there, ordered after its last use
-by an event.  The pool keeps at most POOL_BYTES of scratch per device;
-release_plans() empties it, and so does a forward that runs out of memory.
+by an event.  The pool's memory is outside PyTorch's allocator, so it is kept
+small and given back early: at most POOL_BYTES of scratch per device (a plan
+over that, from about 390^3 cells on, is freed with its graph and made anew by
+the next forward), none where less than SPARE_BYTES of the device is free when
+a graph is freed, all of it when a forward or backward here runs out of memory,
+and on release_plans(), for a client that is about to take nearly all there is.
 """
 import sys
 import threading
@@ -24,6 +28,7 @@ from . import core
 from ._lib import ERR_ALLOC, KERNEL_MP4, PREC_F64, PpmgError
 
 POOL_BYTES = 2 << 30
+SPARE_BYTES = 16 << 30
 _lock = threading.RLock()   # a collection inside it may run another plan's __del__
 _pool = {}    # device index -> [(plan, event, (device, stream) of its last use, scratch bytes)]
 
@@ -36,6 +41,17 @@ def release_plans(device=None):
     for plan, event, _, _ in entries:
         event.synchronize()
         plan.close()
+
+
+def _with_retry(call):
+    """call(), again after giving the pool back if it runs out of memory."""
+    try:
+        return call()
+    except (PpmgError, torch.OutOfMemoryError) as e:
+        if (isinstance(e, PpmgError) and e.code != ERR_ALLOC) or not any(_pool.values()):
+            raise
+    release_plans()
+    return call()
 
 
 class _GraphPlan:
@@ -82,6 +98,10 @@ class _GraphPlan:
         if self.plan is None or sys.is_finalizing():
             return
         try:
+            if torch.cuda.mem_get_info(self.device)[0] < SPARE_BYTES:   # (3 us)
+                release_plans(self.device)
+                self.drop()
+                return
             n = self.plan.scratch_bytes()
             with _lock:
                 free = _pool.setdefault(self.device, [])
@@ -89,7 +109,7 @@ class _GraphPlan:
                     free.append((self.plan, self.event, self.last, n))
                     self.plan = None
             if self.plan is not None:
-                self.plan.close()
+                self.drop()
         except Exception:
             pass
 
@@ -98,17 +118,11 @@ class P2MFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, xp, up, mesh, kernel, prec):
         lda = up.shape[1]
-        field = torch.empty(mesh.compact_shape(lda), dtype=core.VAL_DTYPE[prec], device=up.device)
+        field = _with_retry(lambda: torch.empty(mesh.compact_shape(lda), dtype=core.VAL_DTYPE[prec], device=up.device))
         held = _GraphPlan()
-        x, u = xp.contiguous(), up.contiguous()
         try:
-            try:
-                core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)
-            except PpmgError as e:
-                if e.code != ERR_ALLOC or not _pool:
-                    raise
-                release_plans()
-                core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan)
+            x, u = _with_retry(lambda: (xp.contiguous(), up.contiguous()))
+            _with_retry(lambda: core.p2m(mesh, x, u, field, [0] * mesh.dim, kernel, prec, held.plan))
             held.used()
         except BaseException:
             held.drop()
@@ -123,14 +137,17 @@ class P2MFunction(torch.autograd.Function):
         want_x, want_u = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (want_x or want_u):
             return None, None, None, None, None
-        g = gfield.to(core.VAL_DTYPE[ctx.prec]).contiguous()
+
+        def adjoint():
+            g = gfield.to(core.VAL_DTYPE[ctx.prec]).contiguous()
+            gu, gx = core.p2m_adjoint(ctx.mesh, xp.contiguous(), up.contiguous(), g, [0] * ctx.mesh.dim,
+                                      ctx.plan.plan, ctx.kernel, ctx.prec, want_u=want_u, want_x=want_x)
+            return gu, gx if gx is None else gx.to(xp.dtype)
+
         try:
-            gu, gx = core.p2m_adjoint(ctx.mesh, xp.contiguous(), up.contiguous(), g, [0] * ctx.mesh.dim, ctx.plan.plan,
-                                      ctx.kernel, ctx.prec, want_u=want_u, want_x=want_x)
+            gu, gx = _with_retry(adjoint)
         finally:
             ctx.plan.used()   # a failed call's launches too
-        if gx is not None:
-            gx = gx.to(xp.dtype)
         return gx, gu, None, None, None
 
 

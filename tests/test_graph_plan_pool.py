@@ -150,3 +150,61 @@ def test_failed_backward_is_covered(dev, monkeypatch):
         torch.autograd.grad(f.sum(), xu)
     del f
     assert autograd._pool[0][0][1].stream is other
+
+
+def _pooled(dev):
+    """Two plans in device 0's pool."""
+    f, _ = _graph()
+    g, _ = _graph()
+    del f, g
+    entries = list(autograd._pool[0])
+    assert len(entries) == 2
+    return [e[0] for e in entries]
+
+
+def _once(real, error):
+    """real, the first call of which raises error."""
+    left = [error]
+
+    def call(*a, **k):
+        if left:
+            raise left.pop()
+        return real(*a, **k)
+    return call
+
+
+def test_given_back_when_the_field_does_not_fit(dev, monkeypatch):
+    plans = _pooled(dev)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", _once(torch.empty, torch.OutOfMemoryError("out of memory")))
+        f, _ = _graph()
+    assert f.shape == (8, 8, 1) and all(p.closed for p in plans)
+
+
+@pytest.mark.parametrize("error", [torch.OutOfMemoryError("out of memory"),
+                                   _lib.PpmgError(-1, _lib.ERR_ALLOC, "hipMalloc failed")])
+def test_given_back_when_the_backward_does_not_fit(dev, monkeypatch, error):
+    f, xu = _graph()
+    plans = _pooled(dev)
+    monkeypatch.setattr(core, "p2m_adjoint", _once(core.p2m_adjoint, error))
+    torch.autograd.grad(f.sum(), xu)
+    assert all(p.closed for p in plans) and not dev.plans[-1].closed
+
+
+@pytest.mark.parametrize("error", [torch.OutOfMemoryError("out of memory"),
+                                   _lib.PpmgError(-1, _lib.ERR_ALLOC, "hipMalloc failed")])
+def test_out_of_memory_with_nothing_to_give_back(dev, monkeypatch, error):
+    monkeypatch.setattr(core, "p2m", _once(core.p2m, error))
+    with pytest.raises(type(error)):
+        _graph()
+
+
+def test_nothing_pooled_where_memory_is_short(dev, monkeypatch):
+    """With less than SPARE_BYTES free, a graph's plan is freed with it, and
+    so are those in the pool."""
+    f, _ = _graph()
+    plans = _pooled(dev)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (autograd.SPARE_BYTES - 1, 1 << 40))
+    last = f.grad_fn.plan.plan
+    del f
+    assert last.closed and all(p.closed for p in plans) and not autograd._pool.get(0)
