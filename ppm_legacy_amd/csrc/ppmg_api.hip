@@ -41,6 +41,17 @@ static bool injected_alloc_failure(size_t n) {
     return n > (size_t)std::strtoull(e, nullptr, 10);
 }
 
+// A refused allocation's HIP error is taken here, not left for the next call's
+// launch check.
+static hipError_t device_malloc(void** p, size_t n) {
+    const hipError_t e = injected_alloc_failure(n) ? hipErrorOutOfMemory : hipMalloc(p, n);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 static thread_local Arena* g_arena = nullptr;
 void bind_arena(Arena* a) { g_arena = a; }
 bool arena_bound() { return g_arena != nullptr; }
@@ -64,16 +75,21 @@ int DevBuf::ensure(size_t n) {
         borrowed = true;
         return 0;
     }
-    hipError_t e = injected_alloc_failure(want) ? hipErrorOutOfMemory : hipMalloc(&p, want);
+    const hipError_t e = device_malloc(&p, want);
     if (e != hipSuccess) {
-        (void)hipGetLastError();   // reported here, not again by the next call's launch check
-        p = nullptr;
-        bytes = 0;
         set_error(PPMG_ERROR_FATAL, PPMG_ERR_ALLOC, std::string("hipMalloc of device scratch failed: ") + hipGetErrorString(e));
         return PPMG_ERROR_FATAL;
     }
     bytes = want;
     return 0;
+}
+bool DevBuf::try_ensure(size_t n) {
+    if (g_arena || (n <= bytes && p)) return ensure(n) == 0;
+    release();
+    const size_t want = n < 256 ? 256 : n;
+    if (device_malloc(&p, want) != hipSuccess) return false;
+    bytes = want;
+    return true;
 }
 void DevBuf::release() {
     if (p && !borrowed) (void)hipFree(p);

@@ -407,6 +407,7 @@ struct DevBuf {
     size_t bytes = 0;
     bool borrowed = false;   // carved from a bound Arena: never freed
     int ensure(size_t n);
+    bool try_ensure(size_t n);   // for scratch a call can do without: no error is set where it is refused
     void release();
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };

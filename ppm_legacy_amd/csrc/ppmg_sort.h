@@ -142,7 +142,7 @@ struct WorkList {
 bool work_list_applies(const ppmg_plan* plan, int tz);
 // The pieces of all tile columns, in the plan's scratch, and their number
 // (slots: resident workgroups of the kernel); the list stays empty where it
-// would take too much scratch.
+// would take too much scratch, or where the scratch is refused.
 int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, int slots, hipStream_t s, WorkList* list,
                unsigned* nitems);
 // This workgroup's tile column and planes [z0, z1): from the work list, or

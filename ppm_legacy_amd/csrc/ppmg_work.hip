@@ -113,8 +113,10 @@ int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, int slots
     const int64_t nid = (int64_t)w.ntx * w.nty * nseg, cap = nid * WK_SEG;
     // more pieces than the scratch should hold, or planes than an item's word: no list
     if (nid >= (int64_t)1 << 21 || w.planes >= 1 << 25) return 0;
-    if (plan->work.ensure(sizeof(int2) * (size_t)(WK_CLASSES * cap)) || plan->work_cnt.ensure(sizeof(int) * WK_CLASSES))
-        return PPMG_ERROR_FATAL;
+    // (1 KiB per column segment: 16 MiB at 512^3.)  The grid does without it.
+    if (!plan->work.try_ensure(sizeof(int2) * (size_t)(WK_CLASSES * cap)) ||
+        !plan->work_cnt.try_ensure(sizeof(int) * WK_CLASSES))
+        return 0;
     int* count = plan->work_cnt.as<int>();
     const double load = ((double)w.ntx * w.nty * w.planes + 1.5 * (double)plan->np / ((double)w.tx * w.ty)) / slots;
     // Clustered input (half a particle a cell, four blobs), FP64, lda 3.  The

@@ -115,3 +115,42 @@ def test_graph_plan_retry_after_refused_allocation(core, monkeypatch):
     monkeypatch.setattr(core, "p2m", refusing)
     got = autograd.p2m(x, u, mesh)
     assert len(calls) == 2 and torch.equal(got, want)
+
+
+def _crowded(core, N=128, n=1 << 17):
+    """Particles in an eighth of the mesh per axis, 32 to a cell there."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.rand((n, 3), dtype=torch.float64, device="cuda", generator=g) / 8 + 0.4
+    u = torch.randn((n, 1), dtype=torch.float64, device="cuda", generator=g)
+    mesh = core.Mesh(3, N + 1)
+    return mesh, x, u, torch.empty(mesh.compact_shape(1), dtype=torch.float64, device="cuda")
+
+
+def test_work_list_without_memory(core, monkeypatch):
+    """Crowded input with the work list's scratch refused (all else is there
+    from calls of the general path): deposit, gather and adjoint run without
+    it, bitwise as with it."""
+    mesh, x, u, f = _crowded(core)
+
+    def cycle(plan):
+        core.p2m(mesh, x, u, f, [0] * 3, plan=plan)
+        gu, gx = core.p2m_adjoint(mesh, x, u, f, [0] * 3, plan)
+        out = torch.empty_like(u)
+        core.m2p(mesh, x, f, [0] * 3, out, plan=plan)
+        return f.clone(), gu, gx, out
+
+    want = cycle(core.Plan())
+    plan = core.Plan()
+    monkeypatch.setenv("PPMG_GENERAL", "1")
+    core.p2m(mesh, x, u, f, [0] * 3, plan=plan)
+    core.p2m(mesh, x, u, f, [0] * 3, plan=plan)
+    monkeypatch.delenv("PPMG_GENERAL")
+    before = plan.scratch_bytes()
+    monkeypatch.setenv("PPMG_FAIL_ALLOC_ABOVE", "0")
+    got = cycle(plan)
+    assert plan.scratch_bytes() == before
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    monkeypatch.delenv("PPMG_FAIL_ALLOC_ABOVE")
+    got = cycle(plan)
+    assert plan.scratch_bytes() > before       # the list has its scratch now
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
