@@ -997,18 +997,39 @@ __global__ void __launch_bounds__(256) k_heads(const int* __restrict__ ks, int64
     if (sampled && tid == 0 && ncrowd > 0) atomicAdd(&err[8 + (blockIdx.x / stride & 63)], ncrowd);
 }
 
-// Stable sort of n keys below 2^bits by LSD radix passes: the sorted keys
-// (*sorted_keys, in the plan's scratch), and the permutation (plus vadd) at
-// positions below vmax in vout.
+// Digit width of a sort of keys below nkeys (and its passes).
+static int radix_bits(int64_t nkeys, int* passes) {
+    int bits = 1;
+    while (bits < 31 && ((int64_t)1 << bits) < nkeys) ++bits;
+    const int p8 = (bits + 7) / 8, p9 = (bits + 8) / 9;
+    *passes = p9 < p8 ? p9 : p8;
+    return p9 < p8 ? 9 : 8;
+}
+
+// Scratch of a sort of n keys below nkeys: the pairs twice (16 bytes a key) and
+// the tiles' counts.  False, with nothing kept, where it is refused (the
+// counting path does without).
+static bool radix_scratch(ppmg_plan* plan, int64_t n, int64_t nkeys) {
+    int passes;
+    const int64_t buckets = (int64_t)1 << radix_bits(nkeys, &passes), tile = buckets * RS_ITEMS;
+    const size_t pairs = sizeof(int) * (size_t)n, hist = sizeof(int) * (size_t)(2 * (buckets * ((n + tile - 1) / tile) + 4));
+    DevBuf* bufs[] = {&plan->rkey[0], &plan->rkey[1], &plan->rval[0], &plan->rval[1], &plan->rhist};
+    for (DevBuf* b : bufs)
+        if (!b->try_ensure(b == &plan->rhist ? hist : pairs)) {
+            for (DevBuf* r : bufs) r->release();
+            return false;
+        }
+    return true;
+}
+
+// Stable sort of n keys below 2^bits by LSD radix passes, in the scratch of
+// radix_scratch: the sorted keys (*sorted_keys, in that scratch), and the
+// permutation (plus vadd) at positions below vmax in vout.
 template <int BITS>
 static int radix_sort_bits(ppmg_plan* plan, const int* keys, int64_t n, int passes, int* vout, int vadd, int64_t vmax,
                            hipStream_t s, const int** sorted_keys) {
     using R = Radix<BITS>;
     const int64_t ntiles = (n + R::TILE - 1) / R::TILE;
-    if (plan->rkey[0].ensure(sizeof(int) * (size_t)n) || plan->rkey[1].ensure(sizeof(int) * (size_t)n) ||
-        plan->rval[0].ensure(sizeof(int) * (size_t)n) || plan->rval[1].ensure(sizeof(int) * (size_t)n) ||
-        plan->rhist.ensure(sizeof(int) * (size_t)(2 * (R::BUCKETS * ntiles + 4))))
-        return PPMG_ERROR_FATAL;
     int* hist = plan->rhist.as<int>();
     int* offs = hist + R::BUCKETS * ntiles + 4;   // 16-byte aligned, n + 1 entries
     const int* kin = keys;
@@ -1032,11 +1053,10 @@ static int radix_sort_bits(ppmg_plan* plan, const int* keys, int64_t n, int pass
 
 static int radix_sort(ppmg_plan* plan, const int* keys, int64_t n, int64_t nkeys, int* vout, int vadd, int64_t vmax,
                       hipStream_t s, const int** sorted_keys) {
-    int bits = 1;
-    while (bits < 31 && ((int64_t)1 << bits) < nkeys) ++bits;
-    const int p8 = (bits + 7) / 8, p9 = (bits + 8) / 9;
-    if (p9 < p8) return radix_sort_bits<9>(plan, keys, n, p9, vout, vadd, vmax, s, sorted_keys);
-    return radix_sort_bits<8>(plan, keys, n, p8, vout, vadd, vmax, s, sorted_keys);
+    int passes;
+    if (radix_bits(nkeys, &passes) == 9)
+        return radix_sort_bits<9>(plan, keys, n, passes, vout, vadd, vmax, s, sorted_keys);
+    return radix_sort_bits<8>(plan, keys, n, passes, vout, vadd, vmax, s, sorted_keys);
 }
 
 // Heads of the sorted keys ks, and the plan's crowded-cell estimate from a
@@ -1169,12 +1189,13 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     // 1.04 ms; 2.1M 129 against 173 us, 1.03M 109 against 96); PPMG_RADIX=1
     // forces that path for input not predicted in cell order, PPMG_RADIX=0
     // rules it out (both for tests).  Allocation-free calls keep the counting
-    // path (the sort needs four more int32 per particle).
+    // path (the sort needs four more int32 per particle), and so do calls
+    // whose sort is refused its scratch.
     const char* rx = std::getenv("PPMG_RADIX");
     const bool radix = rx && rx[0] ? rx[0] == '1'
                                    : plan->crowded_cells * 64 > np ||
                                          (np >= FAR_MIN_NP && plan->far_particles * 4 > np);
-    if (!predict_sorted && radix && !arena_bound()) {
+    if (!predict_sorted && radix && !arena_bound() && radix_scratch(plan, np, ncells)) {
         if (sorted_lists()) return PPMG_ERROR_FATAL;
         if (fill_zero(plan->err.p, sizeof(int) * ERR_WORDS, s)) return PPMG_ERROR_FATAL;
         plan->lattice_flag_clear = true;
@@ -1451,6 +1472,10 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
     int64_t inside = np - stats[0];
     if (radix) {
         const int* ks = nullptr;
+        if (!radix_scratch(plan, np, ncells + 1)) {
+            set_error(PPMG_ERROR_FATAL, PPMG_ERR_ALLOC, "scratch of the radix sort refused");
+            return PPMG_ERROR_FATAL;
+        }
         if (radix_sort(plan, plan->key.as<int>(), np, ncells + 1, lpdx, 1, inside, s, &ks)) return PPMG_ERROR_FATAL;
         hipLaunchKernelGGL(k_heads, dim3(nblk(ncells, HEADS_CELLS)), dim3(256), 0, s, ks, np, ncells, lhbx, 1, 1,
                            (int*)nullptr);

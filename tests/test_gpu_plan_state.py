@@ -117,10 +117,10 @@ def test_graph_plan_retry_after_refused_allocation(core, monkeypatch):
     assert len(calls) == 2 and torch.equal(got, want)
 
 
-def _crowded(core, N=128, n=1 << 17):
-    """Particles in an eighth of the mesh per axis, 32 to a cell there."""
+def _crowded(core, N=128, n=1 << 19):
+    """Particles in a quarter of the mesh per axis, 16 to a cell there."""
     g = torch.Generator(device="cuda").manual_seed(4)
-    x = torch.rand((n, 3), dtype=torch.float64, device="cuda", generator=g) / 8 + 0.4
+    x = torch.rand((n, 3), dtype=torch.float64, device="cuda", generator=g) / 4 + 0.4
     u = torch.randn((n, 1), dtype=torch.float64, device="cuda", generator=g)
     mesh = core.Mesh(3, N + 1)
     return mesh, x, u, torch.empty(mesh.compact_shape(1), dtype=torch.float64, device="cuda")
@@ -154,3 +154,21 @@ def test_work_list_without_memory(core, monkeypatch):
     got = cycle(plan)
     assert plan.scratch_bytes() > before       # the list has its scratch now
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_radix_binning_without_memory(core, monkeypatch):
+    """Crowded input whose radix sort is refused its scratch is binned by
+    counting: the same keys, permutation, heads and field."""
+    mesh, x, u, f = _crowded(core)
+    plan, got, size = core.Plan(), [], []
+    # counted without the sort; sort refused, twice; sorted
+    for env in ({"PPMG_RADIX": "0"}, {"PPMG_FAIL_ALLOC_ABOVE": "0"}, {"PPMG_FAIL_ALLOC_ABOVE": "0"}, {}):
+        with monkeypatch.context() as m:
+            for k, v in env.items():
+                m.setenv(k, v)
+            core.p2m(mesh, x, u, f, [0] * 3, plan=plan)
+        size.append(plan.scratch_bytes())
+        got.append((f.clone(),) + plan.sort_view())
+    assert size[0] == size[1] == size[2] < size[3]
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(other, got[0]))
