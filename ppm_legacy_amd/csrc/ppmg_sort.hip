@@ -1436,9 +1436,12 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
     // no order, eight to a box: 0.46 against 1.34 ms; 10^6: 102 against 114 us,
     // 2^19: 98 against 85); slot
     // atomics and per-cell sorts keep the small ones, whose counts stay in L2
-    // and which have few launches (PPMG_RADIX forces either, as in the binning).
+    // and which have few launches (PPMG_RADIX forces either, as in the binning),
+    // and those whose sort is refused its scratch (20 bytes a particle with the
+    // keys, where counting takes 8 and 4 per box).
     const char* rx = std::getenv("PPMG_RADIX");
-    const bool radix = np > 0 && (rx && rx[0] ? rx[0] == '1' : np >= RANK_RADIX_NP);
+    const bool radix = np > 0 && (rx && rx[0] ? rx[0] == '1' : np >= RANK_RADIX_NP) &&
+                       radix_scratch(plan, np, ncells + 1);
     if (plan->key.ensure(sizeof(int) * (size_t)(np > 0 ? np : 1)) || plan->err.ensure(sizeof(int) * 4)) return PPMG_ERROR_FATAL;
     if (!radix && (plan->slot.ensure(sizeof(int) * (size_t)(np > 0 ? np : 1)) ||
                    plan->count.ensure(sizeof(int) * (size_t)ncells)))
@@ -1472,10 +1475,6 @@ int rank_particles(ppmg_plan* plan, const RankGeom& g, int prec, int64_t np, con
     int64_t inside = np - stats[0];
     if (radix) {
         const int* ks = nullptr;
-        if (!radix_scratch(plan, np, ncells + 1)) {
-            set_error(PPMG_ERROR_FATAL, PPMG_ERR_ALLOC, "scratch of the radix sort refused");
-            return PPMG_ERROR_FATAL;
-        }
         if (radix_sort(plan, plan->key.as<int>(), np, ncells + 1, lpdx, 1, inside, s, &ks)) return PPMG_ERROR_FATAL;
         hipLaunchKernelGGL(k_heads, dim3(nblk(ncells, HEADS_CELLS)), dim3(256), 0, s, ks, np, ncells, lhbx, 1, 1,
                            (int*)nullptr);

@@ -172,3 +172,19 @@ def test_radix_binning_without_memory(core, monkeypatch):
     assert size[0] == size[1] == size[2] < size[3]
     for other in got[1:]:
         assert all(torch.equal(a, b) for a, b in zip(other, got[0]))
+
+
+def test_rank_without_memory_for_the_sort(core, monkeypatch):
+    """util_rank whose radix sort is refused its scratch ranks by counting."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.rand((20000, 3), dtype=torch.float64, device="cuda", generator=g) * 1.1
+    plan, got, size = core.Plan(), [], []
+    for env in ({"PPMG_RADIX": "0"}, {"PPMG_RADIX": "1", "PPMG_FAIL_ALLOC_ABOVE": "0"}, {"PPMG_RADIX": "1"}):
+        with monkeypatch.context() as m:
+            for k, v in env.items():
+                m.setenv(k, v)
+            got.append(core.util_rank(x, [0.0] * 3, [1.0] * 3, (9, 8, 7), [1, 0, 0, 0, 1, 0], plan))
+        size.append(plan.scratch_bytes())
+    assert size[0] == size[1] < size[2]
+    for other in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(other, got[0]))
