@@ -1176,12 +1176,13 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     const bool predict_sorted = plan->sorted_input;
     // Unsorted input for a reader of the slot table: the key pass fills the
     // table, and no keys, scan or scatter follow.  A plan whose table
-    // overflowed bins its next 16 inputs without one.  Allocation-free calls
+    // overflowed, or was refused its memory, bins its next 16 inputs without
+    // one.  Allocation-free calls
     // take the heads (the table needs 32 bytes per cell), and so does every
     // call under PPMG_NO_TABLE=1 (used to cross-check the two layouts).
     const char* no_table = std::getenv("PPMG_NO_TABLE");
     if (no_table && no_table[0] && no_table[0] != '0') table = false;
-    const bool use_table = table && !predict_sorted && plan->table_skip == 0 && !arena_bound();
+    bool use_table = table && !predict_sorted && plan->table_skip == 0 && !arena_bound();
     if (table && !predict_sorted && plan->table_skip > 0) --plan->table_skip;
     // Crowded input (the last binning's sample found a cell of nine or more
     // particles per 64 particles), and large input in no order, is binned by the
@@ -1201,8 +1202,11 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
         plan->lattice_flag_clear = true;
         return bin_crowded(plan, m, prec, np, xp, s, nbad);
     }
-    if (use_table ? plan->table.ensure(sizeof(int) * TABLE_SLOTS * (size_t)ncells) : sorted_lists())
-        return PPMG_ERROR_FATAL;
+    if (use_table && !plan->table.try_ensure(sizeof(int) * TABLE_SLOTS * (size_t)ncells)) {
+        use_table = false;
+        plan->table_skip = 16;
+    }
+    if (!use_table && sorted_lists()) return PPMG_ERROR_FATAL;
     if (plan->count.ensure(count_alloc) ||
         plan->multi.ensure(sizeof(int) * (size_t)nblk(np, KEYS_BLOCK) * KEYS_BLOCK) ||
         plan->multi_n.ensure(sizeof(int) * (size_t)nblk(np, KEYS_BLOCK)))

@@ -188,3 +188,40 @@ def test_rank_without_memory_for_the_sort(core, monkeypatch):
     assert size[0] == size[1] < size[2]
     for other in got[1:]:
         assert all(torch.equal(a, b) for a, b in zip(other, got[0]))
+
+
+@pytest.mark.parametrize("case", ["periodic", "open", "2d", "remesh", "m2p", "m2p_open"])
+def test_slot_table_without_memory(core, monkeypatch, case):
+    """A slot table (32 bytes a cell) that is refused: the particles are binned
+    to heads and a permutation, with bitwise the same result."""
+    dim, N, n = (2, 256, 3000) if case == "2d" else (3, 40, 3000)
+    bc = [1] * (2 * dim)
+    if "open" in case:
+        bc[4:] = [7, 7]
+    mesh = core.Mesh(dim, N + 1, bcdef=bc)
+    rng = np.random.default_rng(12)
+    x = torch.as_tensor(rng.uniform(0, 1, (n, dim))).cuda()
+    u = torch.as_tensor(rng.normal(size=(n, 2))).cuda()
+    f0 = torch.as_tensor(rng.normal(size=mesh.padded_shape(2, [2] * dim))).cuda()
+
+    def run(plan):
+        f, out = f0.clone(), torch.empty_like(u)
+        if "m2p" in case:
+            core.m2p(mesh, x, f, [-2] * dim, out, plan=plan)
+            return out
+        if case == "remesh":
+            core.remesh(mesh, x, u, core.comp_weights(mesh, x), f, [-2] * dim, plan=plan)
+        else:
+            core.p2m(mesh, x, u, f, [-2] * dim, plan=plan)
+        return f
+
+    table = 32 * int(np.prod([N + (b != 1) for b in bc[::2]]))
+    want, plan = run(core.Plan()), core.Plan()
+    with monkeypatch.context() as m:
+        m.setenv("PPMG_FAIL_ALLOC_ABOVE", str(table - 1))
+        for _ in range(3):
+            assert torch.equal(run(plan), want)
+    assert plan.scratch_bytes() < table
+    for _ in range(16):
+        assert torch.equal(run(plan), want)
+    assert plan.scratch_bytes() > table        # asked for again after 16 inputs
