@@ -35,21 +35,30 @@ int debug_level() { return g_debug.load(); }
 // PPMG_FAIL_ALLOC_ABOVE=<bytes> set, every new scratch allocation larger than
 // that many bytes fails as a refused hipMalloc would (read only when a buffer
 // has to grow, so calls that reuse their scratch never look at it).
+// PPMG_FAIL_ALLOC_TOTAL=<bytes> refuses what would leave the calling thread
+// with more than that many bytes allocated and not freed.
+static thread_local int64_t g_thread_bytes = 0;
 static bool injected_alloc_failure(size_t n) {
     const char* e = std::getenv("PPMG_FAIL_ALLOC_ABOVE");
-    if (!e || !*e) return false;
-    return n > (size_t)std::strtoull(e, nullptr, 10);
+    if (e && *e && n > (size_t)std::strtoull(e, nullptr, 10)) return true;
+    e = std::getenv("PPMG_FAIL_ALLOC_TOTAL");
+    return e && *e && g_thread_bytes + (int64_t)n > std::strtoll(e, nullptr, 10);
 }
 
 // A refused allocation's HIP error is taken here, not left for the next call's
-// launch check.
+// launch check.  It is tried once more if the registry had an idle plan to give
+// up for it.
 static hipError_t device_malloc(void** p, size_t n) {
-    const hipError_t e = injected_alloc_failure(n) ? hipErrorOutOfMemory : hipMalloc(p, n);
-    if (e != hipSuccess) {
+    for (;;) {
+        const hipError_t e = injected_alloc_failure(n) ? hipErrorOutOfMemory : hipMalloc(p, n);
+        if (e == hipSuccess) {
+            g_thread_bytes += (int64_t)n;
+            return e;
+        }
         (void)hipGetLastError();
         *p = nullptr;
+        if (!release_idle_plan()) return e;
     }
-    return e;
 }
 
 static thread_local Arena* g_arena = nullptr;
@@ -92,7 +101,10 @@ bool DevBuf::try_ensure(size_t n) {
     return true;
 }
 void DevBuf::release() {
-    if (p && !borrowed) (void)hipFree(p);
+    if (p && !borrowed) {
+        (void)hipFree(p);
+        g_thread_bytes -= (int64_t)bytes;
+    }
     p = nullptr;
     bytes = 0;
     borrowed = false;

@@ -412,6 +412,10 @@ struct DevBuf {
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Frees the calling thread's registry plan that its last registry call did not
+// use (ppmg_registry.hip); false if there is none.
+bool release_idle_plan();
+
 // Fixed device memory of an allocation-free call.  While an arena is bound on
 // the calling thread, DevBuf::ensure carves buffers from it in bump order
 // (256-byte aligned) instead of calling hipMalloc, and a request past its end

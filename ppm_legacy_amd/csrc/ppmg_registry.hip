@@ -27,16 +27,21 @@ static int g_prec_mode = PPMG_PREC_F64;
 // of its own: a client's P2M and M2P bin particles in different orders
 // (advected ones, and often a fresh lattice), and one plan's predictions for
 // the one are wrong for the other (64^3: 90 us of a second binning per pass).
+// The plan the last call did not use is given up where memory is short, and all
+// of it by ppmg_finalize, for the calling thread, or at the thread's end.
 struct Staging {
     ppmg_plan* plan = nullptr;
     ppmg_plan* m2p_plan = nullptr;
+    ppmg_plan* last = nullptr;   // the one the last call used
     DevBuf xp, up, field, w[3], conv_up, conv_field, lp, lh;
-    ~Staging() {
+    void release() {
         DevBuf* b[] = {&xp, &up, &field, &w[0], &w[1], &w[2], &conv_up, &conv_field, &lp, &lh};
         for (DevBuf* x : b) x->release();
         if (plan) ppmg_plan_destroy(plan);
         if (m2p_plan) ppmg_plan_destroy(m2p_plan);
+        plan = m2p_plan = last = nullptr;
     }
+    ~Staging() { release(); }
 };
 static thread_local Staging g_stage;
 
@@ -59,12 +64,21 @@ static int lookup(int topo_id, int mesh_id, Topo* out) {
 
 static ppmg_plan* stage_plan() {
     if (!g_stage.plan) ppmg_plan_create(&g_stage.plan);
-    return g_stage.plan;
+    return g_stage.last = g_stage.plan;
 }
 
 static ppmg_plan* stage_m2p_plan() {
     if (!g_stage.m2p_plan) ppmg_plan_create(&g_stage.m2p_plan);
-    return g_stage.m2p_plan;
+    return g_stage.last = g_stage.m2p_plan;
+}
+
+// (Freeing its buffers waits for whatever still runs.)
+bool release_idle_plan() {
+    ppmg_plan*& idle = g_stage.plan && g_stage.plan != g_stage.last ? g_stage.plan : g_stage.m2p_plan;
+    if (!idle || idle == g_stage.last) return false;
+    ppmg_plan_destroy(idle);
+    idle = nullptr;
+    return true;
 }
 
 // Host arrays are copied to device scratch; device arrays pass through.
@@ -147,6 +161,7 @@ int ppmg_init(int dim, int prec, int tolexp, int debug) {
 }
 
 int ppmg_finalize(void) {
+    g_stage.release();
     std::lock_guard<std::mutex> lk(g_mu);
     g_topos.clear();
     g_initialized = false;

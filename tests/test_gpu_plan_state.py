@@ -225,3 +225,47 @@ def test_slot_table_without_memory(core, monkeypatch, case):
     for _ in range(16):
         assert torch.equal(run(plan), want)
     assert plan.scratch_bytes() > table        # asked for again after 16 inputs
+
+
+def test_registry_in_the_memory_of_one_plan(core, monkeypatch):
+    """The registry keeps a plan per direction.  Where there is memory for one
+    only, the idle one is given up; ppm_finalize gives up both.  A thread of its
+    own, which starts with nothing."""
+    import threading
+
+    from ppm_legacy_amd import ppm
+    N = 40
+    rng = np.random.default_rng(13)
+    x = torch.as_tensor(rng.uniform(0, 1, (3000, 3))).cuda()
+    u = torch.as_tensor(rng.normal(size=(3000, 2))).cuda()
+    mesh = core.Mesh(3, N + 1)
+    f = torch.zeros(mesh.padded_shape(2, [2] * 3), dtype=torch.float64, device="cuda")
+    back = torch.empty_like(u)
+    p, q = core.p2m(mesh, x, u, f, [-2] * 3), core.m2p(mesh, x, f, [-2] * 3, back)
+    one = max(p.scratch_bytes(), q.scratch_bytes())
+    torch.cuda.synchronize()
+    failed = []
+
+    def work():
+        try:
+            assert ppm.ppm_init(3, ppm.ppm_kind_double, -15, None, 0) == 0
+            info, topo, meshid = ppm.ppm_mktopo([0.0] * 3, [1.0] * 3, [1] * 6, [N + 1] * 3, [2] * 3)
+            assert info == 0
+            monkeypatch.setenv("PPMG_FAIL_ALLOC_TOTAL", str(one + 65536))
+            for _ in range(2):
+                g, b = torch.zeros_like(f), torch.zeros_like(u)
+                torch.cuda.synchronize()
+                assert ppm.ppm_interp_m2p(x, 3000, b, topo, meshid, MP4, [2] * 3, f) == 0
+                assert ppm.ppm_interp_p2m(x, 3000, u, topo, meshid, MP4, [2] * 3, g) == 0
+                assert torch.equal(g, f) and torch.equal(b, back)
+            assert ppm.ppm_finalize() == 0
+            core.p2m(mesh, x, u, g, [-2] * 3)
+            torch.cuda.synchronize()
+            assert torch.equal(g, f)
+        except BaseException as e:
+            failed.append(repr(e))
+
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    assert not failed
