@@ -7,6 +7,8 @@
 // M2P and the adjoint are particle-owned gathers.  ppmg_p2m3d.hip holds the
 // tiled fast path for the 3D M'4 workloads; this file is the reference-exact
 // path it is checked against and the path every other variant runs on.
+#include <algorithm>
+
 #include "ppmg_internal.h"
 #include "ppmg_interp.h"
 #include "ppmg_sort.h"
@@ -824,11 +826,16 @@ int comp_weights_general(const DevMesh& m, int kernel, int prec, int64_t np, con
                          void* w3, hipStream_t s) {
     if (np <= 0) return 0;
     const bool mp4 = kernel == PPMG_KERNEL_MP4;
-    const unsigned g = nblk(mp4 ? 2 * np : np, 256);   // two lanes per M'4 particle
-#define CW(D, K, P, V) hipLaunchKernelGGL((k_comp_weights<D, K, P, V>), dim3(g), dim3(256), 0, s, (const P*)xp, np, m, (V*)w1, (V*)w2, (V*)w3)
+    // two lanes per M'4 particle, 2^30 particles a launch: under 2^32 threads
+    for (int64_t p0 = 0; p0 < np; p0 += (int64_t)1 << 30) {
+        const int64_t n = std::min(np - p0, (int64_t)1 << 30);
+        const unsigned g = nblk(mp4 ? 2 * n : n, 256);
+#define CW(D, K, P, V) hipLaunchKernelGGL((k_comp_weights<D, K, P, V>), dim3(g), dim3(256), 0, s, (const P*)xp + p0 * D, n, m, \
+                                          (V*)w1 + p0 * K, (V*)w2 + p0 * K, D == 3 ? (V*)w3 + p0 * K : nullptr)
 #define CWP(D, K) do { if (prec == PPMG_PREC_F64) CW(D, K, double, double); else if (prec == PPMG_PREC_F32C) CW(D, K, double, float); else CW(D, K, float, float); } while (0)
-    if (m.dim == 3) { if (mp4) CWP(3, 4); else CWP(3, 2); }
-    else { if (mp4) CWP(2, 4); else CWP(2, 2); }
+        if (m.dim == 3) { if (mp4) CWP(3, 4); else CWP(3, 2); }
+        else { if (mp4) CWP(2, 4); else CWP(2, 2); }
+    }
 #undef CWP
 #undef CW
     PPMG_HIP(hipGetLastError());
