@@ -344,6 +344,19 @@ int ppmg_plan_sort_view(const ppmg_plan* plan, const int** key, const int** perm
         if (materialize_keys(w, w->bin_stream)) return g_status.info;
         PPMG_HIP(hipStreamSynchronize(w->bin_stream));
     }
+    // a binning that failed (a particle outside the sub) may have left no heads
+    // or permutation, or those of a smaller one: the arrays are there all the same
+    ppmg_plan* w = const_cast<ppmg_plan*>(plan);
+    auto hold = [&](DevBuf& b, int64_t n) -> int {
+        const size_t bytes = sizeof(int) * (size_t)n;
+        if (b.p && b.bytes >= bytes) return 0;
+        if (b.ensure(bytes) || fill_zero(b.p, bytes, w->bin_stream)) return PPMG_ERROR_FATAL;
+        PPMG_HIP(hipStreamSynchronize(w->bin_stream));
+        return 0;
+    };
+    if ((key && hold(w->key, plan->np)) || (perm && hold(w->perm, plan->np)) ||
+        (start && hold(w->start, plan->ncells + 1)))
+        return g_status.info;
     if (key) *key = plan->key.as<int>();
     if (perm) *perm = plan->perm.as<int>();
     if (start) *start = plan->start.as<int>();

@@ -1255,7 +1255,10 @@ int bin_particles(ppmg_plan* plan, const DevMesh& m, int prec, int64_t np, const
     }
     plan->crowded_cells = 64 * crowd;   // estimates from the 1-in-64 samples
     plan->far_particles = 64 * far;
-    if (herr[0]) return 0;
+    if (herr[0]) {
+        plan->keys_written = false;   // (made on demand)
+        return 0;
+    }
     plan->lattice_pred = herr[5] == 0 && np == ncells;
     plan->lattice_prec = prec;
     plan->lattice_mesh = m;

@@ -269,3 +269,35 @@ def test_registry_in_the_memory_of_one_plan(core, monkeypatch):
     t.start()
     t.join()
     assert not failed
+
+
+@pytest.mark.parametrize("sizes", [(12,), (4, 30)], ids=["new", "grown"])
+def test_sort_view_after_a_refused_binning(core, sizes):
+    """Particles outside the sub: P2M refuses them, and the plan's view still
+    has arrays of the right size, with the keys (-1 outside)."""
+    from ppm_legacy_amd import _lib
+    plan = core.Plan()
+    for N in sizes:
+        rng = np.random.default_rng(N)
+        n = N ** 3
+        x = rng.uniform(0, 1, (n, 3))
+        x[[1, n // 2]] = [1.5, 0.5, 0.5]
+        mesh = core.Mesh(3, N + 1)
+        u = torch.ones((n, 1), dtype=torch.float64, device="cuda")
+        f = torch.empty(mesh.compact_shape(1), dtype=torch.float64, device="cuda")
+        if N != sizes[-1]:       # a smaller binning first, which leaves small arrays
+            core.p2m(mesh, torch.as_tensor(rng.uniform(0, 1, (n, 3))).cuda(), u, f, [0] * 3, plan=plan)
+            plan.sort_view()
+            continue
+        xd = torch.as_tensor(x).cuda()
+        with pytest.raises(_lib.PpmgError) as e:
+            core.p2m(mesh, xd, u, f, [0] * 3, plan=plan)
+        assert e.value.code == _lib.ERR_PART_UNASS
+        key, perm, start = plan.sort_view()
+        c = np.floor(x * N).astype(int)
+        want = np.where((x < 1).all(1), c[:, 0] + N * (c[:, 1] + N * c[:, 2]), -1)
+        assert np.array_equal(key.cpu().numpy(), want)
+        assert perm.shape == (n,) and start.shape == (N ** 3 + 1,)
+        xd[[1, n // 2]] = 0.5
+        core.p2m(mesh, xd, u, f, [0] * 3, plan=plan)
+        assert abs(f.sum().item() - n) < 1e-9 * n
