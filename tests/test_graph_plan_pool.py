@@ -208,3 +208,25 @@ def test_nothing_pooled_where_memory_is_short(dev, monkeypatch):
     last = f.grad_fn.plan.plan
     del f
     assert last.closed and all(p.closed for p in plans) and not autograd._pool.get(0)
+
+
+def test_free_memory_is_asked_for_now_and_then(dev, monkeypatch):
+    """A steady loop does not ask at every graph, but does after ASK_SECONDS."""
+    now, asked = [100.0], []
+    monkeypatch.setattr(autograd, "_asked", {})
+    monkeypatch.setattr(autograd.time, "monotonic", lambda: now[0])
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (asked.append(now[0]), (1 << 40, 1 << 40))[1])
+    for _ in range(5):
+        f, _ = _graph()
+        del f
+    assert len(asked) == 1
+    now[0] += 2 * autograd.ASK_SECONDS
+    for _ in range(5):
+        f, _ = _graph()
+        del f
+    assert len(asked) == 2
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (0, 1 << 40))
+    now[0] += 2 * autograd.ASK_SECONDS
+    f, _ = _graph()
+    del f
+    assert not autograd._pool.get(0) and dev.plans[-1].closed
