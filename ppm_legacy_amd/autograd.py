@@ -51,7 +51,9 @@ def release_plans(device=None):
 def _given_back(e):
     """Whether e says that memory ran out and the pool had some to give back:
     worth another try."""
-    if (isinstance(e, PpmgError) and e.code != ERR_ALLOC) or not any(_pool.values()):
+    with _lock:
+        some = any(_pool.values())
+    if not some or (isinstance(e, PpmgError) and e.code != ERR_ALLOC):
         return False
     release_plans()
     return True
