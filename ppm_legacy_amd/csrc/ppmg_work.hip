@@ -10,6 +10,8 @@
 // that the dispatcher hands them out evenly over the XCDs and the light ones
 // fill in behind.  Which workgroup makes a node, and where its tile column is
 // cut, does not change the order of the node's additions.
+#include <algorithm>
+
 #include "ppmg_internal.h"
 #include "ppmg_sort.h"
 
@@ -119,14 +121,21 @@ int build_work(ppmg_plan* plan, const DevMesh& m, const TileWindow& w, int slots
         return 0;
     int* count = plan->work_cnt.as<int>();
     const double load = ((double)w.ntx * w.nty * w.planes + 1.5 * (double)plan->np / ((double)w.tx * w.ty)) / slots;
-    // Clustered input (half a particle a cell, four blobs), FP64, lda 3.  The
-    // deposit pays for a cut with its halo planes: 512^3 9.7, 9.2, 9.0 ms and
-    // 168 x 169 x 249 718, 734, 774 us at shares of 0.5, 0.75 and 1.  A gather
-    // pays little: 168 x 169 x 249 432 and 498 us, its adjoint 874 and 1124 us,
-    // at 0.25 and 0.5; at 512^3 cuts cost locality, 8.0 and 7.8 ms at 0.25 and 1.
-    // (A fixed cost of 800, right for 512^3, took 2850 and 830 us at 168 x 169 x 249;
-    // chunks of one height 1459 and 753 us.)
-    const double share = w.halo ? 0.75 : std::min(std::max(load / 1000.0, 0.25), 0.75);
+    // Clustered input (half a particle a cell, four blobs), M'4.  The deposit pays
+    // for a cut with its halo planes: FP64, lda 3, 512^3 9.7, 9.2, 9.0 ms and
+    // 168 x 169 x 249 718, 734, 774 us at shares of 0.5, 0.75 and 1.  A gather pays
+    // little and is best cut fine, whatever its size.  At shares of 0.25, 0.5 and
+    // 0.75, us (loads of 9, 54, 125, 431 and 1000):
+    //                       gather FP64 lda 3    FP32c lda 3       FP64 lda 1       adjoint FP64 lda 3
+    //   100 x 90 x 110      139 141 175          144 148 175       102 102 121      279 294 346
+    //   168 x 169 x 249     477 592 679          449 542 648       327 398 466      952 1402 1533
+    //   256^3               961 1309 1141        913 1250 1038     740 898 861      2298 2524 2622
+    //   384^3               3311 3356 3440       2980 3071 3114    2415 2487 2471   7239 7276 7334
+    //   512^3               8099 8050 8078       7397 7259 7176    6179 6171 6134   16750 16608 16691
+    // (0.15 is within 3% of 0.25 but for the FP64 adjoint at 256^3, 2002; BSP2 gathers
+    // differ by up to 3% from 0.15 to 0.5 and lose at 0.75.  A fixed cost of 800 took
+    // 2850 and 830 us at 168 x 169 x 249; chunks of one height 1459 and 753 us.)
+    const double share = w.halo ? 0.75 : 0.25;
     const int most = (int)std::min(std::max(load * share, 4.0), 1e6);
     if (fill_zero(count, sizeof(int) * WK_CLASSES, s)) return PPMG_ERROR_FATAL;
     hipLaunchKernelGGL(k_work_cut, dim3((unsigned)nid), dim3(256), 0, s, m, w, plan->start.as<int>(), nseg, most, count,
