@@ -120,8 +120,8 @@ int ppmg_plan_scratch_bytes(const ppmg_plan* plan, int64_t* bytes);
  * (ppm_map_field_ghost init/ghost_put/push/send/pop, ppm_interp_p2m.f:3670-3716).
  * Stored nodes real in every axis receive the folded sum; nodes outside the
  * real range in some axis receive the raw (unfolded) scatter, as the
- * reference leaves them.  Particles are binned by a stable counting sort whose
- * permutation and cell keys stay in the plan for ppmg_p2m_adjoint. */
+ * reference leaves them.  Particles are binned in stable cell order, and the
+ * binning stays in the plan for ppmg_p2m_adjoint until the plan bins again. */
 int ppmg_p2m(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, const void* xp, int lda,
              const void* up, const ppmg_field* field, ppmg_plan* plan, void* stream);
 
@@ -168,9 +168,9 @@ int ppmg_m2p_prebin(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, con
  * periodic and non-periodic axes): each particle collects g from every stored
  * node the forward writes it into (a real node and its periodic copies, such
  * as node N beside node 0, and a ghost node's raw sum).  grad_up = dL/du
- * (np, lda), grad_xp = dL/dx (np, dim); either may be NULL.  Uses the
- * permutation and cell keys that the last ppmg_p2m on this plan left (same
- * mesh, kernel, np and xp required). */
+ * (np, lda), grad_xp = dL/dx (np, dim); either may be NULL.  Uses the binning
+ * that the last ppmg_p2m on this plan left (same mesh, kernel, np and xp
+ * required); refused once another call has binned over it. */
 int ppmg_p2m_adjoint(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, const void* xp,
                      int lda, const void* up, const ppmg_field* g, void* grad_up, void* grad_xp,
                      ppmg_plan* plan, void* stream);
@@ -180,7 +180,9 @@ int ppmg_p2m_adjoint(const ppmg_mesh* mesh, int kernel, int prec, int64_t np, co
  * reference (cells per axis), ngl = Ngl(1:2*dim).  lpdx (capacity np) gets the
  * 1-based particle indices in cell order, lhbx (prod(ncells+ngl_lo+ngl_hi)+1)
  * the 1-based cell heads; *icount = particles inside the mesh.  prec selects
- * float (PPMG_PREC_F32) or double positions and bounds. */
+ * float (PPMG_PREC_F32) or double positions and bounds.  Scratch in the plan: 8
+ * bytes a particle and 4 a box, or from 786,432 particles 20 bytes a particle
+ * (where those are refused, the former). */
 int ppmg_util_rank(int dim, int prec, int64_t np, const void* xp, const void* xmin,
                    const void* xmax, const int* ncells, const int* ngl, int* lpdx, int* lhbx,
                    int64_t* icount, ppmg_plan* plan, void* stream);
@@ -257,7 +259,9 @@ int ppmg_plan_timings(ppmg_plan* plan, double* ms, int n);
  * stable cell order, 0-based) and start[ncells+1] (cell heads, 0-based).
  * Input already in cell order is binned without writing keys or the identity
  * permutation; this call then computes them, reading the positions that
- * binning was given, which must still hold them.
+ * binning was given, which must still hold them.  After a binning that refused
+ * particles outside the sub, key is -1 for those, and perm and start have their
+ * sizes but no meaning.
  * The ppm_util_rank3d analogue of these is ppmg_util_rank (1-based). */
 int ppmg_plan_sort_view(const ppmg_plan* plan, const int** key, const int** perm, const int** start,
                         int64_t* np, int64_t* ncells);
@@ -271,6 +275,8 @@ int ppmg_device_sync(void* stream);
 /* ppm_init(dim,prec,tolexp,comm,debug,info) (ppm_init.f:161): prec is
  * PPM's ppm_kind_double/single, here PPMG_PREC_F64 / PPMG_PREC_F32. */
 int ppmg_init(int dim, int prec, int tolexp, int debug);
+/* Forgets the topologies and frees the calling thread's registry scratch (staging
+ * buffers and two plans, one for M2P; other threads' go when they end). */
 int ppmg_finalize(void);
 /* Selects the arithmetic form used by the double-precision registry entry
  * points (PPMG_PREC_F64 or PPMG_PREC_F32C); the reference signatures stay

@@ -417,7 +417,7 @@ static int launch_a3_rows(ppmg_plan* plan, const DevMesh& m, const PosT* xp, con
 }
 
 // Rows of 32 lanes where they cover the mesh with fewer lanes, as in the
-// gather (75% of the issue slots at 512^3).  FP64, lda 3: 512^3 9.46 -> 8.85
+// gather (VALU 78% busy at 512^3).  FP64, lda 3: 512^3 9.46 -> 8.85
 // ms, 200^3 635 -> 575 us, stored boxes 200^3 775 -> 745 us, 58^3 33 -> 29 us.
 template <int LL, typename PosT, typename ValT, typename AccT, bool BOXED, bool TABLE = false>
 static int launch_a3_form(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const ValT* up, const ValT* g,

@@ -463,7 +463,7 @@ struct ppmg_plan {
     // counts in `count`) instead of `start` and `perm`; materialize_heads()
     // builds those two from it.
     bool bin_table = false;
-    int table_skip = 0;          // binnings to run without the table after one overflowed it
+    int table_skip = 0;          // binnings to run without the table after one overflowed it or was refused it
     // The last binning found a lattice in cell order (particle p in cell p,
     // np == ncells) on lattice_mesh in precision lattice_prec; bin_lattice:
     // the current binning is that lattice, taken without a pass and not yet

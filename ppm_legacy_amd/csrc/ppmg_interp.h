@@ -41,8 +41,10 @@ int p2m2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, const vo
 
 // 3D tiled gather (ppmg_m2p3d.hip), M'4 or BSP2, same layouts as the deposit:
 // bins the particles into the plan first (unless prebinned: the plan already
-// holds their binning); returns 1 without touching up when a particle lies
-// outside the sub.
+// holds their binning).  Returns 1 when a particle lies outside the sub, for
+// the general path, which writes every row of up: where a lattice was taken
+// without a binning pass (gather_checked), up already holds the values of a
+// gather that took each particle for its cell's.
 bool m2p3d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg);
 // The mesh takes an unchecked lattice (bin_particles' `lattice`).
 bool m2p3d_lattice_applicable(const DevMesh& m);
@@ -51,8 +53,8 @@ int m2p3d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t 
 
 // 2D tiled gather (ppmg_m2p2d.hip), M'4 or BSP2: periodic axes compact or a
 // stored box holding 0..N, open axes a box holding every node a stencil
-// reaches (no periodic box beside an open axis).  Bins first; returns 1
-// without touching up when a particle lies outside the sub.
+// reaches (no periodic box beside an open axis).  Bins first; returns 1 as the
+// 3D gather does.
 bool m2p2d_fast_applicable(const DevMesh& m, int kernel, const FieldGeom& fg);
 int m2p2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp,
                const FieldGeom& fg, const void* field, void* up, hipStream_t s);

@@ -282,8 +282,9 @@ static int m2p2d_typed(ppmg_plan* plan, const DevMesh& m, const PosT* xp, const 
     return 0;
 }
 
-// Bins the particles into the plan, then gathers.  Returns 1 (nothing done)
-// when some particle lies outside the sub, for the general path.  Sums in
+// Bins the particles into the plan, then gathers.  Returns 1 when some particle
+// lies outside the sub, for the general path, which writes every row of up (a
+// lattice taken without a binning pass has been gathered by then).  Sums in
 // FP64 in every form, as the 3D gather.
 int m2p2d_fast(ppmg_plan* plan, const DevMesh& m, int kernel, int prec, int64_t np, const void* xp,
                const FieldGeom& fg, const void* field, void* up, hipStream_t s) {

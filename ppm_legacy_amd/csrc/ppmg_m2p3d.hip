@@ -396,7 +396,7 @@ static int launch_m3_rows(ppmg_plan* plan, const DevMesh& m, const PosT* xp, con
 }
 
 // Rows of 32 or 16 lanes.  The M'4 gather is bound by its FP64 instructions
-// (92% of the issue slots at 512^3), and of a row all but three lanes carry
+// (78% of the issue slots at 512^3), and of a row all but three lanes carry
 // particles: 29 of 32 where the longer rows cover the mesh with fewer lanes,
 // else 13 of 16.  lda 3, lattice: 512^3 FP64 3.09 -> 2.89 ms, 256^3 FP32c
 // 374 -> 345 us.  (BSP2, 31 of 32 against 15 of 16, has too little to gain.)
@@ -445,9 +445,10 @@ static int m2p3d_typed(ppmg_plan* plan, const DevMesh& m, int64_t np, const PosT
     return 0;
 }
 
-// Bins the particles into the plan, then gathers.  Returns 1 (nothing done)
-// when some particle lies outside the sub, so the caller can use the general
-// path, which reads such particles' stencils with bounds checks.
+// Bins the particles into the plan, then gathers.  Returns 1 when some particle
+// lies outside the sub, so the caller can use the general path, which reads
+// such particles' stencils with bounds checks and writes every row of up (a
+// lattice taken without a binning pass has been gathered by then).
 //
 // Arithmetic: FP64 in every form.  On gfx950 (packed FP32 off) an FP64 FMA
 // issues at the FP32 rate, so the FP32-compensated form keeps FP32 only where

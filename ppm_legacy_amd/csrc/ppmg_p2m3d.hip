@@ -4,7 +4,7 @@
 // 2540-3055) plus its periodic ghost fold (:3670-3716) for 3D M'4 on periodic
 // and open axes, written in the compact layout (the unique nodes of periodic
 // axes) or into a stored box holding the real range (the reference's
-// field_up(1-g:Nm+g)), whose node N and ghost layers two small kernels fill.
+// field_up(1-g:Nm+g)), whose node N and ghost layers one more launch fills.
 //
 // Work decomposition (three wavefronts per workgroup):
 //   * a workgroup owns a 13 x 21 node tile in x,y and a chunk of node planes in z;
