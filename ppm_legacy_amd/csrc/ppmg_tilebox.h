@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(256) k_box_shell(DevMesh m, FieldGeom fg, int3
     // q-th stored node of axis d outside the real range: below 0, then above N
     auto outer = [&](int d, int q) { return q < -fg.lo[d] ? fg.lo[d] + q : m.N[d] + 1 + (q + fg.lo[d]); };
     int n[3];
-    auto locate = [&](auto q) {   // 32-bit divisions wherever the shell's node count fits
+    auto locate = [&](auto q) {   // 32-bit divisions wherever the box's node count fits
         using U = decltype(q);
         const U ra = (U)o2 * (U)e1 * (U)e0, rb = (U)r.z * (U)o1 * (U)e0;
         if (q < ra) {
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(256) k_box_shell(DevMesh m, FieldGeom fg, int3
             n[2] = (int)pl;
         }
     };
-    if ((uint64_t)nshell >> 32) locate((uint64_t)t);
+    if (((uint64_t)e0 * (uint64_t)e1 * (uint64_t)e2) >> 32) locate((uint64_t)t);
     else locate((uint32_t)t);
     double acc[LL];
 #pragma unroll
